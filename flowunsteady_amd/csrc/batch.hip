@@ -152,7 +152,16 @@ __global__ __launch_bounds__(BLK) void uj_f64_items_kernel(const BatchItem *__re
 {
     __shared__ double4 tile[2 * BLK];
     const BatchItem it = items[blockIdx.x];
-    uj_f64_block<K, BLK>(src, it.s0, it.s1, X, it.t0, it.t1, cap, U, J, reset, tile);
+    const int64_t s = (int64_t)it.t0 + threadIdx.x;
+    const int64_t i = min(s, (int64_t)it.t1 - 1);   // lanes past the last target repeat it
+    double d[15];
+    uj_f64_sums<K, BLK, BLK, false>(src, it.s0, it.s1, X[i], X[cap + i], X[2 * cap + i], nullptr,
+                                    tile, d);
+    if (s < it.t1) {
+        double v[12];
+        uj_f64_values(d, v);
+        uj_f64_store(v, s, cap, U, J, reset);
+    }
 }
 
 template <int K, int BLK>

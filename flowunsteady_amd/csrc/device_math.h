@@ -31,8 +31,7 @@ constexpr double INV_SQRT2 = 0.7071067811865476;
 
 // ---------------------------------------------------------------------------
 // FP64, reference form: g and g' exactly as the closed forms above (libm-style
-// erf/exp from the ROCm device math library), A and B assembled as in the
-// reference pair loop.  This is the correctness path.
+// erf/exp from the ROCm device math library); the free-vortex force uses it.
 template <int K>
 __device__ __forceinline__ void g_dg_f64(double rho, double &g, double &dg)
 {
@@ -136,6 +135,172 @@ __device__ __forceinline__ void zeta_zD_f64(double rho, double &z, double &zD)
     } else {
         z = 0.0;
         zD = 0.0;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// FP64 pair math of the all-pairs and near-field sums.
+//
+// What bounds those sums is FP64 VALU issue (4 cycles per wave instruction),
+// so the radial coefficients are evaluated by the shortest sequences that keep
+// their error at a few 1e-16, written from the mathematics below instead of
+// through libm's exp, erf, sqrt and division (169 FP64 instructions per near
+// pair with those, 88 so and 16 more where the series runs; one UJ_gpu call on
+// a rotor wake of 70,001: 24.9 -> 14.8 ms, the kernel at the full issue rate):
+//
+//   1/r          v_rsq_f64 and one third-order Newton step
+//   e^{-x/2}     2^k P(x + 2 k ln 2), P the degree-11 minimax of e^{-t/2} on
+//                |t| <= ln 2 (relative error 3e-18)
+//   erf          with x = rho^2, E = e^{-x/2} and erfcx(z) = e^{z^2} erfc(z),
+//                  g = 1 - E (erfcx(rho/sqrt2) + sqrt(2/pi) rho);
+//                on rho >= 1.5 erfcx(rho/sqrt2) is a polynomial of degree 11 in
+//                t = 1/(1 + rho/4), minimax with weight E on [1.5, 9.6] (error
+//                4e-19 in g; beyond, E g's share is below 1e-19).  That form
+//                loses the digits of g ~ rho^3 as rho -> 0, so on x < 2.25
+//                g/(sqrt(2/pi) rho^3) is a degree-12 polynomial in x (relative
+//                error 2e-18); it runs only when some lane of the wave needs it.
+//   B            from A and E: g' = sqrt(2/pi) rho^2 E gives
+//                  B = (sqrt(2/pi) E / sigma^3 - 3 A) / r^2.
+// Largest relative errors, all in units of 1e-16 against 50 digits (the
+// closed forms through libm in brackets): A 2 (6.8e4 at rho = 0.1, 50 at 0.5,
+// 3 beyond 1.5), B r^2 / A 13 (2e5, 140, 13).
+constexpr double EXP_HALF[12] = {
+    1.0, -0.5, 0.12500000000000044, -0.02083333333333271, 0.002604166666655789,
+    -0.0002604166666737258, 2.1701388986348433e-05, -1.5500991744385246e-06,
+    9.688080655811696e-08, -5.382348117568117e-09, 2.6984676970178313e-10,
+    -1.2204285537793266e-11};
+constexpr double GERF_SMALL[13] = {
+    0.3333333333333333, -0.09999999999999991, 0.01785714285714071, -0.0023148148147943996,
+    0.00023674242414118443, -2.0032050981917798e-05, 1.4467586856913403e-06,
+    -9.118156851100948e-08, 5.098357695475492e-09, -2.5590008622494337e-10,
+    1.1533875250279058e-11, -4.43463176124452e-13, 1.1180962860624989e-14};
+constexpr double ERFCX_T[12] = {
+    3.672063975485439e-05, 0.19869558511481117, 0.20696658778029875, 0.14321399007711033,
+    0.3340213070606755, -0.34968381664740894, 1.0381635337255333, -1.3184589318799849,
+    1.3843842548259702, -0.9042697211592458, 0.31105054273400085, -0.04412010507901784};
+constexpr double TWO_LN2_HI = 1.386294361119326, TWO_LN2_LO = 5.647058112606315e-13;
+constexpr double NEG_HALF_LOG2E = -0.7213475204444817;   // -log2(e)/2
+constexpr double ROUND_MAGIC = 6755399441055744.0;       // 1.5 * 2^52
+constexpr double X_SMALL = 2.25;                         // rho^2 below which the series runs
+constexpr double X_FAR = 90.25;    // rho = 9.5: 1 - g < 3e-19 and rho g' < 2e-17, the pair is singular
+constexpr double RHO_FAR = 9.5;
+constexpr double X_CORE = 120.0;   // e^{-60}: zeta and the core-size derivatives vanish
+constexpr double RHO_CORE = 10.96;
+
+__device__ __forceinline__ double rsq_f64(double a)
+{
+    const double y = __builtin_amdgcn_rsq(a);
+    const double e = fma(-a * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+__device__ __forceinline__ double rcp_f64(double a)
+{
+    const double y = __builtin_amdgcn_rcp(a);
+    const double e = fma(-a, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+
+// a b + c with the constant c in scalar registers.  Left to itself the compiler
+// takes the two-address v_fmac_f64 for a Horner step, with its coefficient
+// copied from a vector register first: twice the instructions and two vector
+// registers per coefficient.  (No operand may come straight from a
+// transcendental instruction, whose result needs a wait the compiler inserts
+// only between instructions of its own.)
+__device__ __forceinline__ double fma_sc(double a, double b, double c)
+{
+    double d;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+    return d;
+}
+
+// c[0] + c[1] t + ... + c[N-1] t^(N-1)
+template <int N>
+__device__ __forceinline__ double horner_f64(const double (&c)[N], double t)
+{
+    double p = fma_sc(t, c[N - 1], c[N - 2]);
+#pragma unroll
+    for (int n = N - 3; n >= 0; --n) p = fma_sc(p, t, c[n]);
+    return p;
+}
+
+// e^{-x/2}, x >= 0 (0 from x ~ 1490 on).
+__device__ __forceinline__ double exp_mhalf(double x)
+{
+    double u;   // min(x, 1500)
+    asm("v_min_f64 %0, %1, %2" : "=v"(u) : "v"(x), "s"(1500.0));
+    const double m = fma(u, NEG_HALF_LOG2E, ROUND_MAGIC);
+    const double k = m - ROUND_MAGIC;
+    const double t = fma(k, TWO_LN2_LO, fma(k, TWO_LN2_HI, u));
+    return ldexp(horner_f64(EXP_HALF, t), (int)(unsigned)__double_as_longlong(m));
+}
+
+// Constant of a source that its pairs need besides 1/sigma: gaussian-erf
+// sqrt(2/pi)/sigma^3, gaussian 3/sigma^3, Winckelmans sigma^2 (finite also
+// for cores so small that 1/sigma^3 overflows).
+template <int K>
+__device__ __forceinline__ double pair_const_f64(double sigma, double is)
+{
+    if constexpr (K == GAUSSIANERF) return fmin(SQRT2_PI * is * is * is, 1e300);
+    else if constexpr (K == GAUSSIAN) return fmin(3.0 * is * is * is, 1e300);
+    else if constexpr (K == WINCKELMANS) return sigma * sigma;
+    else return 0.0;
+}
+
+// A and B of a pair with r2 > 0, x = r2/sigma^2, rinv = 1/r, ri2 = rinv^2;
+// is = 1/sigma, kz = pair_const_f64.
+template <int K>
+__device__ __forceinline__ void radial_f64(double r2, double x, double rinv, double ri2, double is,
+                                           double kz, double &A, double &B)
+{
+    if constexpr (K == GAUSSIANERF) {
+        const double E = exp_mhalf(x);
+        const double rho = r2 * rinv * is;
+        const double t = rcp_f64(fma(0.25, rho, 1.0));
+        const double g = fma(-E, fma(SQRT2_PI, rho, horner_f64(ERFCX_T, t)), 1.0);
+        A = g * (ri2 * rinv);
+        if (__any(x < X_SMALL)) {
+            const double p = horner_f64(GERF_SMALL, x) * kz;
+            A = x < X_SMALL ? p : A;
+        }
+        B = fma(-3.0, A, E * kz) * ri2;
+    } else if constexpr (K == GAUSSIAN) {
+        const double rho = r2 * rinv * is;
+        const double e = exp_mhalf(2.0 * rho * rho * rho);
+        A = (1.0 - e) * (ri2 * rinv);
+        B = fma(-3.0, A, e * kz) * ri2;
+    } else if constexpr (K == WINCKELMANS) {   // s^2 = r^2 + sigma^2: exact rewrite of the closed forms
+        const double si = rsq_f64(r2 + kz), si2 = si * si, si5 = si2 * si2 * si;
+        A = fma(2.5, kz, r2) * si5;
+        B = -3.0 * fma(3.5, kz, r2) * (si5 * si2);
+    } else {
+        A = ri2 * rinv;
+        B = -3.0 * A * ri2;
+    }
+}
+
+// The core-size derivatives A_D = h/r^3 = -4 pi zeta/sigma^3 and
+// B_D = -4 pi zeta'/(rho sigma^5) of the same pair (finite at r = 0).
+template <int K>
+__device__ __forceinline__ void radial_dsig_f64(double r2, double x, double is, double kz,
+                                                double &A, double &B)
+{
+    if constexpr (K == GAUSSIANERF) {
+        const double e = exp_mhalf(x) * kz;
+        A = -e;
+        B = e * (is * is);
+    } else if constexpr (K == GAUSSIAN) {
+        const double rho = sqrt(x);
+        const double e = exp_mhalf(2.0 * x * rho) * kz;
+        A = -e;
+        B = 3.0 * rho * e * (is * is);
+    } else if constexpr (K == WINCKELMANS) {
+        const double si = rsq_f64(r2 + kz), si2 = si * si, s7 = kz * kz * (si2 * si2 * si2 * si);
+        A = -7.5 * s7;
+        B = 52.5 * s7 * si2;
+    } else {
+        A = 0.0;
+        B = 0.0;
     }
 }
 

@@ -48,9 +48,9 @@ struct Scratch {
     double4 *srcE = nullptr;         // FP64 Estr source records, 7 per particle
     double4 *spos = nullptr;         // Morton-sorted (x, y, z, p0) FP64
     float4 *sgam = nullptr;          // Morton-sorted (Gx, Gy, Gz, p1) FP32
-    double4 *tbnd = nullptr;         // per 256-slot tile of the sorted field:
+    double4 *tbnd = nullptr;         // per tile of the sorted field (256 slots mixed, 64 FP64):
                                      // (centre, radius), (largest sigma, -, -, -)
-    // split source ranges of small launches: partial sums (up to 15 per slot
+    // split source ranges of small launches: partial sums (up to 14 per slot
     // per segment; kcap doubles)
     int64_t kcap = 0;
     double *kpart = nullptr;

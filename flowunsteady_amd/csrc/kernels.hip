@@ -22,6 +22,7 @@
 namespace vpmx {
 
 constexpr int UJ_BLOCK = 256;
+constexpr int UJ64_TG = 64;        // targets per workgroup of the FP64 pair kernels
 constexpr int EW_BLOCK = 256;      // elementwise kernels
 constexpr int RED_BLOCKS = 1024;   // partial-sum blocks of the reductions
 
@@ -48,70 +49,125 @@ __global__ __launch_bounds__(EW_BLOCK) void pack_f64_kernel(const double *__rest
     out[2 * i + 1] = make_double4(G[cap + i], G[2 * cap + i], s, 1.0 / s);
 }
 
-template <int K, bool DS>
+// Targets: SORTED, the slots of the source records themselves (results stored
+// through perm, tile bounds tb for the far-field test); otherwise the SoA X of
+// stride cap, results stored in place (perm, tb unused).  64 targets per
+// workgroup of four waves (uj_f64_sums).
+template <int K, bool DS, bool SORTED>
+__device__ __forceinline__ void uj_f64_target(const double4 *__restrict__ src,
+                                              const double *__restrict__ X, int64_t t0,
+                                              int64_t nt, int64_t cap, double &xi, double &yi,
+                                              double &zi)
+{
+    // lanes past the last target repeat it
+    const int64_t i = min(t0 + (int64_t)(threadIdx.x % UJ64_TG), nt - 1);
+    if constexpr (SORTED) {
+        const double4 p = src[2 * i];
+        xi = p.x; yi = p.y; zi = p.z;
+    } else {
+        xi = X[i]; yi = X[cap + i]; zi = X[2 * cap + i];
+    }
+}
+
+template <int K, bool DS, bool SORTED>
 __global__ __launch_bounds__(UJ_BLOCK) void uj_f64_kernel(const double4 *__restrict__ src,
                                                           int64_t ns,
                                                           const double *__restrict__ X,
                                                           int64_t nt, int64_t cap,
+                                                          const double4 *__restrict__ tb,
+                                                          const int32_t *__restrict__ perm,
                                                           double *__restrict__ U,
                                                           double *__restrict__ J, int reset)
 {
     __shared__ double4 tile[2 * UJ_BLOCK];
-    const int64_t t0 = (int64_t)blockIdx.x * UJ_BLOCK;
-    uj_f64_block<K, UJ_BLOCK, DS>(src, 0, ns, X, t0, nt, cap, U, J, reset, tile);
+    const int64_t t0 = (int64_t)blockIdx.x * UJ64_TG;
+    double xi, yi, zi, d[15];
+    uj_f64_target<K, DS, SORTED>(src, X, t0, nt, cap, xi, yi, zi);
+    uj_f64_sums<K, UJ_BLOCK, UJ64_TG, DS>(src, 0, ns, xi, yi, zi, SORTED ? tb : nullptr, tile, d);
+    const int64_t s = t0 + threadIdx.x;
+    if (threadIdx.x < UJ64_TG && s < nt) {
+        double v[12];
+        uj_f64_values(d, v);
+        uj_f64_store(v, SORTED ? (int64_t)perm[s] : s, cap, U, J, reset);
+    }
 }
 
 // Split source range: workgroup (block b, segment g) sums sources
-// [g seglen, (g+1) seglen) for target block b into part[(g 12 + k) pld + i].
-template <int K, bool DS>
+// [g seglen, (g+1) seglen) for target block b into part[(g 12 + k) pld + slot].
+template <int K, bool DS, bool SORTED>
 __global__ __launch_bounds__(UJ_BLOCK) void uj_f64_split_kernel(const double4 *__restrict__ src,
                                                                 int64_t ns,
                                                                 const double *__restrict__ X,
                                                                 int64_t nt, int64_t cap,
+                                                                const double4 *__restrict__ tb,
                                                                 int64_t seglen, int nseg,
                                                                 double *__restrict__ part,
                                                                 int64_t pld)
 {
     __shared__ double4 tile[2 * UJ_BLOCK];
     const int g = (int)(blockIdx.x % nseg);
-    const int64_t t0 = (int64_t)(blockIdx.x / nseg) * UJ_BLOCK;
+    const int64_t t0 = (int64_t)(blockIdx.x / nseg) * UJ64_TG;
     const int64_t s0 = (int64_t)g * seglen;
     const int64_t s1 = s0 + seglen < ns ? s0 + seglen : ns;
-    double d[12];
-    uj_f64_sums<K, UJ_BLOCK, DS>(src, s0, s1, X, t0, nt, cap, tile, d);
-    const int64_t i = t0 + threadIdx.x;
-    if (i < nt)
-        for (int k = 0; k < 12; ++k) part[((int64_t)g * 12 + k) * pld + i] = d[k];
+    double xi, yi, zi, d[15];
+    uj_f64_target<K, DS, SORTED>(src, X, t0, nt, cap, xi, yi, zi);
+    uj_f64_sums<K, UJ_BLOCK, UJ64_TG, DS>(src, s0, s1, xi, yi, zi, SORTED ? tb : nullptr, tile, d);
+    const int64_t s = t0 + threadIdx.x;
+    if (threadIdx.x < UJ64_TG && s < nt) {
+        double v[12];
+        uj_f64_values(d, v);
+        for (int k = 0; k < 12; ++k) part[((int64_t)g * 12 + k) * pld + s] = v[k];
+    }
 }
 
-// Segments of each target added in segment order (bitwise repeatable).
+// Segments of each target added in segment order (bitwise repeatable); slot s
+// is stored at perm[s], or at s when perm is NULL.
 __global__ __launch_bounds__(EW_BLOCK) void uj_f64_split_reduce_kernel(const double *__restrict__ part,
                                                                        int64_t pld, int nseg,
-                                                                       int64_t nt, int64_t ldo,
+                                                                       int64_t nt,
+                                                                       const int32_t *__restrict__ perm,
+                                                                       int64_t ldo,
                                                                        double *__restrict__ U,
                                                                        double *__restrict__ J,
                                                                        int reset)
 {
-    const int64_t i = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
-    if (i >= nt) return;
-    double d[12];
-    for (int k = 0; k < 12; ++k) {
-        double v = 0.0;
-        for (int g = 0; g < nseg; ++g) v += part[((int64_t)g * 12 + k) * pld + i];
-        d[k] = v;
-    }
-    uj_f64_store(d, i, ldo, U, J, reset);
+    // component k of the targets in blockIdx.y = k: 12 x the threads of one
+    // per target, each with a chain of nseg loads
+    const int64_t s = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (s >= nt) return;
+    const int k = blockIdx.y;
+    double v = 0.0;
+    for (int g = 0; g < nseg; ++g) v += part[((int64_t)g * 12 + k) * pld + s];
+    const int64_t i = perm ? (int64_t)perm[s] : s;
+    double *o = k < 3 ? U + k * ldo + i : J + (k - 3) * ldo + i;
+    *o = reset ? v : *o + v;
+}
+
+// Split of an FP64 launch over nt targets and n sources: about 4096 workgroups
+// of 64 targets, so that the few that find near pairs everywhere even out
+// over the 256 CUs, in segments of at least 64 sources.  nseg nt stays below
+// 262,144 + 64 nseg, so the partials fit kpart.
+struct Split {
+    int nseg;
+    int64_t seglen;
+};
+
+static Split split_f64_for(int64_t nt, int64_t n)
+{
+    const int64_t nb = (nt + UJ64_TG - 1) / UJ64_TG;
+    int64_t nseg = std::min<int64_t>(4096 / std::max<int64_t>(nb, 1), (n + 63) / 64);
+    if (nseg <= 1) return {1, n};
+    int64_t seglen = (n + nseg - 1) / nseg;
+    // whole tiles of 256 where a segment holds several, whole runs of 64 otherwise
+    const int64_t q = seglen >= 2 * UJ_BLOCK ? UJ_BLOCK : 64;
+    seglen = (seglen + q - 1) / q * q;
+    return {(int)((n + seglen - 1) / seglen), seglen};
 }
 
 // How a launch over nb target blocks and n sources is split: when the target
 // blocks alone cannot fill the device, the source range is cut into segments
 // (multiples of UJ_BLOCK, at least four tiles each) so that about 1024
 // workgroups run; their partial sums go through `part` (SPLIT_PART doubles).
-struct Split {
-    int nseg;
-    int64_t seglen;
-};
-
 static Split split_for(int64_t nb, int64_t n)
 {
     if (nb >= 512 || n <= 4 * UJ_BLOCK) return {1, n};
@@ -129,24 +185,25 @@ hipError_t launch_pack_f64(hipStream_t st, const DeviceField &f, Scratch &s)
     return hipGetLastError();
 }
 
-template <int K, bool DS = false>
+template <int K, bool DS = false, bool SORTED = false>
 static hipError_t uj_f64_go(hipStream_t st, const double4 *src, int64_t ns, const double *X,
                             int64_t nt, int64_t cap, double *U, double *J, int reset,
-                            double *part)
+                            double *part, const double4 *tb = nullptr,
+                            const int32_t *perm = nullptr)
 {
-    const int64_t nb = (nt + UJ_BLOCK - 1) / UJ_BLOCK;
-    const Split sp = split_for(nb, ns);
+    const int64_t nb = (nt + UJ64_TG - 1) / UJ64_TG;
+    const Split sp = split_f64_for(nt, ns);
     if (sp.nseg == 1 || !part) {
-        uj_f64_kernel<K, DS><<<(unsigned)nb, UJ_BLOCK, 0, st>>>(src, ns, X, nt, cap, U, J, reset);
+        uj_f64_kernel<K, DS, SORTED><<<(unsigned)nb, UJ_BLOCK, 0, st>>>(src, ns, X, nt, cap, tb, perm,
+                                                                        U, J, reset);
         return hipGetLastError();
     }
-    uj_f64_split_kernel<K, DS><<<(unsigned)(nb * sp.nseg), UJ_BLOCK, 0, st>>>(src, ns, X, nt, cap,
-                                                                          sp.seglen, sp.nseg,
-                                                                          part, nt);
+    uj_f64_split_kernel<K, DS, SORTED><<<(unsigned)(nb * sp.nseg), UJ_BLOCK, 0, st>>>(
+        src, ns, X, nt, cap, tb, sp.seglen, sp.nseg, part, nt);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    uj_f64_split_reduce_kernel<<<grid_for(nt, EW_BLOCK), EW_BLOCK, 0, st>>>(part, nt, sp.nseg, nt,
-                                                                           cap, U, J, reset);
+    uj_f64_split_reduce_kernel<<<dim3(grid_for(nt, EW_BLOCK), 12), EW_BLOCK, 0, st>>>(
+        part, nt, sp.nseg, nt, perm, cap, U, J, reset);
     return hipGetLastError();
 }
 
@@ -197,99 +254,30 @@ __global__ __launch_bounds__(EW_BLOCK) void pack_f64_sorted_kernel(const double 
     out[2 * s + 1] = make_double4(G[cap + i], G[2 * cap + i], sig, 1.0 / sig);
 }
 
-// Bounds of each 256-slot tile of the sorted records: bbox centre, half
-// diagonal, largest sigma.  One workgroup per tile.
+// Bounds of each 64-slot run of the sorted records: bbox centre, half
+// diagonal, largest sigma.  One wave per run.
 __global__ __launch_bounds__(UJ_BLOCK) void tile_bounds_f64_kernel(const double4 *__restrict__ src,
                                                                    int64_t n,
                                                                    double4 *__restrict__ tb)
 {
-    __shared__ double red[7][UJ_BLOCK];
-    const int t = threadIdx.x;
-    const int64_t s = (int64_t)blockIdx.x * UJ_BLOCK + t;
-    double v[7] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY, 0.0};
-    if (s < n) {
-        const double4 p = src[2 * s];
-        v[0] = v[3] = p.x;
-        v[1] = v[4] = p.y;
-        v[2] = v[5] = p.z;
-        v[6] = src[2 * s + 1].z;
-    }
-    for (int k = 0; k < 7; ++k) red[k][t] = v[k];
-    __syncthreads();
-    for (int w = UJ_BLOCK / 2; w > 0; w >>= 1) {
-        if (t < w) {
-            for (int k = 0; k < 3; ++k) red[k][t] = fmin(red[k][t], red[k][t + w]);
-            for (int k = 3; k < 7; ++k) red[k][t] = fmax(red[k][t], red[k][t + w]);
+    const int64_t s = (int64_t)blockIdx.x * UJ_BLOCK + threadIdx.x;
+    const int64_t w = s / 64;
+    if (w * 64 >= n) return;   // whole waves leave
+    const int64_t i = min(s, n - 1);
+    const double4 p = src[2 * i];
+    double lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z}, sm = src[2 * i + 1].z;
+    for (int o = 32; o > 0; o >>= 1) {
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
+            hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
         }
-        __syncthreads();
+        sm = fmax(sm, __shfl_xor(sm, o));
     }
-    if (t == 0) {
-        const double hx = 0.5 * (red[3][0] - red[0][0]), hy = 0.5 * (red[4][0] - red[1][0]),
-                     hz = 0.5 * (red[5][0] - red[2][0]);
-        tb[2 * blockIdx.x] = make_double4(red[0][0] + hx, red[1][0] + hy, red[2][0] + hz,
-                                          sqrt(hx * hx + hy * hy + hz * hz));
-        tb[2 * blockIdx.x + 1] = make_double4(red[6][0], 0.0, 0.0, 0.0);
+    if ((threadIdx.x & 63) == 0) {
+        const double hx = 0.5 * (hi[0] - lo[0]), hy = 0.5 * (hi[1] - lo[1]), hz = 0.5 * (hi[2] - lo[2]);
+        tb[2 * w] = make_double4(lo[0] + hx, lo[1] + hy, lo[2] + hz, sqrt(hx * hx + hy * hy + hz * hz));
+        tb[2 * w + 1] = make_double4(sm, 0.0, 0.0, 0.0);
     }
-}
-
-template <int K>
-__global__ __launch_bounds__(UJ_BLOCK) void uj_f64s_kernel(const double4 *__restrict__ src,
-                                                           int64_t n,
-                                                           const double4 *__restrict__ tb,
-                                                           const int32_t *__restrict__ perm,
-                                                           int64_t cap, double *__restrict__ U,
-                                                           double *__restrict__ J, int reset)
-{
-    __shared__ double4 tile[2 * UJ_BLOCK];
-    const int64_t t0 = (int64_t)blockIdx.x * UJ_BLOCK;
-    double d[15];
-    uj_f64s_sums<K, UJ_BLOCK>(src, 0, n, t0, n, tb, tile, d);
-    const int64_t s = t0 + threadIdx.x;
-    if (s < n) uj_f64s_store(d, perm[s], cap, U, J, reset);
-}
-
-// Split source range: workgroup (block b, segment g) writes its 15 sums to
-// part[(g 15 + k) pld + slot].
-template <int K>
-__global__ __launch_bounds__(UJ_BLOCK) void uj_f64s_split_kernel(const double4 *__restrict__ src,
-                                                                 int64_t n,
-                                                                 const double4 *__restrict__ tb,
-                                                                 int64_t seglen, int nseg,
-                                                                 double *__restrict__ part,
-                                                                 int64_t pld)
-{
-    __shared__ double4 tile[2 * UJ_BLOCK];
-    const int g = (int)(blockIdx.x % nseg);
-    const int64_t t0 = (int64_t)(blockIdx.x / nseg) * UJ_BLOCK;
-    const int64_t s0 = (int64_t)g * seglen;
-    const int64_t s1 = s0 + seglen < n ? s0 + seglen : n;
-    double d[15];
-    uj_f64s_sums<K, UJ_BLOCK>(src, s0, s1, t0, n, tb, tile, d);
-    const int64_t s = t0 + threadIdx.x;
-    if (s < n)
-        for (int k = 0; k < 15; ++k) part[((int64_t)g * 15 + k) * pld + s] = d[k];
-}
-
-// Segments of each slot added in segment order (bitwise repeatable), stored
-// through perm.
-__global__ __launch_bounds__(EW_BLOCK) void uj_f64s_split_reduce_kernel(const double *__restrict__ part,
-                                                                        int64_t pld, int nseg,
-                                                                        int64_t n,
-                                                                        const int32_t *__restrict__ perm,
-                                                                        int64_t ldo,
-                                                                        double *__restrict__ U,
-                                                                        double *__restrict__ J,
-                                                                        int reset)
-{
-    const int64_t s = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
-    if (s >= n) return;
-    double d[15];
-    for (int k = 0; k < 15; ++k) {
-        double v = 0.0;
-        for (int g = 0; g < nseg; ++g) v += part[((int64_t)g * 15 + k) * pld + s];
-        d[k] = v;
-    }
-    uj_f64s_store(d, perm[s], ldo, U, J, reset);
 }
 
 hipError_t launch_pack_f64_sorted(hipStream_t st, const DeviceField &f, Scratch &s)
@@ -304,41 +292,21 @@ hipError_t launch_pack_f64_sorted(hipStream_t st, const DeviceField &f, Scratch 
     return hipGetLastError();
 }
 
-template <int K>
-static hipError_t uj_f64s_go(hipStream_t st, const DeviceField &f, const Scratch &s, int reset)
-{
-    const int64_t n = f.np;
-    const int64_t nb = (n + UJ_BLOCK - 1) / UJ_BLOCK;
-    const Split sp = split_for(nb, n);
-    if (sp.nseg == 1 || !s.kpart || (int64_t)sp.nseg * 15 * n > s.kcap) {
-        uj_f64s_kernel<K><<<(unsigned)nb, UJ_BLOCK, 0, st>>>(s.src64, n, s.tbnd, s.perm, f.cap,
-                                                             f.U, f.J, reset);
-        return hipGetLastError();
-    }
-    uj_f64s_split_kernel<K><<<(unsigned)(nb * sp.nseg), UJ_BLOCK, 0, st>>>(
-        s.src64, n, s.tbnd, sp.seglen, sp.nseg, s.kpart, n);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    uj_f64s_split_reduce_kernel<<<grid_for(n, EW_BLOCK), EW_BLOCK, 0, st>>>(
-        s.kpart, n, sp.nseg, n, s.perm, f.cap, f.U, f.J, reset);
-    return hipGetLastError();
-}
-
 hipError_t launch_uj_f64_sorted(hipStream_t st, int kernel, const DeviceField &f,
                                 const Scratch &s, int reset)
 {
-    if (f.np == 0) return hipSuccess;
+    const int64_t n = f.np;
+    if (n == 0) return hipSuccess;
+#define VPMX_UJ64S(KK) \
+    return uj_f64_go<KK, false, true>(st, s.src64, n, nullptr, n, f.cap, f.U, f.J, reset, s.kpart, s.tbnd, s.perm)
     switch (kernel) {
-    case SINGULAR: return uj_f64s_go<SINGULAR>(st, f, s, reset);
-    case GAUSSIAN: return uj_f64s_go<GAUSSIAN>(st, f, s, reset);
-    case GAUSSIANERF: return uj_f64s_go<GAUSSIANERF>(st, f, s, reset);
-    case WINCKELMANS:
-        // no far-field form (1 - g decays as rho^-4): the unsorted-target
-        // kernel over the sorted sources keeps its higher occupancy
-        return uj_f64_go<WINCKELMANS>(st, s.src64, f.np, f.X, f.np, f.cap, f.U, f.J, reset,
-                                      s.kpart);
+    case SINGULAR: VPMX_UJ64S(SINGULAR);
+    case GAUSSIAN: VPMX_UJ64S(GAUSSIAN);
+    case GAUSSIANERF: VPMX_UJ64S(GAUSSIANERF);
+    case WINCKELMANS: VPMX_UJ64S(WINCKELMANS);
     default: return hipErrorInvalidValue;
     }
+#undef VPMX_UJ64S
 }
 
 // Caller-owned device arrays (stride n) and a caller-provided scratch block:
@@ -351,7 +319,7 @@ static size_t uj_f64_dev_part_offset(int64_t n)
 
 size_t uj_f64_dev_scratch_bytes(int64_t n)
 {
-    const Split sp = split_for((n + UJ_BLOCK - 1) / UJ_BLOCK, n);
+    const Split sp = split_f64_for(n, n);
     const size_t part = sp.nseg > 1 ? (size_t)sp.nseg * 12 * (size_t)n * sizeof(double) : 0;
     return uj_f64_dev_part_offset(n) + part;
 }
@@ -371,17 +339,20 @@ hipError_t launch_uj_f64_dev(hipStream_t st, int kernel, int64_t n, const double
 }
 
 // Core-size derivatives D[U], D[J] of every particle into DU (3 x cap) and DJ
-// (9 x cap), FP64, from the source records of the UJ that just ran.
+// (9 x cap), FP64, from the sorted source records of the UJ that just ran.
 hipError_t launch_dsig_f64(hipStream_t st, int kernel, const DeviceField &f, const Scratch &s,
                            double *DU, double *DJ)
 {
     if (f.np == 0) return hipSuccess;
+#define VPMX_DS64(KK) \
+    return uj_f64_go<KK, true, true>(st, s.src64, f.np, nullptr, f.np, f.cap, DU, DJ, 1, s.kpart, nullptr, s.perm)
     switch (kernel) {
-    case GAUSSIAN: return uj_f64_go<GAUSSIAN, true>(st, s.src64, f.np, f.X, f.np, f.cap, DU, DJ, 1, s.kpart);
-    case GAUSSIANERF: return uj_f64_go<GAUSSIANERF, true>(st, s.src64, f.np, f.X, f.np, f.cap, DU, DJ, 1, s.kpart);
-    case WINCKELMANS: return uj_f64_go<WINCKELMANS, true>(st, s.src64, f.np, f.X, f.np, f.cap, DU, DJ, 1, s.kpart);
+    case GAUSSIAN: VPMX_DS64(GAUSSIAN);
+    case GAUSSIANERF: VPMX_DS64(GAUSSIANERF);
+    case WINCKELMANS: VPMX_DS64(WINCKELMANS);
     default: return hipErrorInvalidValue;
     }
+#undef VPMX_DS64
 }
 
 // ===========================================================================

@@ -11,210 +11,166 @@
 
 namespace vpmx {
 
-// FP64 source record pair (x, y, z, Gx) (Gy, Gz, sigma, 1/sigma), as written by
-// pack_f64_kernel.  Targets [t0, t1) read X (SoA, stride cap); sources
-// [s0, s1).  Reference pair algebra: src/FLOWUnsteady_processing_force.jl:888-905
-// extended to J = grad U.  `tile` holds 2*BLK records.  d = (U0..2, J0..8).
-// DS: the core-size derivatives D[U], D[J] instead (g, g' -> h, h').
-template <int K, int BLK, bool DS = false>
-__device__ __forceinline__ void uj_f64_sums(const double4 *__restrict__ src, int64_t s0,
-                                            int64_t s1, const double *__restrict__ X, int64_t t0,
-                                            int64_t t1, int64_t cap, double4 *tile, double d[12])
-{
-    const int t = threadIdx.x;
-    const int64_t i = t0 + t;
-    const bool active = i < t1;
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    if (active) {
-        xi = X[i];
-        yi = X[cap + i];
-        zi = X[2 * cap + i];
-    }
-    double u0 = 0, u1 = 0, u2 = 0;
-    double j0 = 0, j1 = 0, j2 = 0, j3 = 0, j4 = 0, j5 = 0, j6 = 0, j7 = 0, j8 = 0;
+// ---------------------------------------------------------------------------
+// FP64.  Source records (x, y, z, Gx) (Gy, Gz, sigma, 1/sigma).  The 15 sums
+// of a target are kept without the -1/(4 pi) factor:
+// d = (u 0..2, w = sum A Gamma 0..2, radial J 0..8 (k + 3 l)).
 
-    for (int64_t base = s0; base < s1; base += BLK) {
-        __syncthreads();
-        const int64_t js = base + t;
-        if (js < s1) {
-            tile[2 * t] = src[2 * js];
-            tile[2 * t + 1] = src[2 * js + 1];
-        }
-        __syncthreads();
-        const int cnt = (int)((s1 - base) < BLK ? (s1 - base) : BLK);
-        for (int jj = 0; jj < cnt; ++jj) {
-            const double4 a = tile[2 * jj], b = tile[2 * jj + 1];
-            const double dX1 = xi - a.x, dX2 = yi - a.y, dX3 = zi - a.z;
-            const double r2 = dX1 * dX1 + dX2 * dX2 + dX3 * dX3;
-            if (r2 > 0.0) {   // the reference skips r == 0
-                const double r = sqrt(r2);
-                double g, dg;
-                if constexpr (DS)
-                    h_dh_f64<K>(r * b.w, g, dg);
-                else
-                    g_dg_f64<K>(r * b.w, g, dg);
-                const double rinv = 1.0 / r;
-                const double r3i = rinv * rinv * rinv;
-                const double G1 = a.w, G2 = b.x, G3 = b.y;
-                const double c1 = -INV4PI * r3i * (dX2 * G3 - dX3 * G2);
-                const double c2 = -INV4PI * r3i * (dX3 * G1 - dX1 * G3);
-                const double c3 = -INV4PI * r3i * (dX1 * G2 - dX2 * G1);
-                u0 += g * c1;
-                u1 += g * c2;
-                u2 += g * c3;
-                const double aux = dg * b.w * rinv - 3.0 * g * rinv * rinv;
-                j0 += aux * c1 * dX1; j1 += aux * c2 * dX1; j2 += aux * c3 * dX1;
-                j3 += aux * c1 * dX2; j4 += aux * c2 * dX2; j5 += aux * c3 * dX2;
-                j6 += aux * c1 * dX3; j7 += aux * c2 * dX3; j8 += aux * c3 * dX3;
-                const double a2 = -INV4PI * g * r3i;
-                j1 -= a2 * G3;
-                j2 += a2 * G2;
-                j3 += a2 * G3;
-                j5 -= a2 * G1;
-                j6 -= a2 * G2;
-                j7 += a2 * G1;
-            }
-        }
-    }
-    d[0] = u0; d[1] = u1; d[2] = u2;
-    d[3] = j0; d[4] = j1; d[5] = j2; d[6] = j3; d[7] = j4; d[8] = j5;
-    d[9] = j6; d[10] = j7; d[11] = j8;
+// One pair with radial coefficients A, B added to the sums.
+__device__ __forceinline__ void f64_accumulate(const double4 a, const double4 b, double dx,
+                                               double dy, double dz, double A, double B,
+                                               double d[15])
+{
+    const double G1 = a.w, G2 = b.x, G3 = b.y;
+    const double c1 = fma(dy, G3, -dz * G2), c2 = fma(dz, G1, -dx * G3), c3 = fma(dx, G2, -dy * G1);
+    d[0] = fma(A, c1, d[0]); d[1] = fma(A, c2, d[1]); d[2] = fma(A, c3, d[2]);
+    d[3] = fma(A, G1, d[3]); d[4] = fma(A, G2, d[4]); d[5] = fma(A, G3, d[5]);
+    const double ex = B * dx, ey = B * dy, ez = B * dz;
+    d[6] = fma(c1, ex, d[6]); d[7] = fma(c2, ex, d[7]); d[8] = fma(c3, ex, d[8]);
+    d[9] = fma(c1, ey, d[9]); d[10] = fma(c2, ey, d[10]); d[11] = fma(c3, ey, d[11]);
+    d[12] = fma(c1, ez, d[12]); d[13] = fma(c2, ez, d[13]); d[14] = fma(c3, ez, d[14]);
 }
 
-// ---------------------------------------------------------------------------
-// FP64 on the Morton-sorted field.  Sources and targets are slots of the
-// sorted records (x, y, z, Gx) (Gy, Gz, sigma, 1/sigma) (pack_f64_sorted);
-// results go through perm.  The 15 sums are kept without the -1/(4 pi)
-// factor: d = (u 0..2, w = sum g r^-3 Gamma 0..2, radial J 0..8 (k + 3 l)).
-//
-// Far field: for the gaussian kernels 1 - g(rho) < 3e-19 and rho g'(rho)
-// < 2e-17 at rho >= 9.5, so g = 1 and g' = 0 to FP64 rounding there and the
-// pair is the singular one: no erf / exp / sqrt / division.  A source tile
-// whose gap to the target block is >= 9.5 sigma_max (> 0 for the singular
-// kernel) runs f64_pair_far for every pair; within other tiles a wave whose
-// every lane has rho^2 >= 90.25 for the current source takes it too.
-constexpr double RHO2_FAR_F64 = 90.25;
-constexpr double RHO_FAR_F64 = 9.5;
-
+// A pair known to be the singular one: for the gaussian kernels 1 - g(rho) <
+// 3e-19 and rho g'(rho) < 2e-17 at rho >= 9.5, so g = 1 and g' = 0 to FP64
+// rounding (no exp, no division).
 __device__ __forceinline__ void f64_pair_far(const double4 a, const double4 b, double xi,
                                              double yi, double zi, double d[15])
 {
-    const double dX1 = xi - a.x, dX2 = yi - a.y, dX3 = zi - a.z;
-    const double r2 = dX1 * dX1 + dX2 * dX2 + dX3 * dX3;
-    const double rinv = rsqrt(r2);
-    const double ri2 = rinv * rinv, r3i = ri2 * rinv;
-    const double G1 = a.w, G2 = b.x, G3 = b.y;
-    const double c1 = r3i * (dX2 * G3 - dX3 * G2);
-    const double c2 = r3i * (dX3 * G1 - dX1 * G3);
-    const double c3 = r3i * (dX1 * G2 - dX2 * G1);
-    d[0] += c1; d[1] += c2; d[2] += c3;
-    d[3] += r3i * G1; d[4] += r3i * G2; d[5] += r3i * G3;
-    const double aux = -3.0 * ri2;
-    const double e1 = aux * c1, e2 = aux * c2, e3 = aux * c3;
-    d[6] += e1 * dX1; d[7] += e2 * dX1; d[8] += e3 * dX1;
-    d[9] += e1 * dX2; d[10] += e2 * dX2; d[11] += e3 * dX2;
-    d[12] += e1 * dX3; d[13] += e2 * dX3; d[14] += e3 * dX3;
+    const double dx = xi - a.x, dy = yi - a.y, dz = zi - a.z;
+    const double rinv = rsq_f64(fma(dx, dx, fma(dy, dy, dz * dz)));
+    const double ri2 = rinv * rinv, A = ri2 * rinv;
+    f64_accumulate(a, b, dx, dy, dz, A, -3.0 * A * ri2, d);
 }
 
-// Full evaluation (reference pair algebra, src/FLOWUnsteady_processing_force.jl:888-905
-// extended to J); coincident pairs skipped.
-template <int K>
-__device__ __forceinline__ void f64_pair_full(const double4 a, const double4 b, double xi,
-                                              double yi, double zi, double d[15])
+// Any pair: the far form while every lane of the wave has rho^2 >= 90.25,
+// else the full evaluation; coincident pairs skipped
+// (src/FLOWUnsteady_processing_force.jl:895).  b.z holds pair_const_f64 here.
+// DS: the core-size derivatives D[U], D[J] in the same sums, which vanish
+// beyond rho^2 = 120 for the gaussian kernels.
+template <int K, bool DS>
+__device__ __forceinline__ void f64_pair(const double4 a, const double4 b, double xi, double yi,
+                                         double zi, double d[15])
 {
-    const double dX1 = xi - a.x, dX2 = yi - a.y, dX3 = zi - a.z;
-    const double r2 = dX1 * dX1 + dX2 * dX2 + dX3 * dX3;
-    if (!(r2 > 0.0)) return;   // the reference skips r == 0
-    const double r = sqrt(r2);
-    double g, dg;
-    g_dg_f64<K>(r * b.w, g, dg);
-    const double rinv = 1.0 / r;
-    const double ri2 = rinv * rinv, r3i = ri2 * rinv;
-    const double G1 = a.w, G2 = b.x, G3 = b.y;
-    const double c1 = r3i * (dX2 * G3 - dX3 * G2);
-    const double c2 = r3i * (dX3 * G1 - dX1 * G3);
-    const double c3 = r3i * (dX1 * G2 - dX2 * G1);
-    d[0] += g * c1; d[1] += g * c2; d[2] += g * c3;
-    const double gr = g * r3i;
-    d[3] += gr * G1; d[4] += gr * G2; d[5] += gr * G3;
-    const double aux = dg * b.w * rinv - 3.0 * g * ri2;
-    const double e1 = aux * c1, e2 = aux * c2, e3 = aux * c3;
-    d[6] += e1 * dX1; d[7] += e2 * dX1; d[8] += e3 * dX1;
-    d[9] += e1 * dX2; d[10] += e2 * dX2; d[11] += e3 * dX2;
-    d[12] += e1 * dX3; d[13] += e2 * dX3; d[14] += e3 * dX3;
-}
-
-// One target block (slots [t0, t1), t0 a multiple of BLK) against source
-// slots [s0, s1) (s0 a multiple of BLK).  tb: bounds of each BLK-slot tile
-// (centre, radius), (largest sigma, -, -, -).  `tile` holds 2 BLK records.
-template <int K, int BLK>
-__device__ __forceinline__ void uj_f64s_sums(const double4 *__restrict__ src, int64_t s0,
-                                             int64_t s1, int64_t t0, int64_t t1,
-                                             const double4 *__restrict__ tb, double4 *tile,
-                                             double d[15])
-{
-    const int t = threadIdx.x;
-    const int64_t s = t0 + t;
-    double xi = 0.0, yi = 0.0, zi = 0.0;
-    if (s < t1) {
-        const double4 p = src[2 * s];
-        xi = p.x;
-        yi = p.y;
-        zi = p.z;
-    }
-    const double4 T = tb[2 * (t0 / BLK)];
-    for (int k = 0; k < 15; ++k) d[k] = 0.0;
-    for (int64_t base = s0; base < s1; base += BLK) {
-        __syncthreads();
-        const int64_t js = base + t;
-        if (js < s1) {
-            tile[2 * t] = src[2 * js];
-            tile[2 * t + 1] = src[2 * js + 1];
+    const double dx = xi - a.x, dy = yi - a.y, dz = zi - a.z;
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const double x = r2 * (b.w * b.w);
+    if constexpr (K == GAUSSIANERF || K == GAUSSIAN) {
+        if (__all(x >= (DS ? X_CORE : X_FAR))) {
+            if constexpr (!DS) {
+                const double rinv = rsq_f64(r2), ri2 = rinv * rinv, A = ri2 * rinv;
+                f64_accumulate(a, b, dx, dy, dz, A, -3.0 * A * ri2, d);
+            }
+            return;
         }
+    }
+    if (!(r2 > 0.0)) return;
+    double A, B;
+    if constexpr (DS) {
+        radial_dsig_f64<K>(r2, x, b.w, b.z, A, B);
+    } else {
+        const double rinv = K == WINCKELMANS ? 0.0 : rsq_f64(r2);
+        radial_f64<K>(r2, x, rinv, rinv * rinv, b.w, b.z, A, B);
+    }
+    f64_accumulate(a, b, dx, dy, dz, A, B, d);
+}
+
+// The 15 sums of TG targets (thread t of the workgroup holds target
+// t % TG at (xi, yi, zi)) against source slots [s0, s1), staged through LDS NT
+// records at a time, the next tile loading while one computes.  With TG < NT
+// the workgroup's NT / TG waves of a target share each tile: slice t / TG takes
+// its NT / TG-th run of the records, and the slices are added in order at the
+// end (slice 0's threads hold the totals).  A field of n particles gives n / TG
+// workgroups that way, and with the split source ranges of small launches
+// enough of them to fill the 256 CUs from a few hundred particles on: with one
+// target per thread of 256 and segments of 1024 a field of 8,000 ran as 256
+// workgroups, one wave per SIMD (RK3 step with relaxation 2.90 -> 1.24 ms
+// together with the shorter pair; 601 particles, 0.50 -> 0.18 ms per UJ_gpu).
+//
+// With tile bounds `tb` (per 64 slots from slot 0: (centre, radius), (largest
+// sigma, -, -, -); TG = 64, s0 a multiple of 64) a run whose gap to the targets'
+// box is >= 9.5 sigma_max (> 0 for the singular kernel) takes f64_pair_far for
+// every pair without the per-pair test.
+template <int K, int NT, int TG, bool DS>
+__device__ __forceinline__ void uj_f64_sums(const double4 *__restrict__ src, int64_t s0,
+                                            int64_t s1, double xi, double yi, double zi,
+                                            const double4 *__restrict__ tb, double4 *tile,
+                                            double d[15])
+{
+    constexpr int SL = NT / TG;
+    static_assert(NT % TG == 0 && TG % 64 == 0, "whole waves per slice");
+    const int t = threadIdx.x, sl = t / TG;
+    double cx = 0.0, cy = 0.0, cz = 0.0, rad = 0.0;
+    if (tb) {   // box of the wave's 64 targets
+        double lo[3] = {xi, yi, zi}, hi[3] = {xi, yi, zi};
+        for (int o = 32; o > 0; o >>= 1)
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
+                hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
+            }
+        const double hx = 0.5 * (hi[0] - lo[0]), hy = 0.5 * (hi[1] - lo[1]), hz = 0.5 * (hi[2] - lo[2]);
+        cx = lo[0] + hx;
+        cy = lo[1] + hy;
+        cz = lo[2] + hz;
+        rad = sqrt(hx * hx + hy * hy + hz * hz);
+    }
+    for (int k = 0; k < 15; ++k) d[k] = 0.0;
+    double4 ra = make_double4(0.0, 0.0, 0.0, 0.0), rb = make_double4(0.0, 0.0, 1.0, 1.0);
+    if (s0 + t < s1) {
+        ra = src[2 * (s0 + t)];
+        rb = src[2 * (s0 + t) + 1];
+    }
+    for (int64_t base = s0; base < s1; base += NT) {
         __syncthreads();
-        const int cnt = (int)((s1 - base) < BLK ? (s1 - base) : BLK);
+        tile[2 * t] = ra;
+        tile[2 * t + 1] = make_double4(rb.x, rb.y, pair_const_f64<K>(rb.z, rb.w), rb.w);
+        __syncthreads();
+        const int64_t js = base + NT + t;
+        if (js < s1) {
+            ra = src[2 * js];
+            rb = src[2 * js + 1];
+        }
+        // this slice's run of the tile: TG records, or its share of a partial tile
+        const int have = (int)(s1 - base < NT ? s1 - base : NT);
+        const int run = have == NT ? TG : (have + SL - 1) / SL;
+        const int j0 = sl * run, cnt = min(run, have - j0);   // may be <= 0
         bool far = false;
-        if constexpr (K == GAUSSIANERF || K == GAUSSIAN || K == SINGULAR) {
-            if (cnt == BLK) {
-                const int64_t ts = base / BLK;
+        if constexpr (!DS && TG == 64 && K != WINCKELMANS) {
+            if (tb && have == NT) {
+                const int64_t ts = (base + j0) / TG;
                 const double4 S = tb[2 * ts];
-                const double ex = S.x - T.x, ey = S.y - T.y, ez = S.z - T.z;
-                const double gap = sqrt(ex * ex + ey * ey + ez * ez) - S.w - T.w;
-                if constexpr (K == SINGULAR)
-                    far = gap > 0.0;
-                else
-                    far = gap >= RHO_FAR_F64 * tb[2 * ts + 1].x;
+                const double ex = S.x - cx, ey = S.y - cy, ez = S.z - cz;
+                const double gap = sqrt(ex * ex + ey * ey + ez * ez) - S.w - rad;
+                far = K == SINGULAR ? gap > 0.0 : gap >= RHO_FAR * tb[2 * ts + 1].x;
             }
         }
+        const double4 *tj = tile + 2 * j0;
         if (far) {
 #pragma unroll 2
-            for (int jj = 0; jj < BLK; ++jj)
-                f64_pair_far(tile[2 * jj], tile[2 * jj + 1], xi, yi, zi, d);
+            for (int jj = 0; jj < TG; ++jj) f64_pair_far(tj[2 * jj], tj[2 * jj + 1], xi, yi, zi, d);
         } else {
-            for (int jj = 0; jj < cnt; ++jj) {
-                const double4 a = tile[2 * jj], b = tile[2 * jj + 1];
-                bool lane_far = false;
-                if constexpr (K == GAUSSIANERF || K == GAUSSIAN) {
-                    const double dX1 = xi - a.x, dX2 = yi - a.y, dX3 = zi - a.z;
-                    const double rho2 = (dX1 * dX1 + dX2 * dX2 + dX3 * dX3) * (b.w * b.w);
-                    lane_far = rho2 >= RHO2_FAR_F64;
-                }
-                if (__all(lane_far))
-                    f64_pair_far(a, b, xi, yi, zi, d);
-                else
-                    f64_pair_full<K>(a, b, xi, yi, zi, d);
-            }
+            for (int jj = 0; jj < cnt; ++jj)
+                f64_pair<K, DS>(tj[2 * jj], tj[2 * jj + 1], xi, yi, zi, d);
+        }
+    }
+    if constexpr (SL > 1) {   // the slices of a target, added in slice order
+        double *red = reinterpret_cast<double *>(tile);
+        static_assert(15 * TG <= 8 * NT, "a slice's sums fit the tile");
+        for (int s = 1; s < SL; ++s) {
+            __syncthreads();
+            if (sl == s)
+                for (int k = 0; k < 15; ++k) red[k * TG + t % TG] = d[k];
+            __syncthreads();
+            if (sl == 0)
+                for (int k = 0; k < 15; ++k) d[k] += red[k * TG + t];
         }
     }
 }
 
-// U and J of particle i (stride ldo) from the 15 sums of uj_f64s_sums.
-__device__ __forceinline__ void uj_f64s_store(const double d[15], int64_t i, int64_t ldo,
-                                              double *__restrict__ U, double *__restrict__ J,
-                                              int reset)
+// The 12 values (U, J column-major) of a target from its 15 sums.
+__device__ __forceinline__ void uj_f64_values(const double d[15], double v[12])
 {
     const double k = -INV4PI;
-    double v[12];
     v[0] = k * d[0]; v[1] = k * d[1]; v[2] = k * d[2];
     v[3] = k * d[6];
     v[4] = k * (d[7] - d[5]);
@@ -225,30 +181,15 @@ __device__ __forceinline__ void uj_f64s_store(const double d[15], int64_t i, int
     v[9] = k * (d[12] - d[4]);
     v[10] = k * (d[13] + d[3]);
     v[11] = k * d[14];
-    for (int q = 0; q < 3; ++q) U[q * ldo + i] = reset ? v[q] : U[q * ldo + i] + v[q];
-    for (int q = 0; q < 9; ++q) J[q * ldo + i] = reset ? v[3 + q] : J[q * ldo + i] + v[3 + q];
 }
 
-// U and J of target i (stride ldo) from the 12 FP64 sums.
-__device__ __forceinline__ void uj_f64_store(const double d[12], int64_t i, int64_t ldo,
+// U and J of target i (stride ldo) from its 12 values.
+__device__ __forceinline__ void uj_f64_store(const double v[12], int64_t i, int64_t ldo,
                                              double *__restrict__ U, double *__restrict__ J,
                                              int reset)
 {
-    for (int k = 0; k < 3; ++k) U[k * ldo + i] = reset ? d[k] : U[k * ldo + i] + d[k];
-    for (int k = 0; k < 9; ++k) J[k * ldo + i] = reset ? d[3 + k] : J[k * ldo + i] + d[3 + k];
-}
-
-template <int K, int BLK, bool DS = false>
-__device__ __forceinline__ void uj_f64_block(const double4 *__restrict__ src, int64_t s0,
-                                             int64_t s1, const double *__restrict__ X,
-                                             int64_t t0, int64_t t1, int64_t cap,
-                                             double *__restrict__ U, double *__restrict__ J,
-                                             int reset, double4 *tile)
-{
-    double d[12];
-    uj_f64_sums<K, BLK, DS>(src, s0, s1, X, t0, t1, cap, tile, d);
-    const int64_t i = t0 + threadIdx.x;
-    if (i < t1) uj_f64_store(d, i, cap, U, J, reset);
+    for (int k = 0; k < 3; ++k) U[k * ldo + i] = reset ? v[k] : U[k * ldo + i] + v[k];
+    for (int k = 0; k < 9; ++k) J[k * ldo + i] = reset ? v[3 + k] : J[k * ldo + i] + v[3 + k];
 }
 
 // Mixed precision: the 14 FP64 sums of one target block against sources
