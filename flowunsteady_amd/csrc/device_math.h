@@ -93,29 +93,6 @@ __device__ __forceinline__ double eta_f64(double rho)
 // algebra of U and J with (g, g') replaced by (h, h'); in radial-coefficient
 // form A_D = h/r^3 = -4 pi zeta/sigma^3 and B_D = -4 pi zeta'/(rho sigma^5),
 // both finite at r = 0 and negligible beyond the core (no far field).
-template <int K>
-__device__ __forceinline__ void h_dh_f64(double rho, double &h, double &dh)
-{
-    if constexpr (K == GAUSSIANERF) {
-        const double e = exp(-0.5 * rho * rho);
-        const double r2 = rho * rho;
-        h = -SQRT2_PI * r2 * rho * e;
-        dh = -SQRT2_PI * r2 * (3.0 - r2) * e;
-    } else if constexpr (K == GAUSSIAN) {
-        const double r3 = rho * rho * rho;
-        const double e = exp(-r3);
-        h = -3.0 * r3 * e;
-        dh = -9.0 * rho * rho * (1.0 - r3) * e;
-    } else if constexpr (K == WINCKELMANS) {
-        const double r2 = rho * rho, q = r2 + 1.0;
-        const double q72 = q * q * q * sqrt(q);
-        h = -7.5 * r2 * rho / q72;
-        dh = -7.5 * (3.0 * r2 - 7.0 * r2 * r2 / q) / q72;
-    } else {
-        h = 0.0;
-        dh = 0.0;
-    }
-}
 
 // zeta(rho) and zD(rho) together (one exp).
 template <int K>
@@ -248,10 +225,12 @@ __device__ __forceinline__ double pair_const_f64(double sigma, double is)
 }
 
 // A and B of a pair with r2 > 0, x = r2/sigma^2, rinv = 1/r, ri2 = rinv^2;
-// is = 1/sigma, kz = pair_const_f64.
-template <int K>
+// is = 1/sigma, kz = pair_const_f64.  DYN: also the core-size derivatives
+// A_D, B_D of radial_dsig_f64, which share the exponential (or the root).
+template <int K, bool DYN = false>
 __device__ __forceinline__ void radial_f64(double r2, double x, double rinv, double ri2, double is,
-                                           double kz, double &A, double &B)
+                                           double kz, double &A, double &B, double *AD = nullptr,
+                                           double *BD = nullptr)
 {
     if constexpr (K == GAUSSIANERF) {
         const double E = exp_mhalf(x);
@@ -263,19 +242,34 @@ __device__ __forceinline__ void radial_f64(double r2, double x, double rinv, dou
             const double p = horner_f64(GERF_SMALL, x) * kz;
             A = x < X_SMALL ? p : A;
         }
-        B = fma(-3.0, A, E * kz) * ri2;
+        const double e = E * kz;
+        B = fma(-3.0, A, e) * ri2;
+        if constexpr (DYN) {
+            *AD = -e;
+            *BD = e * (is * is);
+        }
     } else if constexpr (K == GAUSSIAN) {
         const double rho = r2 * rinv * is;
-        const double e = exp_mhalf(2.0 * rho * rho * rho);
-        A = (1.0 - e) * (ri2 * rinv);
-        B = fma(-3.0, A, e * kz) * ri2;
+        const double E = exp_mhalf(2.0 * rho * rho * rho), e = E * kz;
+        A = (1.0 - E) * (ri2 * rinv);
+        B = fma(-3.0, A, e) * ri2;
+        if constexpr (DYN) {
+            *AD = -e;
+            *BD = 3.0 * rho * e * (is * is);
+        }
     } else if constexpr (K == WINCKELMANS) {   // s^2 = r^2 + sigma^2: exact rewrite of the closed forms
-        const double si = rsq_f64(r2 + kz), si2 = si * si, si5 = si2 * si2 * si;
+        const double si = rsq_f64(r2 + kz), si2 = si * si, si5 = si2 * si2 * si, si7 = si5 * si2;
         A = fma(2.5, kz, r2) * si5;
-        B = -3.0 * fma(3.5, kz, r2) * (si5 * si2);
+        B = -3.0 * fma(3.5, kz, r2) * si7;
+        if constexpr (DYN) {
+            const double s7 = kz * kz * si7;
+            *AD = -7.5 * s7;
+            *BD = 52.5 * s7 * si2;
+        }
     } else {
         A = ri2 * rinv;
         B = -3.0 * A * ri2;
+        if constexpr (DYN) *AD = *BD = 0.0;
     }
 }
 

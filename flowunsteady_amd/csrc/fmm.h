@@ -251,12 +251,13 @@ hipError_t launch_fmm_zeta(hipStream_t st, const FmmState &S, int kernel, const 
 hipError_t launch_fmm_pse(hipStream_t st, const FmmState &S, int kernel, const DeviceField &f,
                           const Scratch &s, double nu, double4 *rec);
 // Core-size derivatives D[U] (3 x cap) and D[J] (9 x cap) over the near-field
-// lists of the last FMM evaluation (overwritten; the far field has none).
-hipError_t launch_fmm_dsig(hipStream_t st, const FmmState &S, int kernel, int precision,
-                           const DeviceField &f, const Scratch &s, double *DU, double *DJ);
+// lists of the last FMM evaluation, mixed path (overwritten; the far field has
+// none).  The FP64 path takes D[J] in the evaluation itself (launch_fmm_eval).
+hipError_t launch_fmm_dsig_mixed(hipStream_t st, const FmmState &S, int kernel,
+                                 const DeviceField &f, const Scratch &s, double *DU, double *DJ);
 
 // Near-field work items of the current lists (S.chunks, S.nchunk, S.nslot;
-// S.part sized for 14 values per slot).  nleaf = S.plan.nleaves.
+// S.part sized for 21 values per slot).  nleaf = S.plan.nleaves.
 hipError_t fmm_p2p_chunks(hipStream_t st, FmmState &S, int64_t nleaf);
 
 // Dual tree traversal on the device: fills m2l_off/m2l_src and p2p_off/p2p_src
@@ -289,7 +290,8 @@ hipError_t launch_fmm_sort(hipStream_t st, void *tmp, size_t bytes, const uint64
                            uint64_t *kout, const int32_t *vin, int32_t *perm, int64_t n);
 hipError_t launch_fmm_gather(hipStream_t st, const DeviceField &f, const int32_t *perm,
                              double4 *rec, double *ssig);
+// DJ (9 x cap, FP64 only): also the core-size derivative D[J] over the near lists.
 hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, int kernel,
-                           int precision, const DeviceField &f, int reset);
+                           int precision, const DeviceField &f, int reset, double *DJ);
 
 }  // namespace vpmx

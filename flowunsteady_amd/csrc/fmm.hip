@@ -36,6 +36,7 @@
 #include "device_math.h"
 #include "fmm.h"
 #include "internal.h"
+#include "uj_block.h"
 
 namespace vpmx {
 
@@ -897,12 +898,17 @@ __global__ __launch_bounds__(P2P_BLOCK) void l2p_kernel(const int32_t *__restric
 }
 
 // Stores of the near-field kernels, shared with the reduction of partial sums:
-// FP64 P2P sums d = (U, J) added to U, J.
-__device__ __forceinline__ void p2p_f64_finish(const double d[12], int64_t i, int64_t cap,
-                                               double *__restrict__ U, double *__restrict__ J)
+// FP64 P2P values d = (U, J) added to U, J; NV = 21: followed by D[J], which
+// overwrites DJ (every particle belongs to exactly one leaf).
+template <int NV>
+__device__ __forceinline__ void p2p_f64_finish(const double *d, int64_t i, int64_t cap,
+                                               double *__restrict__ U, double *__restrict__ J,
+                                               double *__restrict__ DJ)
 {
     for (int k = 0; k < 3; ++k) U[k * cap + i] += d[k];
     for (int k = 0; k < 9; ++k) J[k * cap + i] += d[3 + k];
+    if constexpr (NV == 21)
+        for (int k = 0; k < 9; ++k) DJ[k * cap + i] = d[12 + k];
 }
 
 // Mixed P2P sums d = (U, W, J0..7) before -1/(4 pi): U and J added to U, J
@@ -921,85 +927,6 @@ __device__ __forceinline__ void p2p_mixed_finish(const double d[14], int64_t i, 
     J[6 * cap + i] += k * (d[12] - d[4]);
     J[7 * cap + i] += k * (d[13] + d[3]);
     J[8 * cap + i] += -k * (d[6] + d[10]);
-}
-
-// P2P near field, FP64: one block (one wave) per work item (a target leaf and
-// a run of its list), one target per lane, source leaves staged through LDS.
-// Adds to U, J (or writes partial sums).  DS: the core-size derivatives D[U],
-// D[J] instead (g, g' -> h, h'), added to U, J as given.
-template <int KK, bool DS = false>
-__global__ __launch_bounds__(P2P_BLOCK) void p2p_f64_kernel(const P2PChunk *__restrict__ chunks,
-                                                            const FmmCellDev *__restrict__ cells,
-                                                            const int32_t *__restrict__ src,
-                                                            const double4 *__restrict__ rec,
-                                                            const int32_t *__restrict__ perm,
-                                                            int64_t cap, double *__restrict__ U,
-                                                            double *__restrict__ J,
-                                                            double *__restrict__ part,
-                                                            int64_t pstride)
-{
-    __shared__ double4 tile[2 * P2P_BLOCK];
-    const P2PChunk ch = chunks[blockIdx.x];
-    const int c = ch.c;
-    const FmmCellDev A = cells[c];
-    for (int tb = A.begin; tb < A.end; tb += P2P_BLOCK) {
-        const int it = tb + threadIdx.x;
-        const bool active = it < A.end;
-        double xi = 0, yi = 0, zi = 0;
-        if (active) {
-            const double4 a = rec[2 * it];
-            xi = a.x; yi = a.y; zi = a.z;
-        }
-        double u0 = 0, u1 = 0, u2 = 0, j0 = 0, j1 = 0, j2 = 0, j3 = 0, j4 = 0, j5 = 0, j6 = 0,
-               j7 = 0, j8 = 0;
-        for (int64_t e = ch.e0; e < ch.e1; e++) {
-            const FmmCellDev B = cells[src[e]];
-            for (int sb = B.begin; sb < B.end; sb += P2P_BLOCK) {
-                __syncthreads();
-                const int js = sb + threadIdx.x;
-                if (js < B.end) {
-                    tile[2 * threadIdx.x] = rec[2 * js];
-                    tile[2 * threadIdx.x + 1] = rec[2 * js + 1];
-                }
-                __syncthreads();
-                const int cnt = min(P2P_BLOCK, B.end - sb);
-                for (int jj = 0; jj < cnt; ++jj) {
-                    const double4 a = tile[2 * jj], b = tile[2 * jj + 1];
-                    const double dX1 = xi - a.x, dX2 = yi - a.y, dX3 = zi - a.z;
-                    const double r2 = dX1 * dX1 + dX2 * dX2 + dX3 * dX3;
-                    if (r2 > 0.0) {
-                        const double r = sqrt(r2);
-                        double g, dg;
-                        if constexpr (DS)
-                            h_dh_f64<KK>(r * b.w, g, dg);
-                        else
-                            g_dg_f64<KK>(r * b.w, g, dg);
-                        const double rinv = 1.0 / r;
-                        const double r3i = rinv * rinv * rinv;
-                        const double G1 = a.w, G2 = b.x, G3 = b.y;
-                        const double c1 = -INV4PI * r3i * (dX2 * G3 - dX3 * G2);
-                        const double c2 = -INV4PI * r3i * (dX3 * G1 - dX1 * G3);
-                        const double c3 = -INV4PI * r3i * (dX1 * G2 - dX2 * G1);
-                        u0 += g * c1; u1 += g * c2; u2 += g * c3;
-                        const double aux = dg * b.w * rinv - 3.0 * g * rinv * rinv;
-                        j0 += aux * c1 * dX1; j1 += aux * c2 * dX1; j2 += aux * c3 * dX1;
-                        j3 += aux * c1 * dX2; j4 += aux * c2 * dX2; j5 += aux * c3 * dX2;
-                        j6 += aux * c1 * dX3; j7 += aux * c2 * dX3; j8 += aux * c3 * dX3;
-                        const double a2 = -INV4PI * g * r3i;
-                        j1 -= a2 * G3; j2 += a2 * G2; j3 += a2 * G3;
-                        j5 -= a2 * G1; j6 -= a2 * G2; j7 += a2 * G1;
-                    }
-                }
-            }
-        }
-        if (active) {
-            const double d[12] = {u0, u1, u2, j0, j1, j2, j3, j4, j5, j6, j7, j8};
-            if (ch.part < 0)
-                p2p_f64_finish(d, perm[it], cap, U, J);
-            else
-                for (int k = 0; k < 12; ++k) part[k * pstride + ch.part + (it - A.begin)] = d[k];
-        }
-    }
 }
 
 // P2P near field, mixed: FP32 pair math on coordinates relative to the
@@ -1047,6 +974,149 @@ __device__ __forceinline__ int stream_particle(const int32_t *lbeg, const int32_
         if (lpre[mid] <= q) lo = mid; else hi = mid;
     }
     return lbeg[lo] + (q - lpre[lo]);
+}
+
+// P2P near field, FP64: one wave per work item (a target leaf and a run of its
+// list), the source leaves streamed through LDS and the targets of small
+// leaves replicated as in p2p_mixed_kernel: a leaf holds ncrit / 2 particles on
+// average, so with one target per lane half of them idled.  R = 64 / nt slices
+// (at most 16); their values are added in slice order by lane reads.  Adds to
+// U, J (or writes partial sums).  DYN: the core-size derivative D[J] of the
+// dynamic SFS model in the same pass, which shares the separation, the
+// exponential and the cross product; a pass of its own cost 0.69 of this one.
+// Its R is at most 2: the model's quotient of two small sums shows how far a
+// sum's rounding depends on its order.  After two steps of a 20,000-particle
+// blob the CPU FMM (one sum per target, list order) is 1.3e-12 of max |Gamma|
+// off its own terms added in long double, this kernel 8e-13 (R <= 16: 7e-13,
+// one lane per target: 1.9e-12), and R <= 2 keeps the two within 1e-12 of each
+// other; leaves of ncrit = 50 mostly take R = 2 in any case.
+// Bound by FP64 issue (91 instructions per pair, 112 with D[J]).  Rotor wakes,
+// p = 4, per UJ: 200,003 particles 21.0 -> 7.5 ms; 100,003 with D[J]
+// 13.1 + 9.0 -> 6.6 ms.
+//
+// J is summed with its Kronecker part A eps_klm G_m pair by pair: the two parts
+// of near pairs largely cancel, and summed apart (as the direct kernels do, 3
+// instructions less) J carried 1.3 times the rounding error.
+__device__ __forceinline__ void p2p_f64_j(const double c[3], double dx, double dy, double dz,
+                                          double A, double B, double G1, double G2, double G3,
+                                          double (&j)[9])
+{
+    const double ex = B * dx, ey = B * dy, ez = B * dz;
+    j[0] = fma(c[0], ex, j[0]);
+    j[1] = fma(-A, G3, fma(c[1], ex, j[1]));
+    j[2] = fma(A, G2, fma(c[2], ex, j[2]));
+    j[3] = fma(A, G3, fma(c[0], ey, j[3]));
+    j[4] = fma(c[1], ey, j[4]);
+    j[5] = fma(-A, G1, fma(c[2], ey, j[5]));
+    j[6] = fma(-A, G2, fma(c[0], ez, j[6]));
+    j[7] = fma(A, G1, fma(c[1], ez, j[7]));
+    j[8] = fma(c[2], ez, j[8]);
+}
+
+// One pair; sums without the -1/(4 pi) factor.
+template <int KK, bool DYN>
+__device__ __forceinline__ void p2p_f64_pair(const double4 a, const double4 b, double xi, double yi,
+                                             double zi, double (&u)[3], double (&j)[9],
+                                             double (&dj)[9])
+{
+    const double dx = xi - a.x, dy = yi - a.y, dz = zi - a.z;
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const double x = r2 * (b.w * b.w);
+    bool far = false;
+    if constexpr (KK == GAUSSIANERF || KK == GAUSSIAN) far = __all(x >= X_FAR);
+    double A, B, AD = 0.0, BD = 0.0;
+    if (far) {
+        const double rinv = rsq_f64(r2), ri2 = rinv * rinv;
+        A = ri2 * rinv;
+        B = -3.0 * A * ri2;
+    } else {
+        if (!(r2 > 0.0)) return;   // coincident pairs are skipped
+        const double rinv = KK == WINCKELMANS ? 0.0 : rsq_f64(r2);
+        radial_f64<KK, DYN>(r2, x, rinv, rinv * rinv, b.w, b.z, A, B, &AD, &BD);
+    }
+    const double G1 = a.w, G2 = b.x, G3 = b.y;
+    const double c[3] = {fma(dy, G3, -dz * G2), fma(dz, G1, -dx * G3), fma(dx, G2, -dy * G1)};
+    for (int k = 0; k < 3; ++k) u[k] = fma(A, c[k], u[k]);
+    p2p_f64_j(c, dx, dy, dz, A, B, G1, G2, G3, j);
+    if constexpr (DYN)
+        if (!far) p2p_f64_j(c, dx, dy, dz, AD, BD, G1, G2, G3, dj);
+}
+
+template <int KK, bool DYN>
+__global__ __launch_bounds__(P2P_BLOCK) __attribute__((amdgpu_waves_per_eu(DYN ? 2 : 4)))
+void p2p_f64_kernel(
+    const P2PChunk *__restrict__ chunks, const FmmCellDev *__restrict__ cells,
+    const int32_t *__restrict__ src, const double4 *__restrict__ rec,
+    const int32_t *__restrict__ perm, int64_t cap, double *__restrict__ U, double *__restrict__ J,
+    double *__restrict__ DJ, double *__restrict__ part, int64_t pstride)
+{
+    constexpr int NV = DYN ? 21 : 12;
+    __shared__ double4 tile[2 * P2P_BLOCK];
+    __shared__ int32_t lbeg[P2P_SLOTS], lpre[P2P_SLOTS + 1];
+    const int lane = threadIdx.x;
+    const P2PChunk ch = chunks[blockIdx.x];
+    const FmmCellDev A = cells[ch.c];
+    for (int tb = A.begin; tb < A.end; tb += P2P_BLOCK) {
+        const int nt = min(P2P_BLOCK, A.end - tb);
+        const int R = min(P2P_BLOCK / nt, DYN ? 2 : 16);
+        const int sl0 = lane / nt;
+        const int t = lane - sl0 * nt;             // target of this lane
+        const int sl = sl0 < R ? sl0 : 0;          // its slice (lanes past R nt repeat slice 0)
+        double xi, yi, zi;
+        {
+            const double4 a = rec[2 * (tb + t)];
+            xi = a.x; yi = a.y; zi = a.z;
+        }
+        double u[3] = {0.0, 0.0, 0.0}, jm[9], dj[9];
+        for (int k = 0; k < 9; ++k) jm[k] = dj[k] = 0.0;
+        for (int64_t eb = ch.e0; eb < ch.e1; eb += P2P_SLOTS) {
+            const int nl = (int)min<int64_t>(P2P_SLOTS, ch.e1 - eb);
+            __syncthreads();
+            const int total = stream_setup(cells, src, eb, nl, lane, lbeg, lpre);
+            // the records of the next tile load while this one computes
+            double4 ra = make_double4(0.0, 0.0, 0.0, 0.0), rb = make_double4(0.0, 0.0, 1.0, 1.0);
+            if (lane < total) {
+                const int js = stream_particle(lbeg, lpre, nl, lane);
+                ra = rec[2 * js];
+                rb = rec[2 * js + 1];
+            }
+            for (int base = 0; base < total; base += P2P_BLOCK) {
+                __syncthreads();
+                tile[2 * lane] = ra;
+                tile[2 * lane + 1] = make_double4(rb.x, rb.y, pair_const_f64<KK>(rb.z, rb.w), rb.w);
+                __syncthreads();
+                const int qn = base + P2P_BLOCK + lane;
+                if (qn < total) {
+                    const int js = stream_particle(lbeg, lpre, nl, qn);
+                    ra = rec[2 * js];
+                    rb = rec[2 * js + 1];
+                }
+                const int cnt = min(P2P_BLOCK, total - base);
+                for (int j = sl; j < cnt; j += R)
+                    p2p_f64_pair<KK, DYN>(tile[2 * j], tile[2 * j + 1], xi, yi, zi, u, jm, dj);
+            }
+        }
+        double v[NV];
+        for (int k = 0; k < 3; ++k) v[k] = -INV4PI * u[k];
+        for (int k = 0; k < 9; ++k) v[3 + k] = -INV4PI * jm[k];
+        if constexpr (DYN)
+            for (int k = 0; k < 9; ++k) v[12 + k] = -INV4PI * dj[k];
+        if (R > 1) {   // the slices of each target added in slice order
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                double w = v[k];
+                for (int s = 1; s < R; ++s) w += __shfl(v[k], t + s * nt);
+                v[k] = w;
+            }
+        }
+        if (lane < nt) {
+            if (ch.part < 0)
+                p2p_f64_finish<NV>(v, perm[tb + lane], cap, U, J, DJ);
+            else
+                for (int k = 0; k < NV; ++k)
+                    part[k * pstride + ch.part + (tb + lane - A.begin)] = v[k];
+        }
+    }
 }
 
 template <int KK, int R, bool DS>
@@ -1900,8 +1970,8 @@ __global__ __launch_bounds__(P2P_BLOCK) void fmm_estr_mixed_kernel(
 }
 
 // Partial sums of the leaves cut into several work items, added in item order
-// and stored.  MODE 0: FP64 P2P (12 sums), 1: mixed P2P (14), 2: Estr (3),
-// 3: Estr and D[E] (6).
+// and stored.  MODE 0: FP64 P2P (12 values), 1: mixed P2P (14), 2: Estr (3),
+// 3: Estr and D[E] (6), 4: FP64 P2P with D[J] (21; E carries DJ).
 template <int MODE>
 __global__ __launch_bounds__(P2P_BLOCK) void p2p_part_reduce_kernel(
     const int32_t *__restrict__ leaves, const int64_t *__restrict__ coff,
@@ -1909,7 +1979,7 @@ __global__ __launch_bounds__(P2P_BLOCK) void p2p_part_reduce_kernel(
     const double *__restrict__ part, int64_t pstride, const int32_t *__restrict__ perm,
     int64_t cap, double *__restrict__ U, double *__restrict__ J, double *__restrict__ E)
 {
-    constexpr int NV = MODE == 0 ? 12 : MODE == 1 ? 14 : MODE == 2 ? 3 : 6;
+    constexpr int NV = MODE == 0 ? 12 : MODE == 1 ? 14 : MODE == 2 ? 3 : MODE == 3 ? 6 : 21;
     const int64_t li = blockIdx.x;
     const int64_t n = coff[li + 1] - coff[li];
     if (n <= 1) return;
@@ -1922,8 +1992,8 @@ __global__ __launch_bounds__(P2P_BLOCK) void p2p_part_reduce_kernel(
         for (int64_t j = 0; j < n; ++j)
             for (int k = 0; k < NV; ++k) d[k] += part[k * pstride + pb + j * nt + t];
         const int64_t i = perm[A.begin + t];
-        if constexpr (MODE == 0)
-            p2p_f64_finish(d, i, cap, U, J);
+        if constexpr (MODE == 0 || MODE == 4)
+            p2p_f64_finish<NV>(d, i, cap, U, J, E);
         else if constexpr (MODE == 1)
             p2p_mixed_finish(d, i, cap, U, J);
         else if constexpr (MODE == 2)
@@ -1998,16 +2068,16 @@ hipError_t launch_fmm_estr(hipStream_t st, const FmmState &S, int kernel, int tr
                                  S.nslot, s.perm, f.cap, nullptr, nullptr, f.E);
 }
 
-// Core-size derivatives over the near-field lists: the P2P kernels in their
-// DS mode, adding into DU, DJ cleared first.
+// Core-size derivatives over the near-field lists, mixed path: the P2P kernel
+// in its DS mode, adding into DU, DJ cleared first.
 __global__ __launch_bounds__(FMM_BLOCK) void fmm_zero_kernel(double *__restrict__ p, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
     if (i < n) p[i] = 0.0;
 }
 
-hipError_t launch_fmm_dsig(hipStream_t st, const FmmState &S, int kernel, int precision,
-                           const DeviceField &f, const Scratch &s, double *DU, double *DJ)
+hipError_t launch_fmm_dsig_mixed(hipStream_t st, const FmmState &S, int kernel,
+                                 const DeviceField &f, const Scratch &s, double *DU, double *DJ)
 {
     if (f.np == 0) return hipSuccess;
     fmm_zero_kernel<<<gridn(3 * f.cap, FMM_BLOCK), FMM_BLOCK, 0, st>>>(DU, 3 * f.cap);
@@ -2018,13 +2088,8 @@ hipError_t launch_fmm_dsig(hipStream_t st, const FmmState &S, int kernel, int pr
     if (nleaf == 0 || S.nchunk == 0) return hipSuccess;
     const unsigned g = (unsigned)S.nchunk;
 #define VPMX_DS(KK)                                                                             \
-    if (precision == 0)                                                                         \
-        p2p_f64_kernel<KK, true><<<g, P2P_BLOCK, 0, st>>>(S.chunks, S.cells, S.p2p_src, s.src64, \
-                                                         s.perm, f.cap, DU, DJ, S.part, S.nslot); \
-    else                                                                                        \
-        p2p_mixed_kernel<KK, true><<<g, P2P_BLOCK, 0, st>>>(S.chunks, S.cells, S.p2p_src,       \
-                                                           s.src64, s.perm, f.cap, DU, DJ,       \
-                                                           S.part, S.nslot);
+    p2p_mixed_kernel<KK, true><<<g, P2P_BLOCK, 0, st>>>(S.chunks, S.cells, S.p2p_src, s.src64,   \
+                                                       s.perm, f.cap, DU, DJ, S.part, S.nslot)
     switch (kernel) {
     case GAUSSIAN: VPMX_DS(GAUSSIAN); break;
     case GAUSSIANERF: VPMX_DS(GAUSSIANERF); break;
@@ -2034,11 +2099,8 @@ hipError_t launch_fmm_dsig(hipStream_t st, const FmmState &S, int kernel, int pr
 #undef VPMX_DS
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return precision == 0
-               ? launch_part_reduce<0>(st, S.leaves, nleaf, S.chunk_off, S.part_base, S.cells,
-                                       S.part, S.nslot, s.perm, f.cap, DU, DJ, nullptr)
-               : launch_part_reduce<1>(st, S.leaves, nleaf, S.chunk_off, S.part_base, S.cells,
-                                       S.part, S.nslot, s.perm, f.cap, DU, DJ, nullptr);
+    return launch_part_reduce<1>(st, S.leaves, nleaf, S.chunk_off, S.part_base, S.cells, S.part,
+                                 S.nslot, s.perm, f.cap, DU, DJ, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -2930,7 +2992,7 @@ hipError_t fmm_p2p_chunks(hipStream_t st, FmmState &S, int64_t nleaf)
     S.nchunk = S.h_chunk_tot[0];
     S.nslot = S.h_chunk_tot[1];
     VPMX_CHK(grow(&S.chunks, S.cap_chunk, std::max<int64_t>(S.nchunk, 1), st));
-    VPMX_CHK(grow(&S.part, S.cap_part, std::max<int64_t>(14 * S.nslot, 1), st));
+    VPMX_CHK(grow(&S.part, S.cap_part, std::max<int64_t>(21 * S.nslot, 1), st));
     p2p_chunk_fill_kernel<<<gridn(nleaf, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
         S.leaves, nleaf, S.p2p_off, S.cells, S.chunk_off, S.part_base, S.chunks);
     return hipGetLastError();
@@ -3043,7 +3105,7 @@ static int m2l_mfma_grid(const void *fn, int P, int ncell)
 }
 
 hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, int kernel,
-                           int precision, const DeviceField &f, int reset)
+                           int precision, const DeviceField &f, int reset, double *DJ)
 {
     const int K = d.K, P = d.P;
     const size_t shK = sizeof(double) * 4 * K;
@@ -3119,9 +3181,14 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
         if (e != hipSuccess) return e;
         const unsigned g = (unsigned)d.nchunk;
 #define VPMX_P2P(KK)                                                                              \
-    if (precision == 0)                                                                           \
-        p2p_f64_kernel<KK><<<g, P2P_BLOCK, 0, st>>>(d.chunks, d.cells, d.p2p_src, d.rec, d.perm,   \
-                                                   f.cap, f.U, f.J, d.part, d.nslot);             \
+    if (precision == 0 && DJ)                                                                     \
+        p2p_f64_kernel<KK, true><<<g, P2P_BLOCK, 0, st>>>(d.chunks, d.cells, d.p2p_src, d.rec,     \
+                                                         d.perm, f.cap, f.U, f.J, DJ, d.part,     \
+                                                         d.nslot);                                \
+    else if (precision == 0)                                                                      \
+        p2p_f64_kernel<KK, false><<<g, P2P_BLOCK, 0, st>>>(d.chunks, d.cells, d.p2p_src, d.rec,    \
+                                                          d.perm, f.cap, f.U, f.J, nullptr,       \
+                                                          d.part, d.nslot);                       \
     else                                                                                          \
         p2p_mixed_kernel<KK><<<g, P2P_BLOCK, 0, st>>>(d.chunks, d.cells, d.p2p_src, d.rec, d.perm, \
                                                      f.cap, f.U, f.J, d.part, d.nslot);
@@ -3135,11 +3202,15 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
 #undef VPMX_P2P
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        e = precision == 0
-                ? launch_part_reduce<0>(st, d.leaves, d.nleaf, d.chunk_off, d.part_base, d.cells,
-                                        d.part, d.nslot, d.perm, f.cap, f.U, f.J, nullptr)
-                : launch_part_reduce<1>(st, d.leaves, d.nleaf, d.chunk_off, d.part_base, d.cells,
-                                        d.part, d.nslot, d.perm, f.cap, f.U, f.J, nullptr);
+        if (precision == 0 && DJ)
+            e = launch_part_reduce<4>(st, d.leaves, d.nleaf, d.chunk_off, d.part_base, d.cells,
+                                      d.part, d.nslot, d.perm, f.cap, f.U, f.J, DJ);
+        else if (precision == 0)
+            e = launch_part_reduce<0>(st, d.leaves, d.nleaf, d.chunk_off, d.part_base, d.cells,
+                                      d.part, d.nslot, d.perm, f.cap, f.U, f.J, nullptr);
+        else
+            e = launch_part_reduce<1>(st, d.leaves, d.nleaf, d.chunk_off, d.part_base, d.cells,
+                                      d.part, d.nslot, d.perm, f.cap, f.U, f.J, nullptr);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

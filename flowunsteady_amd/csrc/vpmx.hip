@@ -744,8 +744,10 @@ int fmm_reserve_n(vpmx_ctx *c, FmmState &S, int64_t n)
 }
 
 // One FMM UJ evaluation; lists_only: the tree, the traversal and the
-// near-field work items only (for the viscous sums), no evaluation.
-int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = false)
+// near-field work items only (for the viscous sums), no evaluation; DJ: also
+// the core-size derivative of J (FP64).
+int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = false,
+            double *DJ = nullptr)
 {
     MarkScope ms(c, lists_only ? "vpmx fmm lists" : "vpmx fmm uj");
     if (!c->fmm) c->fmm = new (std::nothrow) FmmState();
@@ -886,7 +888,7 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = f
     {
         TimedScope ts(c, T_FMM);
         MarkScope ms(c, "vpmx fmm evaluation");
-        VPMX_HIP(c, launch_fmm_eval(st, d, pl, P->kernel, P->precision, f, reset));
+        VPMX_HIP(c, launch_fmm_eval(st, d, pl, P->kernel, P->precision, f, reset, DJ));
     }
     VPMX_TRY(sync(c));
     S.stats[0] = t1 - t0;   // device tree build (wall, incl. its read-backs)
@@ -913,14 +915,16 @@ int enqueue_sort(vpmx_ctx *c)
 }
 
 // One UJ evaluation.  `sort` = false reuses the Morton order of the last sort
-// (a time step sorts once and keeps that order through its substeps).
-int enqueue_uj(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool sort = true)
+// (a time step sorts once and keeps that order through its substeps).  dsig: the
+// evaluation of a dynamic SFS stage (FP64 FMM: takes D[J] along).
+int enqueue_uj(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool sort = true, bool dsig = false)
 {
     const DeviceField &f = c->f;
     BatchState &B = c->b;
     if (P->fmm) {
         if (B.nfields) return fail(c, VPMX_EUNSUPPORTED, "the FMM does not run on batched fields");
-        return run_fmm(c, P, reset);
+        return run_fmm(c, P, reset, false,
+                       dsig && P->precision == VPMX_FP64 ? c->f.DJ() : nullptr);
     }
     MarkScope ms(c, "vpmx direct uj");
     if (B.nfields && (B.items_block != B.block || B.items_off != B.off))
@@ -969,15 +973,16 @@ int enqueue_estr(vpmx_ctx *c, const vpmx_uj_params *U, bool dyn = false)
 // Dynamic procedure: core-size derivatives D[U], D[J] of the field, with the
 // scheme and records of the stage's UJ (which must have just run).  The FMM's
 // far field uses the singular kernel and does not depend on sigma, so with
-// the FMM they are near-field sums over its P2P lists.
+// the FMM they are near-field sums over its P2P lists (FP64: taken along by the
+// stage's evaluation).
 int enqueue_dsig(vpmx_ctx *c, const vpmx_uj_params *U)
 {
+    if (U->fmm && U->precision == VPMX_FP64) return VPMX_OK;
     TimedScope ts(c, T_DSIG);
     DeviceField &f = c->f;
     if (U->fmm) {
         if (!c->fmm) return fail(c, VPMX_EINVAL, "the dynamic SFS with the FMM needs an FMM UJ first");
-        VPMX_HIP(c, launch_fmm_dsig(c->stream, *c->fmm, U->kernel, U->precision, f, c->s, f.DU(),
-                                    f.DJ()));
+        VPMX_HIP(c, launch_fmm_dsig_mixed(c->stream, *c->fmm, U->kernel, f, c->s, f.DU(), f.DJ()));
     } else if (U->precision == VPMX_FP64) {
         VPMX_HIP(c, launch_dsig_f64(c->stream, U->kernel, f, c->s, f.DU(), f.DJ()));
     } else {
@@ -1005,7 +1010,7 @@ int enqueue_step(vpmx_ctx *c, const vpmx_uj_params *U, const vpmx_step_params *S
     const int32_t *fid = c->b.nfields ? c->b.fid : nullptr;
     if (rk3) VPMX_HIP(c, launch_fill(c->stream, f.M, 7 * f.cap, 0.0));
     for (int s = 0; s < nst; ++s) {
-        VPMX_TRY(enqueue_uj(c, U, 1, false));
+        VPMX_TRY(enqueue_uj(c, U, 1, false, S->sfs == VPMX_SFS_DYNAMIC));
         if (S->sfs == VPMX_SFS_DYNAMIC) {
             VPMX_TRY(enqueue_dsig(c, U));
             VPMX_TRY(enqueue_estr(c, U, true));

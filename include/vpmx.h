@@ -319,7 +319,8 @@ int vpmx_set_graph(vpmx_ctx *ctx, int32_t on);
 /* Time every launch of the pairwise kernels with HIP events on the context's
  * stream.  which: 0 = UJ pair kernel, 1 = Estr pair kernel, 2 = fused update,
  * 3 = FMM device evaluation (P2M through P2P), 4 = graph replay of a whole step,
- * 5 = the dynamic SFS's core-size derivatives D[U], D[J]
+ * 5 = the dynamic SFS's core-size derivatives D[U], D[J] (with the FP64 FMM they
+ * are part of 3)
  * (the kernels inside a graph are not timed one by one).
  * Returns the summed milliseconds and the launch count since the last reset. */
 int vpmx_set_timing(vpmx_ctx *ctx, int32_t on);

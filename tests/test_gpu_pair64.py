@@ -5,6 +5,10 @@
   50-digit closed forms.  A and B carry a few roundings each (the polynomials'
   own errors are below 1e-17): U = A c is asked to 16 units of 2^-53, J (two
   terms of opposite sign) to 64.
+  Single-leaf FMM fields of every kind of lane packing (1 to 65 targets in a
+  leaf) against the all-pairs oracle, U, J <= 1e-12; a dynamic-SFS step, whose
+  near-field pass also sums D[J], with the numerator's average <= 1e-12 of its
+  largest value.
   Fields whose sizes straddle the 64-target workgroups, the 64- and 256-source
   runs and the segment splits against the oracle, <= 1e-12 as everywhere.
 """
@@ -77,3 +81,39 @@ def test_field_sizes_against_oracle(kernel, n):
         assert not vpm.get_U(pf).any() and not vpm.get_J(pf).any()
         return
     assert normwise(vpm.get_U(pf), U)[0] < 1e-12 and normwise(vpm.get_J(pf), J)[0] < 1e-12
+
+
+@pytest.mark.parametrize("kernel", ["gaussianerf", "gaussian", "winckelmans", "singular"])
+def test_fmm_leaf_sizes_against_oracle(kernel):
+    for n in (1, 2, 3, 4, 5, 7, 9, 12, 16, 17, 21, 22, 31, 32, 33, 50, 63, 64, 65, 70):
+        rng = np.random.default_rng(100 + n)
+        X, G = rng.uniform(-1, 1, (n, 3)), rng.normal(0, 1e-2, (n, 3))
+        s = rng.uniform(0.05, 0.4, n)
+        pf = make_field(X, G, s, kernel=kernel, fmm=vpm.FMM(p=2, ncrit=70, theta=0.4))
+        vpm.UJ_fmm_gpu(pf)
+        assert int(vpm._context(0).fmm_stats()["leaves"]) == 1
+        U, J = O.uj_direct(kernel, X, X, G, s)
+        if n == 1:
+            assert not vpm.get_U(pf).any() and not vpm.get_J(pf).any()
+            continue
+        eu, ej = normwise(vpm.get_U(pf), U)[0], normwise(vpm.get_J(pf), J)[0]
+        assert eu < 1e-12 and ej < 1e-12, (n, eu, ej)
+
+
+@pytest.mark.parametrize("kernel", ["gaussianerf", "gaussian", "winckelmans"])
+@pytest.mark.parametrize("n", [3, 20, 32, 33, 65])
+def test_fmm_dynamic_leaf_sizes_against_oracle(kernel, n):
+    rng = np.random.default_rng(200 + n)
+    X, G = rng.uniform(-1, 1, (n, 3)), rng.normal(0, 1e-2, (n, 3))
+    s = rng.uniform(0.2, 0.6, n)
+    pf = make_field(X, G, s, kernel=kernel, SFS=vpm.DynamicSFS(), relaxation=vpm.norelaxation,
+                    fmm=vpm.FMM(p=2, ncrit=70, theta=0.4))
+    pf.UJ = vpm.UJ_fmm_gpu
+    vpm.euler_gpu(pf, 1e-3)
+    P = O.make_params(kernel, True, "rVPM", sfs="dynamic")
+    F = O.Field(X, G, s)
+    O.euler_step(P, F, 1e-3, False)
+    C = pf.particles[vpm.C_INDEX, :n].T
+    for k in (1, 2):
+        assert np.abs(C[:, k] - F.C[:, k]).max() <= 1e-12 * np.abs(F.C[:, k]).max(), k
+    assert normwise(vpm.get_J(pf), F.J.reshape(n, 9))[0] < 1e-12
