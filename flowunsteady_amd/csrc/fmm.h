@@ -13,48 +13,76 @@ namespace vpmx {
 
 constexpr int FMM_MAX_P = 12;   // K = 455 <= 2 coefficients per thread of 256
 
-// M2L on the matrix cores (orders 1..M2L_MFMA_MAX_P): the operator of one
-// source, T[b][a] = E_{a+b} on the region |a| + |b| <= P, cut into 4 x 4 tiles
-// (rows b = 4 tb + 0..3, columns a = 4 ta + 0..3).  Coefficients are in graded
-// order, so the row length of b -- the number of a with |a| <= P - |b| -- only
-// falls with b: b-tile tb needs a-tiles 0 .. m2l_natile(P, tb) - 1, and a-tile
-// ta meets b-tiles 0 .. m2l_nrows(P, ta) - 1.  Tiles are numbered a-tile by
-// a-tile: tile (tb, ta) is m2l_base(P, ta) + tb.
+// M2L on the matrix cores (orders 1..M2L_MFMA_MAX_P).  Two bases:
+//
+// HARM: the derivatives E_k of 1/r satisfy E_{k+2z} = -(E_{k+2x} + E_{k+2y}), so
+// of the C(P+3, 3) Cartesian coefficients of a multipole or local expansion
+// only the (P+1)^2 with z exponent 0 or 1 are independent: the multipoles are
+// folded onto those before the translation and the locals unfolded after it,
+// which gives the same truncated sum.  At P = 8 the operator's region
+// |a| + |b| <= P then holds 1,365 instead of 3,003 entries, a column 81 instead
+// of 165, and E (whose indices a + b have z exponent <= 2) 109 instead of 165.
+// FULL: every coefficient.  Half the speed; kept for the mixed-precision steps
+// with an SFS model, whose stretching pass rounds differences of J to FP32: the
+// other basis' J differs by 1e-15, which flips a few of those roundings, and a
+// particle's Estr or C then moves by an FP32 ulp (up to 1e-7 of the largest of
+// 786,433) from one version of this library to the next.
+//
+// Coefficient order: graded; FULL as the Cartesian index (x, then y
+// descending); HARM degree n = indices n^2 .. n^2 + 2n: (n-j, j, 0), then
+// (n-1-j, j, 1).  E entries in graded order: FULL the same index; HARM degree n
+// from m2l_ebase(n): z exponents 0, 1, 2, each with y ascending.
+//
+// The operator of one source, T[b][a] = E_{a+b}, is cut into 4 x 4 tiles (rows
+// b = 4 tb + 0..3, columns a = 4 ta + 0..3).  The row length of b -- the number
+// of a with |a| <= P - |b| -- only falls with b: b-tile tb needs a-tiles
+// 0 .. m2l_natile(P, tb) - 1.
 constexpr int M2L_MFMA_MAX_P = 10;
 constexpr int m2l_ncoef(int p) { return p < 0 ? 0 : (p + 1) * (p + 2) * (p + 3) / 6; }
-constexpr int m2l_degree(int k)
+constexpr int m2l_dim(bool harm, int p)
+{
+    return p < 0 ? 0 : harm ? (p + 1) * (p + 1) : m2l_ncoef(p);
+}
+constexpr int m2l_degree(bool harm, int k)
 {
     int n = 0;
-    while (m2l_ncoef(n) <= k) ++n;
+    while (m2l_dim(harm, n) <= k) ++n;
     return n;
 }
-constexpr int m2l_ntile1(int P) { return (m2l_ncoef(P) + 3) / 4; }
-constexpr int m2l_natile(int P, int tb)
+// First E entry of degree n, and the number of entries up to degree P.
+constexpr int m2l_ebase(bool harm, int n)
 {
-    return 4 * tb < m2l_ncoef(P) ? (m2l_ncoef(P - m2l_degree(4 * tb)) + 3) / 4 : 0;
+    return harm ? (n == 0 ? 0 : 1 + 3 * (n - 1) * n / 2) : m2l_ncoef(n - 1);
 }
-constexpr int m2l_nrows(int P, int ta)
+constexpr int m2l_ne(bool harm, int P) { return m2l_ebase(harm, P + 1); }
+constexpr int m2l_ntile1(bool harm, int P) { return (m2l_dim(harm, P) + 3) / 4; }
+constexpr int m2l_natile(bool harm, int P, int tb)
+{
+    return 4 * tb < m2l_dim(harm, P)
+               ? (m2l_dim(harm, P - m2l_degree(harm, 4 * tb)) + 3) / 4 : 0;
+}
+constexpr int m2l_nrows(bool harm, int P, int ta)
 {
     int n = 0;
-    for (int tb = 0; tb < m2l_ntile1(P); ++tb)
-        if (m2l_natile(P, tb) > ta) ++n;
+    for (int tb = 0; tb < m2l_ntile1(harm, P); ++tb)
+        if (m2l_natile(harm, P, tb) > ta) ++n;
     return n;
-}
-constexpr int m2l_base(int P, int ta)
-{
-    int s = 0;
-    for (int t = 0; t < ta; ++t) s += m2l_nrows(P, t);
-    return s;
 }
 // Total tiles: sum over b-tiles of their a-tile counts (= sum of m2l_nrows).
-constexpr int m2l_ntiles(int P)
+constexpr int m2l_ntiles(bool harm, int P)
 {
     int s = 0;
-    for (int tb = 0; tb < m2l_ntile1(P); ++tb) s += m2l_natile(P, tb);
+    for (int tb = 0; tb < m2l_ntile1(harm, P); ++tb) s += m2l_natile(harm, P, tb);
     return s;
 }
 // Tile count padded to whole batches of 8 (the index table's row length).
-constexpr int m2l_ntiles8(int P) { return (m2l_ntiles(P) + 7) / 8 * 8; }
+constexpr int m2l_ntiles8(bool harm, int P) { return (m2l_ntiles(harm, P) + 7) / 8 * 8; }
+// Row length of a multipole as the kernel reads it: tiles in pairs, so that the
+// lane holding column entry `hi` of every tile reads two tiles (16 bytes) at
+// once: entry 4 ta + hi stands at 8 (ta / 2) + 2 hi + ta % 2.
+constexpr int m2l_hrow(bool harm, int P) { return 8 * ((m2l_ntile1(harm, P) + 1) / 2); }
+// Row length of the operator table (entries past m2l_ne are zero).
+constexpr int m2l_trow(bool harm, int P) { return (m2l_ne(harm, P) + 15) / 16 * 16; }
 
 struct FmmCellDev {
     int32_t begin, end, child0, nchild;
@@ -135,13 +163,17 @@ struct FmmTables {
     // of b; m2l_rounds = chunks per thread of a 256-thread block (1, 2, 4 or 8).
     std::vector<int> m2l_chunk, m2l_cfirst;
     int m2l_nchunk = 0, m2l_rounds = 1, m2l_chunk_len = 0;
-    // Matrix-core M2L (P <= M2L_MFMA_MAX_P): for element (row, k) of tile t, at
-    // (row + 4 k) m2l_ntiles8(P) + t, the index of a + b in E, or K (a zero
-    // slot) outside the region and in the padding; bscale[a] = (-1)^|a| / a!,
-    // lscale[b] = 1 / b!.
+    // Matrix-core M2L (1 <= P <= M2L_MFMA_MAX_P) in the basis m2l_harm: for element
+    // (row, k) of tile t, at (row + 4 k) m2l_ntiles8 + t, the byte offset of a + b
+    // in E, or of the zero slot after it outside the region and in the padding.
+    // Folding, CSR by basis index: multipole index a and coefficient (with
+    // (-1)^|a| / a!); unfolding, CSR by full index b: basis index and
+    // coefficient (with 1 / b!).
+    bool m2l_harm = true;
     std::vector<uint16_t> m2l_tile_idx;
-    std::vector<double> m2l_bscale, m2l_lscale;
-    std::vector<int> m2l_erec;   // 4 per k, packed as m2l_mfma_kernel reads them
+    std::vector<int> m2l_fold_off, m2l_fold_idx, m2l_unf_off, m2l_unf_idx;
+    std::vector<double> m2l_fold_coef, m2l_unf_coef;
+    std::vector<int> m2l_erec;   // 4 per E entry, packed as m2l_mfma_kernel reads them
 };
 
 // Tree + lists of one evaluation (host).
@@ -176,10 +208,13 @@ struct FmmDev {
     const int *m2l_cfirst = nullptr;
     int m2l_nchunk = 0, m2l_rounds = 1;
     const uint16_t *m2l_tile_idx = nullptr;
-    const double *m2l_bscale = nullptr, *m2l_lscale = nullptr;
+    const int *m2l_fold_off = nullptr, *m2l_fold_idx = nullptr, *m2l_unf_off = nullptr,
+              *m2l_unf_idx = nullptr;
+    const double *m2l_fold_coef = nullptr, *m2l_unf_coef = nullptr;
     const int4 *m2l_erec = nullptr;
     const int4 *ijk = nullptr;        // per cell (ix, iy, iz, level)
-    const double *etab = nullptr;     // M2L_TAB_ROWS x K operator rows
+    const double *etab = nullptr;     // M2L_TAB_ROWS x m2l_trow operator rows
+    bool m2l_harm = true;
     double ext = 1.0;                 // edge of the root cell
     // near-field work items (fmm_p2p_chunks)
     const P2PChunk *chunks = nullptr;
@@ -201,7 +236,9 @@ struct FmmState {
     int4 *m2l_chunks = nullptr;
     int *m2l_cfirst = nullptr;
     uint16_t *m2l_tile_idx = nullptr;
-    double *m2l_bscale = nullptr, *m2l_lscale = nullptr;
+    int *m2l_fold_off = nullptr, *m2l_fold_idx = nullptr, *m2l_unf_off = nullptr,
+        *m2l_unf_idx = nullptr;
+    double *m2l_fold_coef = nullptr, *m2l_unf_coef = nullptr;
     int4 *m2l_erec = nullptr;
     // near-field work items: per leaf chunk count / partial slots (scanned in
     // place into offsets, nleaf + 1 each), the items, the partial sums
@@ -225,9 +262,10 @@ struct FmmState {
     double *ssig = nullptr;
     uint8_t *sort_tmp = nullptr;
     size_t sort_bytes = 0;
-    // matrix-core M2L operator rows of order etab_p
+    // matrix-core M2L operator rows of order etab_p, basis etab_harm
     double *etab = nullptr;
     int etab_p = -1;
+    bool etab_harm = true, dev_tab_harm = true;
     // statistics of the last evaluation
     double stats[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     DttBufs dtt;
@@ -273,13 +311,13 @@ hipError_t fmm_traverse_device(hipStream_t st, FmmState &S, int64_t ncell, doubl
 hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncrit, FmmPlan &pl,
                                  int64_t *nc_out);
 void free_tree_bufs(TreeBufs &B);
-// The operator table of the matrix-core M2L for order P (1..M2L_MFMA_MAX_P),
-// built once per order from the uploaded recurrence records S.m2l_erec.
-hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P);
+// The operator table of the matrix-core M2L for order P (1..M2L_MFMA_MAX_P) and
+// basis, built once per order from the uploaded recurrence records S.m2l_erec.
+hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P, bool harm);
 
 void fmm_build_tree(FmmPlan &pl, const uint64_t *key, const double *ssig, int64_t n, int ncrit);
 void fmm_traverse(FmmPlan &pl, double theta, double sigcut);
-void fmm_build_tables(FmmTables &T, int P);
+void fmm_build_tables(FmmTables &T, int P, bool harm);
 void fmm_plan_host(FmmPlan &pl, int64_t n, const double *X, const double *sig, int ncrit,
                    double theta, double sigcut);
 

@@ -373,16 +373,30 @@ __global__ __launch_bounds__(FMM_BLOCK) void m2l_kernel(const FmmCellDev *__rest
 // ---------------------------------------------------------------------------
 // With E_k = d^k (1/|r|) (the raw derivatives, k! times the Taylor
 // coefficients), m'_a = (-1)^|a| m_a / a! and l'_b = b! l_b the translation is
-//     l'_b = sum_a E_{a+b} m'_a,   |a| + |b| <= P,
-// a K x K matrix (a Hankel matrix in the multi-index) times the 3 columns of
-// the source's multipole.  One wave owns one target cell and takes its sources
-// four at a time, one per block of v_mfma_f64_4x4x4f64 (four independent
-// 4 x 4 x 4 products): the A operand of block j is a tile of source j's matrix,
-// gathered from its E in LDS through the tile index table; B is the source's
-// m' (columns q = 0, 1, 2 and a zero fourth column); C accumulates l' of the
-// target over every source of the block, one 4 x 4 tile per b-tile, in
-// registers.  At the end the four blocks are added (fixed order) and scaled
-// by 1/b!.
+//     l'_b = sum_a E_{a+b} m'_a,   |a| + |b| <= P.
+// E is harmonic in its index, E_{k+2z} = -(E_{k+2x} + E_{k+2y}), so with every a
+// written as (i, j, r + 2 q), r = 0 or 1, the terms of one (i + 2t, j + 2(q-t), r)
+// add up beforehand (m2l_fold_kernel): sum_t (-1)^q C(q, t) m'_a; l' obeys the
+// same relation in b (same degrees, same truncation), so only b with z exponent
+// 0 or 1 is computed and the others follow (m2l_unfold_kernel).  What is left
+// is an H x H matrix, H = (P+1)^2, times the source's 3 columns.
+//
+// One wave owns one target cell and takes its sources four at a time, one per
+// block of v_mfma_f64_4x4x4f64 (four independent 4 x 4 x 4 products): the A
+// operand of block j is a tile of source j's matrix, gathered from its E in
+// LDS through the tile index table; B is the source's folded m' (columns
+// q = 0, 1, 2 and a zero fourth column); C accumulates l' of the target over
+// every source of the block, one 4 x 4 tile per b-tile, in registers.  At the
+// end the four blocks are added (fixed order).
+//
+// Bound by the LDS gathers (105 ds_read_b64 per group of four sources at P = 8,
+// about 6 cycles each) ahead of the MFMAs (105, 16 cycles on each of 4 SIMDs).
+// In the full Cartesian basis (215 tiles; C and B 84 registers each, two waves
+// per SIMD) the kernel was latency-bound at twice the work: blob of 786,433,
+// P = 8, 61.2 -> 27.6 ms per UJ; rotor wake of 1,000,003, core-aware, 28.4 ->
+// 12.0; rotor 200,003, P = 4, 2.20 -> 2.01.  The fold and unfold passes stream
+// the expansions once each.  (FULL, see fmm.h: the same kernel on the whole
+// basis.)
 //
 // Operand layouts of v_mfma_f64_4x4x4f64 (lane of element (row, k) of A,
 // (k, n) of B and (row, n) of C in block j): A at row + 4 j + 16 k, B at
@@ -391,22 +405,22 @@ __global__ __launch_bounds__(FMM_BLOCK) void m2l_kernel(const FmmCellDev *__rest
 // E of a source from the Taylor coefficients t_k = E_k / k! of 1/r, whose
 // recurrence (that of E_k divided by k!; the k_i factors cancel)
 //     n R^2 t_k = -(2n - 1) sum_i r_i t_{k - e_i} - (n - 1) sum_i t_{k - 2 e_i},
-// n = |k|, runs degree by degree, 16 lanes per source, in place; a last pass
-// multiplies by k!.
+// n = |k|, stays within z exponents <= 2 and runs degree by degree, 16 lanes
+// per source, in place; a last pass multiplies by k!.
 // Tile t -> (ta, tb), in the order the tile index table holds them.
-template <int P>
+template <int P, bool HARM>
 struct M2LTiles {
     struct Map {
-        int ta[m2l_ntiles8(P)], tb[m2l_ntiles8(P)];
+        int ta[m2l_ntiles8(HARM, P)], tb[m2l_ntiles8(HARM, P)];
     };
     static constexpr Map make()
     {
         Map m{};
-        int nat[m2l_ntile1(P)] = {};
-        for (int tb = 0; tb < m2l_ntile1(P); ++tb) nat[tb] = m2l_natile(P, tb);
+        int nat[m2l_ntile1(HARM, P)] = {};
+        for (int tb = 0; tb < m2l_ntile1(HARM, P); ++tb) nat[tb] = m2l_natile(HARM, P, tb);
         int t = 0;
-        for (int ta = 0; ta < m2l_ntile1(P); ++ta)
-            for (int tb = 0; tb < m2l_ntile1(P) && nat[tb] > ta; ++tb, ++t) {
+        for (int ta = 0; ta < m2l_ntile1(HARM, P); ++ta)
+            for (int tb = 0; tb < m2l_ntile1(HARM, P) && nat[tb] > ta; ++tb, ++t) {
                 m.ta[t] = ta;
                 m.tb[t] = tb;
             }
@@ -415,12 +429,12 @@ struct M2LTiles {
     static constexpr Map map = make();
 };
 
-template <int P, int T>
-__device__ __forceinline__ void m2l_mfma_one(double (&C)[m2l_ntile1(P)],
-                                             const double (&B)[m2l_ntile1(P)], double a)
+template <int P, bool HARM, int T>
+__device__ __forceinline__ void m2l_mfma_one(double (&C)[m2l_ntile1(HARM, P)],
+                                             const double (&B)[2 * ((m2l_ntile1(HARM, P) + 1) / 2)], double a)
 {
-    if constexpr (T < m2l_ntiles(P)) {
-        constexpr int ta = M2LTiles<P>::map.ta[T], tb = M2LTiles<P>::map.tb[T];
+    if constexpr (T < m2l_ntiles(HARM, P)) {
+        constexpr int ta = M2LTiles<P, HARM>::map.ta[T], tb = M2LTiles<P, HARM>::map.tb[T];
         C[tb] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, B[ta], C[tb], 0, 0, 0);
     }
 }
@@ -428,9 +442,9 @@ __device__ __forceinline__ void m2l_mfma_one(double (&C)[m2l_ntile1(P)],
 // Eight tiles: one 16-byte LDS read brings this lane's eight E byte offsets
 // (one 16-bit half each, so extracting and adding the row base is a single
 // instruction), then eight independent gathers of E feed eight MFMAs.
-template <int P, int T0, int... J>
-__device__ __forceinline__ void m2l_mfma_batch(double (&C)[m2l_ntile1(P)],
-                                               const double (&B)[m2l_ntile1(P)],
+template <int P, bool HARM, int T0, int... J>
+__device__ __forceinline__ void m2l_mfma_batch(double (&C)[m2l_ntile1(HARM, P)],
+                                               const double (&B)[2 * ((m2l_ntile1(HARM, P) + 1) / 2)],
                                                const uint16_t *tl, const char *Eb,
                                                std::integer_sequence<int, J...>)
 {
@@ -439,17 +453,17 @@ __device__ __forceinline__ void m2l_mfma_batch(double (&C)[m2l_ntile1(P)],
     double a[8];
     ((a[J] = *reinterpret_cast<const double *>(
           Eb + ((J & 1) ? (w[J >> 1] >> 16) : (w[J >> 1] & 0xffffu)))), ...);
-    (m2l_mfma_one<P, T0 + J>(C, B, a[J]), ...);
+    (m2l_mfma_one<P, HARM, T0 + J>(C, B, a[J]), ...);
 }
 
-template <int P, int T0>
-__device__ __forceinline__ void m2l_mfma_group(double (&C)[m2l_ntile1(P)],
-                                               const double (&B)[m2l_ntile1(P)],
+template <int P, bool HARM, int T0>
+__device__ __forceinline__ void m2l_mfma_group(double (&C)[m2l_ntile1(HARM, P)],
+                                               const double (&B)[2 * ((m2l_ntile1(HARM, P) + 1) / 2)],
                                                const uint16_t *tl, const char *Eb)
 {
-    if constexpr (T0 < m2l_ntiles(P)) {
-        m2l_mfma_batch<P, T0>(C, B, tl, Eb, std::make_integer_sequence<int, 8>{});
-        m2l_mfma_group<P, T0 + 8>(C, B, tl, Eb);
+    if constexpr (T0 < m2l_ntiles(HARM, P)) {
+        m2l_mfma_batch<P, HARM, T0>(C, B, tl, Eb, std::make_integer_sequence<int, 8>{});
+        m2l_mfma_group<P, HARM, T0 + 8>(C, B, tl, Eb);
     }
 }
 
@@ -463,7 +477,7 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-constexpr int m2l_erow(int P) { return (m2l_ncoef(P) + 1 + 31) / 32 * 32 + 8; }
+constexpr int m2l_erow(bool harm, int P) { return (m2l_ne(harm, P) + 1 + 31) / 32 * 32 + 8; }
 
 // 1 / ext^n for n = 0 .. M2L_MFMA_MAX_P + 1 (the scales of the M2L's
 // dimensionless expansions), by repeated products.
@@ -477,24 +491,57 @@ __device__ __forceinline__ void m2l_einv(double ext, double *einv)
     }
 }
 
-// M <- m'' = (-1)^|a| / a! m_a tau^-|a| in place, tau = ext 2^-(l+1) the half
-// width of the cell (level l), once the upward pass is done (the multipoles
-// have no reader after the M2L).  erec[k].w >> 24 = |k|.
-__global__ __launch_bounds__(FMM_BLOCK) void m2l_prescale_kernel(double *__restrict__ M, int64_t n,
-                                                                 int K,
-                                                                 const double *__restrict__ bscale,
-                                                                 const int4 *__restrict__ ijk,
-                                                                 const int4 *__restrict__ erec,
-                                                                 double ext)
+// Multipoles MH as the M2L reads them (rows of m2l_hrow doubles, 3 per cell,
+// entries in tile pairs): m'' = sum of (-1)^|a| / a! m_a tau^-|a| over the a
+// folded onto each basis index, tau = ext 2^-(l+1) the half width of the cell
+// (level l); one zero row per component after the last cell.
+template <bool HARM>
+__global__ __launch_bounds__(FMM_BLOCK) void m2l_fold_kernel(
+    const double *__restrict__ M, int64_t ncell, int K, int H, int HS,
+    const int *__restrict__ foff, const int *__restrict__ fidx, const double *__restrict__ fcoef,
+    const int4 *__restrict__ ijk, double ext, double *__restrict__ MH)
 {
     __shared__ double einv[M2L_MFMA_MAX_P + 2];
     if (threadIdx.x == 0) m2l_einv(ext, einv);
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const int k = (int)(i % K), dg = erec[k].w >> 24;
-    const int l = ijk[i / (3 * K)].w;
-    M[i] *= ldexp(bscale[k] * einv[dg], dg * (l + 1));
+    if (i >= (ncell + 1) * 3 * HS) return;
+    const int64_t row = i / HS;
+    const int p = (int)(i - row * HS), h = 4 * (2 * (p >> 3) + (p & 1)) + ((p & 7) >> 1);
+    double v = 0.0;
+    if (row < 3 * ncell && h < H) {
+        const double *m = M + row * K;
+        int dg = 0;
+        while (m2l_dim(HARM, dg) <= h) ++dg;
+        const int sh = dg * (ijk[row / 3].w + 1);
+        for (int e = foff[h]; e < foff[h + 1]; ++e)
+            v = fma(m[fidx[e]], ldexp(fcoef[e] * einv[dg], sh), v);
+    }
+    MH[i] = v;
+}
+
+// Local expansions L (rows of K) from the H values lambda per row:
+// l_b = tau^-(|b|+1) / b! sum of +-C(q, t) lambda_{unfolded b}.
+template <bool HARM>
+__global__ __launch_bounds__(FMM_BLOCK) void m2l_unfold_kernel(
+    const double *__restrict__ LH, int64_t nrow, int K, int H, const int *__restrict__ uoff,
+    const int *__restrict__ uidx, const double *__restrict__ ucoef, const int4 *__restrict__ ijk,
+    double ext, double *__restrict__ L)
+{
+    __shared__ double einv[M2L_MFMA_MAX_P + 2];
+    if (threadIdx.x == 0) m2l_einv(ext, einv);
+    __syncthreads();
+    const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
+    if (i >= nrow * K) return;
+    const int64_t row = i / K;
+    const int b = (int)(i - row * K);
+    int n = 1;   // |b| + 1
+    while (m2l_ncoef(n - 1) <= b) ++n;
+    const double sc = ldexp(einv[n], n * (ijk[row / 3].w + 1));
+    const double *l = LH + row * H;
+    double v = 0.0;
+    for (int e = uoff[b]; e < uoff[b + 1]; ++e) v = fma(l[uidx[e]], ucoef[e] * sc, v);
+    L[i] = v;
 }
 
 // One entry of the Taylor-coefficient recurrence from its six predecessors
@@ -545,13 +592,13 @@ __device__ __forceinline__ M2LPair m2l_pair(const int4 a, const int4 s)
     return p;
 }
 
-// Table rows E_k(v) 2^(dA (|k| + 1)), k < K, one thread per row (the zero
-// offset row holds zeros), by the recurrence of m2l_mfma_kernel.
-template <int P>
+// Table rows E_k(v) 2^(dA (|k| + 1)), k < m2l_ne, zeros up to m2l_trow, one
+// thread per row (the zero offset row holds zeros), by the recurrence of m2l_mfma_kernel.
+template <int P, bool HARM>
 __global__ __launch_bounds__(FMM_BLOCK) void m2l_etab_kernel(const int4 *__restrict__ erec,
                                                              double *__restrict__ tab)
 {
-    constexpr int K = m2l_ncoef(P);
+    constexpr int NE = m2l_ne(HARM, P), TR = m2l_trow(HARM, P);
     const int64_t row = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
     if (row >= M2L_TAB_ROWS) return;
     int64_t q = row;
@@ -561,96 +608,99 @@ __global__ __launch_bounds__(FMM_BLOCK) void m2l_etab_kernel(const int4 *__restr
     q /= M2L_TAB_W;
     const int vx = (int)(q % M2L_TAB_W) - M2L_TAB_V;
     const int dA = (int)(q / M2L_TAB_W);
-    double *t = tab + row * K;
+    double *t = tab + row * TR;
+    for (int k = NE; k < TR; ++k) t[k] = 0.0;
     if (vx == 0 && vy == 0 && vz == 0) {
-        for (int k = 0; k < K; ++k) t[k] = 0.0;
+        for (int k = 0; k < NE; ++k) t[k] = 0.0;
         return;
     }
     const double r0 = vx, r1 = vy, r2 = vz;
     const double R2 = r0 * r0 + r1 * r1 + r2 * r2, iR2 = 1.0 / R2;
     t[0] = 1.0 / sqrt(R2);
-    auto ld = [&](unsigned b) { return b == 8u * K ? 0.0 : t[b >> 3]; };
+    auto ld = [&](unsigned b) { return b == 8u * NE ? 0.0 : t[b >> 3]; };
     for (int n = 1; n <= P; ++n) {
         const double f1 = -(2.0 * n - 1.0) / n * iR2, f2 = -(n - 1.0) / n * iR2;
-        for (int k = m2l_ncoef(n - 1); k < m2l_ncoef(n); ++k) {
+        for (int k = m2l_ebase(HARM, n); k < m2l_ebase(HARM, n + 1); ++k) {
             const int4 e = erec[k];
             const unsigned qx = e.x, qy = e.y, qz = e.z;
             t[k] = m2l_taylor(f1, f2, r0, r1, r2, ld(qx & 0xffffu), ld(qx >> 16), ld(qy & 0xffffu),
                               ld(qy >> 16), ld(qz & 0xffffu), ld(qz >> 16));
         }
     }
-    for (int k = 0; k < K; ++k) t[k] *= m2l_kscale(erec[k].w, dA);
+    for (int k = 0; k < NE; ++k) t[k] *= m2l_kscale(erec[k].w, dA);
 }
 
 // Degree of entry 4 t + h (h = 0..3) of a column or row tile: base[t] +
 // (h >= step[t]) (a tile spans at most one degree boundary).
-template <int P>
+template <int P, bool HARM>
 struct M2LDeg {
     struct Map {
-        int base[m2l_ntile1(P)], step[m2l_ntile1(P)];
+        int base[m2l_ntile1(HARM, P)], step[m2l_ntile1(HARM, P)];
     };
     static constexpr Map make()
     {
         Map m{};
-        for (int t = 0; t < m2l_ntile1(P); ++t) {
-            m.base[t] = m2l_degree(4 * t);
+        for (int t = 0; t < m2l_ntile1(HARM, P); ++t) {
+            m.base[t] = m2l_degree(HARM, 4 * t);
             m.step[t] = 4;
             for (int h = 3; h >= 1; --h)
-                if (4 * t + h < m2l_ncoef(P) && m2l_degree(4 * t + h) > m.base[t]) m.step[t] = h;
+                if (4 * t + h < m2l_dim(HARM, P) && m2l_degree(HARM, 4 * t + h) > m.base[t])
+                    m.step[t] = h;
         }
         return m;
     }
     static constexpr Map map = make();
 };
 
-template <int P>
+template <int P, bool HARM>
 __device__ __forceinline__ int m2l_tile_degree(int t, int h)
 {
-    return M2LDeg<P>::map.base[t] + (h >= M2LDeg<P>::map.step[t] ? 1 : 0);
+    return M2LDeg<P, HARM>::map.base[t] + (h >= M2LDeg<P, HARM>::map.step[t] ? 1 : 0);
 }
 
 // Persistent: block b serves cells k G + (b mod 8) W + b / 8 (k = 0, 1, ...;
 // G = gridDim.x = 8 W), so each XCD (workgroups go round-robin over the 8
 // XCDs) sweeps contiguous runs of cells whose sources overlap in its L2, and
 // the tables are staged in LDS once per block.  `erec` packs, per k, the
-// byte offsets in a row of k - e_i and k - 2 e_i (8 K where absent: the zero
-// slot) and k! | |k| << 24: (j1x | j1y << 16, j1z | j2x << 16, j2y | j2z << 16,
+// byte offsets in a row of k - e_i and k - 2 e_i (the zero slot where absent)
+// and k! | |k| << 24: (j1x | j1y << 16, j1z | j2x << 16, j2y | j2z << 16,
 // k! | |k| << 24).
 //
 // Units: with u = ext 2^-(lf+1) (half the finer cell's width) a pair's
 // separation is u v, v integer, and E_k(u v) = u^-(|k|+1) E_k(v).  The
-// multipoles arrive as m''_a = m'_a tau_S^-|a| (m2l_prescale_kernel) and
+// multipoles arrive as m''_a = m'_a tau_S^-|a| (m2l_fold_kernel) and
 // the kernel accumulates lambda_b = sum_a Ehat_{a+b} m''_a 2^((l_A - l_S)|a|)
 // with Ehat_k = 2^(dA (|k|+1)) E_k(v) (dA = lf - l_A): l'_b =
-// tau_A^-(|b|+1) lambda_b, tau = the half width of each cell.  Ehat is copied
+// tau_A^-(|b|+1) lambda_b, tau = the half width of each cell (applied by
+// m2l_unfold_kernel).  Ehat is copied
 // from the operator table when all four sources of a group have rows there,
 // and otherwise built by the recurrence from v; the powers of two are exact.
 //
-// The four sources' E are rows of m2l_erow(P) doubles: K + 1 (the zero slot at
-// K), rounded so that the rows start 16 banks apart (the layout measured
+// The four sources' E are rows of m2l_erow(P) doubles: m2l_ne + 1 (the zero slot
+// last), rounded so that the rows start 16 banks apart (the layout measured
 // fastest among the ones tried).  Absent sources and the zero fourth B column
 // read the multipole row `zrow` (all zeros).
-template <int P>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(P <= 8 ? 2 : 1)))
+template <int P, bool HARM>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(HARM ? (P <= 8 ? 3 : 2) : (P <= 8 ? 2 : 1))))
 void m2l_mfma_kernel(
     const int4 *__restrict__ ijk, int ncell, const int64_t *__restrict__ off,
     const int32_t *__restrict__ src, const int4 *__restrict__ erec,
-    const uint16_t *__restrict__ tile_idx, const double *__restrict__ lscale,
-    const double *__restrict__ etab, double ext, const double *__restrict__ M, int64_t zrow,
-    double *__restrict__ L)
+    const uint16_t *__restrict__ tile_idx, const double *__restrict__ etab,
+    const double *__restrict__ MH, int64_t zrow, double *__restrict__ LH)
 {
-    constexpr int K = m2l_ncoef(P), NT = m2l_ntile1(P), N8 = m2l_ntiles8(P), ER = m2l_erow(P);
-    constexpr int MAXE = (K + 15) / 16;   // table entries per lane of a source's 16
-    __shared__ double E[4 * ER];
+    constexpr int H = m2l_dim(HARM, P), NE = m2l_ne(HARM, P), NT = m2l_ntile1(HARM, P);
+    constexpr int N8 = m2l_ntiles8(HARM, P), ER = m2l_erow(HARM, P), HS = m2l_hrow(HARM, P);
+    constexpr int TR = m2l_trow(HARM, P), NT2 = HS / 8;
+    constexpr int MAXE = (TR / 2 + 15) / 16;   // pairs of table entries per lane of a source's 16
+    static_assert(TR <= ER, "a table row fits an E row");
+    __shared__ __align__(16) double E[4 * ER];
     __shared__ __align__(16) uint16_t tab[16 * N8];
-    __shared__ int4 rec[K];
-    __shared__ double einv[M2L_MFMA_MAX_P + 2];
-    __shared__ double tsc[M2L_MFMA_MAX_P + 2];   // tau_A^-n of the current cell
+    __shared__ int4 rec[NE];
     const int lane = threadIdx.x;
     for (int i = lane; i < 16 * N8; i += 64) tab[i] = tile_idx[i];
-    for (int i = lane; i < K; i += 64) rec[i] = erec[i];
-    if (lane < 4) E[lane * ER + K] = 0.0;
-    if (lane == 0) m2l_einv(ext, einv);
+    for (int i = lane; i < NE; i += 64) rec[i] = erec[i];
+    if (lane < 4) E[lane * ER + NE] = 0.0;
     __syncthreads();
     const int nq = lane & 3, blk = (lane >> 2) & 3, hi = lane >> 4, sub = lane & 15;
     const uint16_t *tl = tab + (nq + 4 * hi) * N8;   // A element (row = lane & 3, k = lane >> 4)
@@ -661,8 +711,6 @@ void m2l_mfma_kernel(
     const int first = (int)(blockIdx.x & 7) * W + (int)(blockIdx.x >> 3);
     for (int c = first; c < ncell; c += G) {
         const int4 A = ijk[c];
-        wave_lds_sync();   // the previous cell's reads of tsc are done
-        if (lane <= P + 1) tsc[lane] = ldexp(einv[lane], lane * (A.w + 1));
         double Cacc[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) Cacc[t] = 0.0;
@@ -695,23 +743,30 @@ void m2l_mfma_kernel(
                 g.row = m2l_tab_row(0, 2, 0, 0);
             }
             const bool tabled = __all(g.hit);
-            double ev[MAXE];
+            double ev0[MAXE], ev1[MAXE];
             if (tabled) {
-                const double *er = etab + g.row * K;
+                const double2 *er = reinterpret_cast<const double2 *>(etab + g.row * TR);
 #pragma unroll
-                for (int it = 0; it < MAXE; ++it) ev[it] = er[min(sub + 16 * it, K - 1)];
+                for (int it = 0; it < MAXE; ++it) {
+                    const double2 v = er[min(sub + 16 * it, TR / 2 - 1)];
+                    ev0[it] = v.x;
+                    ev1[it] = v.y;
+                }
             }
             const int lsb = ijk[ib].w;   // level of source blk
-            // B operand: m''_blk[4 ta + k][n], k = lane >> 4, n = lane & 3.
-            // Every lane loads from a valid address and multiplies by a 0/1
-            // mask, so the loads issue back to back instead of one guarded
-            // load at a time (the multipoles are finite).
-            double Bv[NT];
-            const double *Mb =
-                M + ((blk < nb && nq < 3) ? (size_t)ib * 3 + nq : (size_t)zrow * 3) * K;
+            // B operand: m''_blk[4 ta + k][n], k = lane >> 4, n = lane & 3, two tiles
+            // per 16-byte load.  Every lane loads from a valid address (the
+            // zero row for absent sources and the fourth column), so the
+            // loads issue back to back.
+            double Bv[2 * NT2];
+            const double2 *Mb = reinterpret_cast<const double2 *>(
+                MH + ((blk < nb && nq < 3) ? (size_t)ib * 3 + nq : (size_t)zrow * 3) * HS);
 #pragma unroll
-            for (int ta = 0; ta < NT - 1; ++ta) Bv[ta] = Mb[4 * ta + hi];
-            Bv[NT - 1] = Mb[min(4 * (NT - 1) + hi, K - 1)] * (4 * (NT - 1) + hi < K ? 1.0 : 0.0);
+            for (int u = 0; u < NT2; ++u) {
+                const double2 m = Mb[4 * u + hi];
+                Bv[2 * u] = m.x;
+                Bv[2 * u + 1] = m.y;
+            }
             S = Sn;
             ie1 = ie2;
             ib = ib1;
@@ -720,23 +775,23 @@ void m2l_mfma_kernel(
             if (tabled) {
 #pragma unroll
                 for (int it = 0; it < MAXE; ++it) {
-                    const int k = sub + 16 * it;
-                    if (k < K) Ej[k] = ev[it];
+                    const int k = sub + 16 * it;   // the row's zero padding covers the zero slot
+                    if (k < TR / 2) reinterpret_cast<double2 *>(Ej)[k] = make_double2(ev0[it], ev1[it]);
                 }
             } else {
                 const double r0 = g.r0, r1 = g.r1, r2 = g.r2;
                 const double R2 = r0 * r0 + r1 * r1 + r2 * r2, iR2 = 1.0 / R2;
                 if (sub == 0) Ej[0] = 1.0 / sqrt(R2);
                 auto ld = [&](unsigned b) { return *reinterpret_cast<const double *>(Ejb + b); };
-                constexpr int MAXIT = ((P + 1) * (P + 2) / 2 + 15) / 16;
+                constexpr int MAXIT = ((HARM ? 3 * P : (P + 1) * (P + 2) / 2) + 15) / 16;
 #pragma unroll
                 for (int n = 1; n <= P; ++n) {
                     wave_lds_sync();
                     const double f1 = -(2.0 * n - 1.0) / n * iR2, f2 = -(n - 1.0) / n * iR2;
 #pragma unroll
                     for (int it = 0; it < MAXIT; ++it) {
-                        const int k = m2l_ncoef(n - 1) + sub + 16 * it;
-                        if (k < m2l_ncoef(n)) {
+                        const int k = m2l_ebase(HARM, n) + sub + 16 * it;
+                        if (k < m2l_ebase(HARM, n + 1)) {
                             const int4 q = rec[k];
                             const unsigned qx = q.x, qy = q.y, qz = q.z;
                             Ej[k] = m2l_taylor(f1, f2, r0, r1, r2, ld(qx & 0xffffu), ld(qx >> 16),
@@ -746,27 +801,25 @@ void m2l_mfma_kernel(
                     }
                 }
                 wave_lds_sync();
-                for (int k = sub; k < K; k += 16) Ej[k] *= m2l_kscale(rec[k].w, g.dA);
+                for (int k = sub; k < NE; k += 16) Ej[k] *= m2l_kscale(rec[k].w, g.dA);
             }
             // level gap of source blk: m''_a 2^((l_A - l_S) |a|), a = 4 ta + hi
             const int eB = A.w - lsb;
             if (__any(eB != 0)) {
 #pragma unroll
-                for (int ta = 0; ta < NT; ++ta) Bv[ta] = ldexp(Bv[ta], eB * m2l_tile_degree<P>(ta, hi));
+                for (int ta = 0; ta < NT; ++ta) Bv[ta] = ldexp(Bv[ta], eB * m2l_tile_degree<P, HARM>(ta, hi));
             }
             wave_lds_sync();
-            m2l_mfma_group<P, 0>(Cacc, Bv, tl, Eb);
+            m2l_mfma_group<P, HARM, 0>(Cacc, Bv, tl, Eb);
         }
-        // sum the four blocks (lanes 4 and 8 apart), scale by tau_A^-(|b|+1) / b!,
-        // write l
+        // sum the four blocks (lanes 4 and 8 apart), write lambda
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             double v = Cacc[t];
             v += __shfl_xor(v, 4);
             v += __shfl_xor(v, 8);
-            const int b = 4 * t + hi, dg = m2l_tile_degree<P>(t, hi);
-            const double ls = lscale[min(b, K - 1)] * tsc[dg + 1];
-            if (blk == 0 && nq < 3 && b < K) L[((size_t)c * 3 + nq) * K + b] = v * ls;
+            const int b = 4 * t + hi;
+            if (blk == 0 && nq < 3 && b < H) LH[((size_t)c * 3 + nq) * H + b] = v;
         }
     }
 }
@@ -1436,13 +1489,14 @@ void fmm_traverse(FmmPlan &pl, double theta, double sigcut)
 }
 
 // Operator tables for expansion order P (host build, uploaded once per P).
-void fmm_build_tables(FmmTables &T, int P)
+void fmm_build_tables(FmmTables &T, int P, bool harm)
 {
     MIndex M;
     M.build(P);
     const int K = M.K;
     T.P = P;
     T.K = K;
+    T.m2l_harm = harm;
     T.mi = M.mi;
     // derivative recurrence: idx(k - e_i), idx(k - 2 e_i)
     T.rec1.assign(4 * K, -1);
@@ -1538,53 +1592,92 @@ void fmm_build_tables(FmmTables &T, int P)
         T.m2l_rounds = best_rounds;
         T.m2l_chunk_len = best_len;
     }
-    // matrix-core M2L: scales and the E index of every tile element
-    {
+    // matrix-core M2L: folding onto the harmonic basis, E records, and the E
+    // offset of every tile element
+    T.m2l_fold_off.clear(); T.m2l_fold_idx.clear(); T.m2l_fold_coef.clear();
+    T.m2l_unf_off.clear(); T.m2l_unf_idx.clear(); T.m2l_unf_coef.clear();
+    T.m2l_erec.clear();
+    T.m2l_tile_idx.clear();
+    if (P >= 1 && P <= M2L_MFMA_MAX_P) {
         auto fact = [](int n) {
             double f = 1.0;
             for (int i = 2; i <= n; i++) f *= i;
             return f;
         };
-        T.m2l_bscale.assign(K, 0.0);
-        T.m2l_lscale.assign(K, 0.0);
+        const int H = m2l_dim(harm, P), NE = m2l_ne(harm, P), N8 = m2l_ntiles8(harm, P);
+        // basis index of (i, j, r), and E entry of (i, j, k) (-1 where an
+        // exponent is negative)
+        auto hidx = [&](int i, int j, int r) {
+            const int n = i + j + r;
+            return harm ? n * n + (r ? n + 1 : 0) + j : M.idx(i, j, r);
+        };
+        auto eidx = [&](int i, int j, int k) {
+            if (i < 0 || j < 0 || k < 0) return -1;
+            const int n = i + j + k;
+            return harm ? m2l_ebase(true, n) + (k == 0 ? 0 : k == 1 ? n + 1 : 2 * n + 1) + j
+                        : M.idx(i, j, k);
+        };
+        std::vector<int> hm(3 * H);   // exponents of each basis index
         for (int k = 0; k < K; k++) {
-            const int *a = &M.mi[3 * k];
-            const double f = fact(a[0]) * fact(a[1]) * fact(a[2]);
-            T.m2l_bscale[k] = ((a[0] + a[1] + a[2]) % 2 ? -1.0 : 1.0) / f;
-            T.m2l_lscale[k] = 1.0 / f;
-        }
-        T.m2l_erec.assign(4 * K, 0);
-        for (int k = 0; k < K; k++) {
-            int j[6];
-            for (int i = 0; i < 3; i++) {
-                j[i] = T.rec1[4 * k + i] >= 0 ? T.rec1[4 * k + i] : K;
-                j[3 + i] = T.rec2[4 * k + i] >= 0 ? T.rec2[4 * k + i] : K;
-            }
-            // byte offsets (8 j) of the entries the recurrence reads, and
-            // k! | |k| << 24 (k! <= 10! < 2^22 for the orders of the
-            // matrix-core M2L)
             const int *m = &M.mi[3 * k];
-            T.m2l_erec[4 * k] = 8 * j[0] | (8 * j[1] << 16);
-            T.m2l_erec[4 * k + 1] = 8 * j[2] | (8 * j[3] << 16);
-            T.m2l_erec[4 * k + 2] = 8 * j[4] | (8 * j[5] << 16);
-            T.m2l_erec[4 * k + 3] =
-                (int)(fact(m[0]) * fact(m[1]) * fact(m[2])) | ((m[0] + m[1] + m[2]) << 24);
+            if (harm && m[2] > 1) continue;
+            const int h = hidx(m[0], m[1], m[2]);
+            for (int q = 0; q < 3; q++) hm[3 * h + q] = m[q];
         }
-        T.m2l_tile_idx.clear();
-        if (P >= 1 && P <= M2L_MFMA_MAX_P) {
-            const int N8 = m2l_ntiles8(P);
-            T.m2l_tile_idx.assign((size_t)16 * N8, (uint16_t)(8 * K));   // byte offsets
-            int t = 0;
-            for (int ta = 0; ta < m2l_ntile1(P); ta++)
-                for (int tb = 0; tb < m2l_nrows(P, ta); tb++, t++)
-                    for (int e = 0; e < 16; e++) {
-                        const int row = e & 3, k = e >> 2, a = 4 * ta + k, b = 4 * tb + row;
-                        if (a >= K || b >= K) continue;
-                        const int *ma = &M.mi[3 * a], *mb = &M.mi[3 * b];
-                        const int s = M.idx(ma[0] + mb[0], ma[1] + mb[1], ma[2] + mb[2]);
-                        if (s >= 0) T.m2l_tile_idx[(size_t)e * N8 + t] = (uint16_t)(8 * s);
-                    }
+        // (I, J, r) collects a = (I - 2t, J - 2u, r + 2(t + u)) with (-1)^q C(q, t), q = t + u
+        T.m2l_fold_off.push_back(0);
+        for (int h = 0; h < H; h++) {
+            const int I = hm[3 * h], J = hm[3 * h + 1], r = hm[3 * h + 2];
+            for (int t = 0; 2 * t <= (harm ? I : 0); t++)
+                for (int u = 0; 2 * u <= (harm ? J : 0); u++) {
+                    const int a[3] = {I - 2 * t, J - 2 * u, r + 2 * (t + u)}, q = t + u;
+                    T.m2l_fold_idx.push_back(M.idx(a[0], a[1], a[2]));
+                    T.m2l_fold_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) *
+                                              ((I + J + r) % 2 ? -1.0 : 1.0) /
+                                              (fact(a[0]) * fact(a[1]) * fact(a[2])));
+                }
+            T.m2l_fold_off.push_back((int)T.m2l_fold_idx.size());
         }
+        // l'_(i, j, r + 2q) = (-1)^q sum_t C(q, t) l'_(i + 2t, j + 2(q - t), r)
+        T.m2l_unf_off.push_back(0);
+        for (int k = 0; k < K; k++) {
+            const int *m = &M.mi[3 * k];
+            const int q = harm ? m[2] / 2 : 0, r = m[2] - 2 * q;
+            for (int t = 0; t <= q; t++) {
+                T.m2l_unf_idx.push_back(hidx(m[0] + 2 * t, m[1] + 2 * (q - t), r));
+                T.m2l_unf_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) /
+                                         (fact(m[0]) * fact(m[1]) * fact(m[2])));
+            }
+            T.m2l_unf_off.push_back((int)T.m2l_unf_idx.size());
+        }
+        T.m2l_erec.assign(4 * NE, 0);
+        for (int n = 0; n <= P; n++)
+            for (int z = 0; z <= (harm ? std::min(n, 2) : n); z++)
+                for (int y = 0; y <= n - z; y++) {
+                    const int x = n - z - y, k = eidx(x, y, z);
+                    int j[6] = {eidx(x - 1, y, z), eidx(x, y - 1, z), eidx(x, y, z - 1),
+                                eidx(x - 2, y, z), eidx(x, y - 2, z), eidx(x, y, z - 2)};
+                    for (int &v : j)
+                        if (v < 0) v = NE;
+                    // byte offsets of the entries the recurrence reads, and
+                    // k! | |k| << 24 (k! <= 10! < 2^22)
+                    T.m2l_erec[4 * k] = 8 * j[0] | (8 * j[1] << 16);
+                    T.m2l_erec[4 * k + 1] = 8 * j[2] | (8 * j[3] << 16);
+                    T.m2l_erec[4 * k + 2] = 8 * j[4] | (8 * j[5] << 16);
+                    T.m2l_erec[4 * k + 3] = (int)(fact(x) * fact(y) * fact(z)) | (n << 24);
+                }
+        T.m2l_tile_idx.assign((size_t)16 * N8, (uint16_t)(8 * NE));
+        int t = 0;
+        for (int ta = 0; ta < m2l_ntile1(harm, P); ta++)
+            for (int tb = 0; tb < m2l_nrows(harm, P, ta); tb++, t++)
+                for (int e = 0; e < 16; e++) {
+                    const int row = e & 3, kk = e >> 2, a = 4 * ta + kk, b = 4 * tb + row;
+                    if (a >= H || b >= H) continue;
+                    const int *ma = &hm[3 * a], *mb = &hm[3 * b];
+                    const int sx = ma[0] + mb[0], sy = ma[1] + mb[1], sz = ma[2] + mb[2];
+                    if (sx + sy + sz > P) continue;
+                    T.m2l_tile_idx[(size_t)e * N8 + t] = (uint16_t)(8 * eidx(sx, sy, sz));
+                }
     }
     // L2P: idx(b + e_j) and idx(b + e_j + e_l)
     T.d1.assign(4 * K, -1);
@@ -2791,9 +2884,9 @@ void free_tree_bufs(TreeBufs &B)
     B = TreeBufs{};
 }
 
-hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P)
+hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P, bool harm)
 {
-    if (P < 1 || P > M2L_MFMA_MAX_P || S.etab_p == P) return hipSuccess;
+    if (P < 1 || P > M2L_MFMA_MAX_P || (S.etab_p == P && S.etab_harm == harm)) return hipSuccess;
     if (!S.m2l_erec) return hipErrorInvalidValue;
     if (S.etab) {
         VPMX_CHK(hipStreamSynchronize(st));
@@ -2801,11 +2894,15 @@ hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P)
         S.etab = nullptr;
         S.etab_p = -1;
     }
-    const int K = m2l_ncoef(P);
-    VPMX_CHK(hipMalloc((void **)&S.etab, (size_t)M2L_TAB_ROWS * K * sizeof(double)));
+    VPMX_CHK(hipMalloc((void **)&S.etab, (size_t)M2L_TAB_ROWS * m2l_trow(harm, P) * sizeof(double)));
     const unsigned g = gridn(M2L_TAB_ROWS, FMM_BLOCK);
-#define VPMX_ETAB(PP)                                                                  \
-    case PP: m2l_etab_kernel<PP><<<g, FMM_BLOCK, 0, st>>>(S.m2l_erec, S.etab); break;
+#define VPMX_ETAB(PP)                                                                       \
+    case PP:                                                                                \
+        if (harm)                                                                           \
+            m2l_etab_kernel<PP, true><<<g, FMM_BLOCK, 0, st>>>(S.m2l_erec, S.etab);         \
+        else                                                                                \
+            m2l_etab_kernel<PP, false><<<g, FMM_BLOCK, 0, st>>>(S.m2l_erec, S.etab);        \
+        break;
     switch (P) {
         VPMX_ETAB(1) VPMX_ETAB(2) VPMX_ETAB(3) VPMX_ETAB(4) VPMX_ETAB(5)
         VPMX_ETAB(6) VPMX_ETAB(7) VPMX_ETAB(8) VPMX_ETAB(9) VPMX_ETAB(10)
@@ -2814,6 +2911,7 @@ hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P)
 #undef VPMX_ETAB
     VPMX_CHK(hipGetLastError());
     S.etab_p = P;
+    S.etab_harm = harm;
     return hipSuccess;
 }
 
@@ -3089,9 +3187,10 @@ hipError_t launch_fmm_gather(hipStream_t st, const DeviceField &f, const int32_t
 // Grid of the persistent matrix-core M2L: resident blocks per CU (from the
 // kernel's register and LDS use) times the CUs, a multiple of 8 (one share
 // per XCD), at most one block per 8 cells.
-static int m2l_mfma_grid(const void *fn, int P, int ncell)
+static int m2l_mfma_grid(const void *fn, int P, bool harm, int ncell)
 {
-    static int cached[M2L_MFMA_MAX_P + 1] = {0};
+    static int cached_of[2][M2L_MFMA_MAX_P + 1] = {};
+    int *cached = cached_of[harm];
     if (!cached[P]) {
         int dev = 0, ncu = 0, nb = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -3124,20 +3223,27 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
         if (e != hipSuccess) return e;
     }
     if (d.ncell > 0 && P >= 1 && P <= M2L_MFMA_MAX_P) {
-        const int64_t nm = (int64_t)d.ncell * 3 * K;
         if (!d.ijk || !d.etab) return hipErrorInvalidValue;
-        m2l_prescale_kernel<<<gridn(nm, FMM_BLOCK), FMM_BLOCK, 0, st>>>(d.M, nm, K, d.m2l_bscale,
-                                                                       d.ijk, d.m2l_erec, d.ext);
-        // the zero multipole row read for absent sources (M holds ncell + 1 rows)
-        fmm_zero_kernel<<<gridn(3 * K, FMM_BLOCK), FMM_BLOCK, 0, st>>>(d.M + nm, 3 * K);
+        // the kernel's multipoles lie in L (written only by the unfolding) and its
+        // result in M (whose multipoles have no reader after the fold)
+        const bool harm = d.m2l_harm;
+        const int H = m2l_dim(harm, P), HS = m2l_hrow(harm, P);
+        const int64_t nf = ((int64_t)d.ncell + 1) * 3 * HS, nl = (int64_t)d.ncell * 3 * K;
+        (harm ? m2l_fold_kernel<true> : m2l_fold_kernel<false>)<<<gridn(nf, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
+            d.M, d.ncell, K, H, HS, d.m2l_fold_off, d.m2l_fold_idx, d.m2l_fold_coef, d.ijk, d.ext,
+            d.L);
+        const auto go = [&](auto fn) {
+            fn<<<m2l_mfma_grid((const void *)fn, P, harm, d.ncell), 64, 0, st>>>(
+                d.ijk, d.ncell, d.m2l_off, d.m2l_src, d.m2l_erec, d.m2l_tile_idx, d.etab, d.L,
+                (int64_t)d.ncell, d.M);
+        };
 #define VPMX_M2LM(PP)                                                                           \
-    case PP: {                                                                                  \
-        const int grid = m2l_mfma_grid((const void *)m2l_mfma_kernel<PP>, PP, d.ncell);          \
-        m2l_mfma_kernel<PP><<<grid, 64, 0, st>>>(d.ijk, d.ncell, d.m2l_off, d.m2l_src,           \
-                                                 d.m2l_erec, d.m2l_tile_idx, d.m2l_lscale,      \
-                                                 d.etab, d.ext, d.M, (int64_t)d.ncell, d.L);    \
-        break;                                                                                  \
-    }
+    case PP:                                                                                    \
+        if (harm)                                                                               \
+            go(m2l_mfma_kernel<PP, true>);                                                      \
+        else                                                                                    \
+            go(m2l_mfma_kernel<PP, false>);                                                     \
+        break;
         switch (P) {
             VPMX_M2LM(1) VPMX_M2LM(2) VPMX_M2LM(3) VPMX_M2LM(4) VPMX_M2LM(5)
             VPMX_M2LM(6) VPMX_M2LM(7) VPMX_M2LM(8) VPMX_M2LM(9) VPMX_M2LM(10)
@@ -3145,6 +3251,11 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
         }
 #undef VPMX_M2LM
         hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        (harm ? m2l_unfold_kernel<true> : m2l_unfold_kernel<false>)<<<gridn(nl, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
+            d.M, (int64_t)d.ncell * 3, K, H, d.m2l_unf_off, d.m2l_unf_idx, d.m2l_unf_coef, d.ijk,
+            d.ext, d.L);
+        e = hipGetLastError();
         if (e != hipSuccess) return e;
     } else if (d.ncell > 0) {
         // derivatives + multipoles of a batch, or the chunk sums at the end

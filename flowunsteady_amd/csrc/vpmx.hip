@@ -700,10 +700,15 @@ int fmm_tables_to_device(vpmx_ctx *c, FmmState &S)
     VPMX_TRY(upload_as(c, &S.m2l_chunks, T.m2l_chunk));
     VPMX_TRY(upload_as(c, &S.m2l_cfirst, T.m2l_cfirst));
     VPMX_TRY(upload_as(c, &S.m2l_tile_idx, T.m2l_tile_idx));
-    VPMX_TRY(upload_as(c, &S.m2l_bscale, T.m2l_bscale));
-    VPMX_TRY(upload_as(c, &S.m2l_lscale, T.m2l_lscale));
+    VPMX_TRY(upload_as(c, &S.m2l_fold_off, T.m2l_fold_off));
+    VPMX_TRY(upload_as(c, &S.m2l_fold_idx, T.m2l_fold_idx));
+    VPMX_TRY(upload_as(c, &S.m2l_fold_coef, T.m2l_fold_coef));
+    VPMX_TRY(upload_as(c, &S.m2l_unf_off, T.m2l_unf_off));
+    VPMX_TRY(upload_as(c, &S.m2l_unf_idx, T.m2l_unf_idx));
+    VPMX_TRY(upload_as(c, &S.m2l_unf_coef, T.m2l_unf_coef));
     VPMX_TRY(upload_as(c, &S.m2l_erec, T.m2l_erec));
     S.dev_tab_p = T.P;
+    S.dev_tab_harm = T.m2l_harm;
     return VPMX_OK;
 }
 
@@ -712,8 +717,9 @@ void free_fmm(FmmState *S)
     if (!S) return;
     void *ptrs[] = {S->mi, S->m2m_off, S->l2l_off, S->m2l_toff, S->rec1, S->rec2, S->d1, S->d2a,
                     S->d2b, S->m2m_idx, S->l2l_idx, S->m2l_tidx, S->m2m_coef, S->l2l_coef,
-                    S->m2l_tcoef, S->m2l_chunks, S->m2l_cfirst, S->m2l_tile_idx, S->m2l_bscale,
-                    S->m2l_lscale, S->m2l_erec, S->chunk_buf, S->chunks, S->part, S->chunk_tmp,
+                    S->m2l_tcoef, S->m2l_chunks, S->m2l_cfirst, S->m2l_tile_idx, S->m2l_fold_off,
+                    S->m2l_fold_idx, S->m2l_fold_coef, S->m2l_unf_off, S->m2l_unf_idx,
+                    S->m2l_unf_coef, S->m2l_erec, S->chunk_buf, S->chunks, S->part, S->chunk_tmp,
                     S->cells, S->ijk, S->etab, S->leaves, S->parents, S->kids, S->parent,
                     S->m2l_off, S->p2p_off, S->m2l_src, S->p2p_src, S->M, S->L, S->kin, S->kout,
                     S->ssig, S->sort_tmp};
@@ -745,8 +751,8 @@ int fmm_reserve_n(vpmx_ctx *c, FmmState &S, int64_t n)
 
 // One FMM UJ evaluation; lists_only: the tree, the traversal and the
 // near-field work items only (for the viscous sums), no evaluation; DJ: also
-// the core-size derivative of J (FP64).
-int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = false,
+// the core-size derivative of J (FP64).  harm: the M2L's basis (fmm.h).
+int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool harm, bool lists_only = false,
             double *DJ = nullptr)
 {
     MarkScope ms(c, lists_only ? "vpmx fmm lists" : "vpmx fmm uj");
@@ -798,14 +804,16 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = f
         VPMX_HIP(c, fmm_build_tree_device(st, S, n, P->ncrit, pl, &nc));
     }
     // device: tables (once per p), expansions
-    if (S.dev_tab_p != P->p) {
-        fmm_build_tables(S.tab, P->p);
+    if (S.dev_tab_p != P->p || S.dev_tab_harm != harm) {
+        fmm_build_tables(S.tab, P->p, harm);
         VPMX_TRY(fmm_tables_to_device(c, S));
     }
-    VPMX_HIP(c, fmm_m2l_table(st, S, P->p));
+    VPMX_HIP(c, fmm_m2l_table(st, S, P->p, harm));
     const int K = S.tab.K;
-    if ((nc + 1) * 3 * K > S.cap_coef) {   // + the zero row of the matrix-core M2L
-        const int64_t cap = std::max<int64_t>((nc + 1) * 3 * K, S.cap_coef + S.cap_coef / 2);
+    // L also holds the multipoles the matrix-core M2L reads (and a zero row)
+    const int64_t ncoef = (nc + 1) * 3 * std::max(K, m2l_hrow(harm, P->p));
+    if (ncoef > S.cap_coef) {
+        const int64_t cap = std::max<int64_t>(ncoef, S.cap_coef + S.cap_coef / 2);
         VPMX_TRY(dalloc(c, &S.M, cap));
         VPMX_TRY(dalloc(c, &S.L, cap));
         S.cap_coef = cap;
@@ -872,12 +880,17 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool lists_only = f
     d.m2l_nchunk = S.tab.m2l_nchunk;
     d.m2l_rounds = S.tab.m2l_rounds;
     d.m2l_tile_idx = S.m2l_tile_idx;
-    d.m2l_bscale = S.m2l_bscale;
-    d.m2l_lscale = S.m2l_lscale;
+    d.m2l_fold_off = S.m2l_fold_off;
+    d.m2l_fold_idx = S.m2l_fold_idx;
+    d.m2l_fold_coef = S.m2l_fold_coef;
+    d.m2l_unf_off = S.m2l_unf_off;
+    d.m2l_unf_idx = S.m2l_unf_idx;
+    d.m2l_unf_coef = S.m2l_unf_coef;
     d.m2l_erec = S.m2l_erec;
     d.ijk = S.ijk;
     d.etab = S.etab;
     d.ext = pl.ext;
+    d.m2l_harm = harm;
     d.chunks = S.chunks;
     d.chunk_off = S.chunk_off;
     d.part_base = S.part_base;
@@ -915,15 +928,17 @@ int enqueue_sort(vpmx_ctx *c)
 }
 
 // One UJ evaluation.  `sort` = false reuses the Morton order of the last sort
-// (a time step sorts once and keeps that order through its substeps).  dsig: the
-// evaluation of a dynamic SFS stage (FP64 FMM: takes D[J] along).
-int enqueue_uj(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool sort = true, bool dsig = false)
+// (a time step sorts once and keeps that order through its substeps).  sfs: a
+// stretching pass will read J (in this evaluation's step); dsig: the evaluation
+// of a dynamic SFS stage (FP64 FMM: takes D[J] along).
+int enqueue_uj(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool sort, bool sfs,
+               bool dsig = false)
 {
     const DeviceField &f = c->f;
     BatchState &B = c->b;
     if (P->fmm) {
         if (B.nfields) return fail(c, VPMX_EUNSUPPORTED, "the FMM does not run on batched fields");
-        return run_fmm(c, P, reset, false,
+        return run_fmm(c, P, reset, !(sfs && P->precision == VPMX_MIXED), false,
                        dsig && P->precision == VPMX_FP64 ? c->f.DJ() : nullptr);
     }
     MarkScope ms(c, "vpmx direct uj");
@@ -1010,7 +1025,7 @@ int enqueue_step(vpmx_ctx *c, const vpmx_uj_params *U, const vpmx_step_params *S
     const int32_t *fid = c->b.nfields ? c->b.fid : nullptr;
     if (rk3) VPMX_HIP(c, launch_fill(c->stream, f.M, 7 * f.cap, 0.0));
     for (int s = 0; s < nst; ++s) {
-        VPMX_TRY(enqueue_uj(c, U, 1, false, S->sfs == VPMX_SFS_DYNAMIC));
+        VPMX_TRY(enqueue_uj(c, U, 1, false, sfs != 0, S->sfs == VPMX_SFS_DYNAMIC));
         if (S->sfs == VPMX_SFS_DYNAMIC) {
             VPMX_TRY(enqueue_dsig(c, U));
             VPMX_TRY(enqueue_estr(c, U, true));
@@ -1033,7 +1048,7 @@ int enqueue_step(vpmx_ctx *c, const vpmx_uj_params *U, const vpmx_step_params *S
                                       rk3 ? RK3_B[s] : 1.0, dt, S->viscous, S->nu));
     }
     if (relax && S->relax_kind != VPMX_RELAX_NONE) {
-        if (rk3) VPMX_TRY(enqueue_uj(c, U, 1, false));
+        if (rk3) VPMX_TRY(enqueue_uj(c, U, 1, false, sfs != 0));
         VPMX_HIP(c, launch_relax(c->stream, f, S->relax_kind, S->rlxf));
     }
     return VPMX_OK;
@@ -1069,7 +1084,7 @@ int core_spreading_reset(vpmx_ctx *c, const vpmx_uj_params *U, const vpmx_step_p
     // With the FMM every vorticity sum runs over the near lists of one tree
     // built here at the current positions and cores (zeta_fmm); directly
     // otherwise (zeta_direct).
-    if (U->fmm) VPMX_TRY(run_fmm(c, U, 1, true));
+    if (U->fmm) VPMX_TRY(run_fmm(c, U, 1, true, true));
     auto zeta = [&](const double *G, int64_t gld, double s0, double *w) -> hipError_t {
         if (U->fmm)
             return launch_fmm_zeta(st, *c->fmm, kernel, f, s, G, gld, s0, mask, s.vrec, w, ld);
@@ -1329,7 +1344,7 @@ int vpmx_uj(vpmx_ctx *c, double *particles, int64_t np, const vpmx_layout *L,
     VPMX_TRY(check_uj_params(c, P));
     if (P->sfs && L->SFS < 0) return fail(c, VPMX_EINVAL, "sfs requested but layout.SFS = -1");
     VPMX_TRY(upload(c, particles, np, L, !P->reset));
-    VPMX_TRY(enqueue_uj(c, P, P->reset));
+    VPMX_TRY(enqueue_uj(c, P, P->reset, true, P->sfs != 0));
     if (P->sfs) VPMX_TRY(enqueue_estr(c, P));
     VPMX_TRY(sync(c));
     return download(c, particles, L, DL_UJ | (P->sfs ? DL_SFS : 0));
@@ -1422,7 +1437,7 @@ int vpmx_uj_resident(vpmx_ctx *c, const vpmx_uj_params *P)
     if (c->b.nfields && P->sfs)
         return fail(c, VPMX_EUNSUPPORTED, "the SFS model does not run on batched fields");
     VPMX_TRY(prepare_batch(c, P->kernel));
-    VPMX_TRY(enqueue_uj(c, P, P->reset));
+    VPMX_TRY(enqueue_uj(c, P, P->reset, true, P->sfs != 0));
     if (P->sfs) VPMX_TRY(enqueue_estr(c, P));
     return sync(c);
 }
@@ -1704,7 +1719,7 @@ int vpmx_batch_uj(vpmx_ctx *c, int32_t nfields, double *const *particles, const 
     if (P->sfs && L->SFS < 0) return fail(c, VPMX_EINVAL, "sfs requested but layout.SFS = -1");
     VPMX_TRY(upload_fields(c, nfields, (const double *const *)particles, np, L, !P->reset));
     VPMX_TRY(prepare_batch(c, P->kernel));
-    VPMX_TRY(enqueue_uj(c, P, P->reset));
+    VPMX_TRY(enqueue_uj(c, P, P->reset, true, P->sfs != 0));
     if (P->sfs) VPMX_TRY(enqueue_estr(c, P));
     VPMX_TRY(sync(c));
     return download_fields(c, nfields, particles, L, DL_UJ | (P->sfs ? DL_SFS : 0));
