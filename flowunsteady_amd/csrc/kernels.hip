@@ -164,15 +164,18 @@ static Split split_f64_for(int64_t nt, int64_t n)
     return {(int)((n + seglen - 1) / seglen), seglen};
 }
 
-// How a launch over nb target blocks and n sources is split: when the target
-// blocks alone cannot fill the device, the source range is cut into segments
-// (multiples of UJ_BLOCK, at least four tiles each) so that about 1024
-// workgroups run; their partial sums go through `part` (SPLIT_PART doubles).
+// Split of a mixed launch over nb target blocks of 256 and n sources: the
+// source range is cut into segments (whole tiles of 256) so that about 2048
+// workgroups run, twice what the chip holds at a time, the second half evening
+// out near and far blocks.  With 1024 workgroups, and no split from 512 target
+// blocks on, the Winckelmans cube of 131,071 ran as 512 workgroups, two waves
+// per SIMD: 22.7 -> 18.0 ms per UJ.  From 2048 blocks on (n = 524,288) the
+// segments' sums (nseg nt <= 2048 256 slots of 14 doubles, written and read
+// again) would buy nothing.  Partial sums go through `part`.
 static Split split_for(int64_t nb, int64_t n)
 {
-    if (nb >= 512 || n <= 4 * UJ_BLOCK) return {1, n};
-    int64_t nseg = std::min<int64_t>((1024 + nb - 1) / nb, (n + 4 * UJ_BLOCK - 1) / (4 * UJ_BLOCK));
-    nseg = std::max<int64_t>(nseg, 1);
+    const int64_t nseg = std::min<int64_t>(2048 / std::max<int64_t>(nb, 1), (n + UJ_BLOCK - 1) / UJ_BLOCK);
+    if (nseg <= 1) return {1, n};
     const int64_t seglen = ((n + nseg - 1) / nseg + UJ_BLOCK - 1) / UJ_BLOCK * UJ_BLOCK;
     return {(int)((n + seglen - 1) / seglen), seglen};
 }
@@ -485,20 +488,28 @@ __global__ __launch_bounds__(UJ_BLOCK) void uj_mixed_split_kernel(const double4 
         for (int k = 0; k < 14; ++k) part[((int64_t)g * 14 + k) * pld + s] = d[k];
 }
 
-__global__ __launch_bounds__(EW_BLOCK) void uj_mixed_split_reduce_kernel(
+// Segments added in segment order.  A workgroup's 14 waves take one component
+// each of 64 slots (a chain of nseg loads per thread), then the first wave
+// assembles U and J.
+constexpr int RED_SLOTS = 64;
+__global__ __launch_bounds__(14 * RED_SLOTS) void uj_mixed_split_reduce_kernel(
     const double *__restrict__ part, int64_t pld, int nseg, int64_t nt,
     const int32_t *__restrict__ perm, int64_t ldo, double *__restrict__ U, double *__restrict__ J,
     int reset)
 {
-    const int64_t s = (int64_t)blockIdx.x * EW_BLOCK + threadIdx.x;
-    if (s >= nt) return;
-    double d[14];
-    for (int k = 0; k < 14; ++k) {
-        double v = 0.0;
+    __shared__ double sum[14][RED_SLOTS];
+    const int k = threadIdx.x / RED_SLOTS, i = threadIdx.x % RED_SLOTS;
+    const int64_t s = (int64_t)blockIdx.x * RED_SLOTS + i;
+    double v = 0.0;
+    if (s < nt)
         for (int g = 0; g < nseg; ++g) v += part[((int64_t)g * 14 + k) * pld + s];
-        d[k] = v;
+    sum[k][i] = v;
+    __syncthreads();
+    if (k == 0 && s < nt) {
+        double d[14];
+        for (int q = 0; q < 14; ++q) d[q] = sum[q][i];
+        uj_mixed_store(d, perm[s], ldo, U, J, reset);
     }
-    uj_mixed_store(d, perm[s], ldo, U, J, reset);
 }
 
 // Target-subset variant (probes): targets need not be spatially compact, so
@@ -622,7 +633,7 @@ static hipError_t uj_mixed_go(hipStream_t st, bool two, const double4 *tgt, int6
                                                             sp.nseg, tb, part, nt);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    uj_mixed_split_reduce_kernel<<<grid_for(nt, EW_BLOCK), EW_BLOCK, 0, st>>>(
+    uj_mixed_split_reduce_kernel<<<grid_for(nt, RED_SLOTS), 14 * RED_SLOTS, 0, st>>>(
         part, nt, sp.nseg, nt, tperm, ldo, U, J, two ? 1 : reset);
     return hipGetLastError();
 }

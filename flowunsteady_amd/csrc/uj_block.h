@@ -198,6 +198,13 @@ __device__ __forceinline__ void uj_f64_store(const double v[12], int64_t i, int6
 // first target in FP64 and rounded to FP32; FP32 partials are folded into
 // FP64 every MIXED_FOLD pairs (once per tile for far tiles).  d = (U0..2, W0..2, J0..7) before the -1/(4 pi) factor.
 //
+// Bound by FP32 issue: a far pair is 34 instructions, about 74 cycles of its SIMD
+// at the rate of two per four cycles, and takes 105 with four waves per SIMD
+// (cube of 1,048,576: 749 ms per UJ).  Two targets per thread halve the LDS reads
+// but leave two or three waves: 925-1036 ms; five waves spill: 843 ms.  The
+// unroll counts keep the near loop at 112 VGPRs, four waves (4 and 4 in place of
+// 8 and 2: 753 ms; a batch of 24 fields 45.0 against 43.5).
+//
 // With tile bounds `tb` (per BLK-slot tile counted from slot `torg`: (centre,
 // radius), (largest sigma, -, -, -); the block's own targets are tile
 // (t0 - torg)/BLK), a tile whose every pair is in the far field -- gap >=
@@ -269,7 +276,7 @@ __device__ __forceinline__ void uj_mixed_sums(const double4 *__restrict__ tgt, i
             if (!far) {
                 if (cnt == BLK) {
                     for (int jb = 0; jb < BLK; jb += MIXED_FOLD) {
-#pragma unroll 4
+#pragma unroll 2
                         for (int jj = jb; jj < jb + MIXED_FOLD; ++jj)
                             mixed_pair_dsig_hl<K>(tpos[jj], tlo[jj], tgam[jj], xi, yi, zi, xl,
                                                   yl, zl, acc);
@@ -286,12 +293,12 @@ __device__ __forceinline__ void uj_mixed_sums(const double4 *__restrict__ tgt, i
         } else if (far) {
             // far pairs are at least 7 core sizes (or a gap) away: their terms
             // stay small and one partial per tile suffices
-#pragma unroll 4
+#pragma unroll 8
             for (int jj = 0; jj < BLK; ++jj)
                 mixed_pair_far<K>(tpos[jj], tgam[jj], xi, yi, zi, acc);
         } else if (cnt == BLK) {
             for (int jb = 0; jb < BLK; jb += MIXED_FOLD) {
-#pragma unroll 4
+#pragma unroll 2
                 for (int jj = jb; jj < jb + MIXED_FOLD; ++jj)
                     mixed_pair_hl<K>(tpos[jj], &tlo[jj], tgam[jj], xi, yi, zi, xl, yl, zl, acc);
                 mixed_fold(d, acc);

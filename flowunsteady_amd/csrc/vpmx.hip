@@ -224,7 +224,7 @@ int ensure_capacity(vpmx_ctx *c, int64_t np)
     VPMX_TRY(dalloc(c, &s.sgam, cap));
     VPMX_TRY(dalloc(c, &s.tbnd, 2 * ((cap + 63) / 64)));
     if (!s.kpart) {
-        s.kcap = 15 * 256 * 1536;   // more than a split launch needs (see split_for, split_f64_for)
+        s.kcap = 14 * 256 * 2048;   // the most a split launch needs (see split_for, split_f64_for)
         VPMX_TRY(dalloc(c, &s.kpart, s.kcap));
     }
     VPMX_TRY(dalloc(c, &s.kin, cap));
