@@ -161,8 +161,7 @@ constexpr double ROUND_MAGIC = 6755399441055744.0;       // 1.5 * 2^52
 constexpr double X_SMALL = 2.25;                         // rho^2 below which the series runs
 constexpr double X_FAR = 90.25;    // rho = 9.5: 1 - g < 3e-19 and rho g' < 2e-17, the pair is singular
 constexpr double RHO_FAR = 9.5;
-constexpr double X_CORE = 120.0;   // e^{-60}: zeta and the core-size derivatives vanish
-constexpr double RHO_CORE = 10.96;
+constexpr double X_CORE = 1500.0;  // e^{-x/2} is zero: so are zeta and the core-size derivatives
 
 __device__ __forceinline__ double rsq_f64(double a)
 {

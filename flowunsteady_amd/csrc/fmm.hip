@@ -34,6 +34,7 @@
 #include <rocprim/device/device_scan.hpp>
 
 #include "device_math.h"
+#include "estr.h"
 #include "fmm.h"
 #include "internal.h"
 #include "uj_block.h"
@@ -1076,7 +1077,7 @@ __device__ __forceinline__ void p2p_f64_pair(const double4 a, const double4 b, d
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     const double x = r2 * (b.w * b.w);
     bool far = false;
-    if constexpr (KK == GAUSSIANERF || KK == GAUSSIAN) far = __all(x >= X_FAR);
+    if constexpr (KK == GAUSSIANERF || KK == GAUSSIAN) far = __all(x >= (DYN ? X_CORE : X_FAR));
     double A, B, AD = 0.0, BD = 0.0;
     if (far) {
         const double rinv = rsq_f64(r2), ri2 = rinv * rinv;
@@ -1725,63 +1726,12 @@ __device__ __forceinline__ void estr_finish(const double *d, int64_t i, int64_t 
     }
 }
 
-// Sorted Estr source records (x, y, z, 1/sigma) (Gamma, 0) (J0..3) (J4..7)
-// (J8, 0, 0, 0); with DYN the last is (J8, DJ0..2) followed by (DJ3..6)
-// (DJ7, DJ8, 0, 0): 7 per particle.
-template <bool DYN>
-__global__ __launch_bounds__(FMM_BLOCK) void fmm_estr_gather_kernel(
-    const double *__restrict__ X, const double *__restrict__ G, const double *__restrict__ sg,
-    const double *__restrict__ Jm, const double *__restrict__ DJ,
-    const int32_t *__restrict__ perm, int64_t n, int64_t cap, double4 *__restrict__ out)
-{
-    constexpr int NR = DYN ? 7 : 5;
-    const int64_t s = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (s >= n) return;
-    const int64_t i = perm[s];
-    double4 *o = out + NR * s;
-    o[0] = make_double4(X[i], X[cap + i], X[2 * cap + i], 1.0 / sg[i]);
-    o[1] = make_double4(G[i], G[cap + i], G[2 * cap + i], 0.0);
-    o[2] = make_double4(Jm[i], Jm[cap + i], Jm[2 * cap + i], Jm[3 * cap + i]);
-    o[3] = make_double4(Jm[4 * cap + i], Jm[5 * cap + i], Jm[6 * cap + i], Jm[7 * cap + i]);
-    if constexpr (DYN) {
-        o[4] = make_double4(Jm[8 * cap + i], DJ[i], DJ[cap + i], DJ[2 * cap + i]);
-        o[5] = make_double4(DJ[3 * cap + i], DJ[4 * cap + i], DJ[5 * cap + i], DJ[6 * cap + i]);
-        o[6] = make_double4(DJ[7 * cap + i], DJ[8 * cap + i], 0.0, 0.0);
-    } else {
-        o[4] = make_double4(Jm[8 * cap + i], 0.0, 0.0, 0.0);
-    }
-}
-
-// The nine J (and with DYN DJ) entries of a record.
-template <bool DYN>
-__device__ __forceinline__ void estr_rec_j(const double4 *r, double *Jv, double *DJv)
-{
-    const double4 q2 = r[2], q3 = r[3], q4 = r[4];
-    Jv[0] = q2.x; Jv[1] = q2.y; Jv[2] = q2.z; Jv[3] = q2.w;
-    Jv[4] = q3.x; Jv[5] = q3.y; Jv[6] = q3.z; Jv[7] = q3.w; Jv[8] = q4.x;
-    if constexpr (DYN) {
-        const double4 q5 = r[5], q6 = r[6];
-        DJv[0] = q4.y; DJv[1] = q4.z; DJv[2] = q4.w;
-        DJv[3] = q5.x; DJv[4] = q5.y; DJv[5] = q5.z; DJv[6] = q5.w;
-        DJv[7] = q6.x; DJv[8] = q6.y;
-    }
-}
-
-template <bool TRANSPOSED, typename T>
-__device__ __forceinline__ void stretch_of(const T *dJ, T gx, T gy, T gz, T &S0, T &S1, T &S2)
-{
-    if constexpr (TRANSPOSED) {   // S_k = sum_l dJ[l,k] G_l
-        S0 = dJ[0] * gx + dJ[1] * gy + dJ[2] * gz;
-        S1 = dJ[3] * gx + dJ[4] * gy + dJ[5] * gz;
-        S2 = dJ[6] * gx + dJ[7] * gy + dJ[8] * gz;
-    } else {                      // S_k = sum_l dJ[k,l] G_l
-        S0 = dJ[0] * gx + dJ[3] * gy + dJ[6] * gz;
-        S1 = dJ[1] * gx + dJ[4] * gy + dJ[7] * gz;
-        S2 = dJ[2] * gx + dJ[5] * gy + dJ[8] * gz;
-    }
-}
-
-// Estr over the near-field lists, FP64; DYN adds D[E] (zeta_zD_f64).
+// Estr over the near-field lists, FP64; DYN adds D[E] (the pair sums of
+// estr.h).  One wave per work item, the source leaves streamed through LDS and
+// the targets of small leaves replicated as in p2p_f64_kernel (with D[E] at most
+// twice, as there).  Bound by FP64 issue, 31 instructions per pair, 42 with D[E].
+// 100,003 particles with D[E], ncrit = 50: 8.6 -> 3.2 ms (one lane per target,
+// leaf by leaf, before).
 template <int KK, bool TRANSPOSED, bool DYN>
 __global__ __launch_bounds__(P2P_BLOCK) void fmm_estr_kernel(const P2PChunk *__restrict__ chunks,
                                                              const FmmCellDev *__restrict__ cells,
@@ -1793,66 +1743,59 @@ __global__ __launch_bounds__(P2P_BLOCK) void fmm_estr_kernel(const P2PChunk *__r
                                                              double *__restrict__ part,
                                                              int64_t pstride)
 {
-    constexpr int NR = DYN ? 7 : 5;
-    constexpr int NV = DYN ? 6 : 3;
-    __shared__ double4 tile[NR * P2P_BLOCK];
+    constexpr int NR = ESTR_NR<DYN>, NL = ESTR_NL<DYN>, NV = DYN ? 6 : 3;
+    __shared__ double2 tile[NL * P2P_BLOCK];
+    __shared__ int32_t lbeg[P2P_SLOTS], lpre[P2P_SLOTS + 1];
+    const int lane = threadIdx.x;
     const P2PChunk ch = chunks[blockIdx.x];
-    const int c = ch.c;
-    const FmmCellDev A = cells[c];
+    const FmmCellDev A = cells[ch.c];
     for (int tb = A.begin; tb < A.end; tb += P2P_BLOCK) {
-        const int it = tb + threadIdx.x;
-        const bool active = it < A.end;
-        double xi = 0, yi = 0, zi = 0, Ji[9], DJi[9];
-        for (int k = 0; k < 9; ++k) Ji[k] = DJi[k] = 0.0;
-        if (active) {
-            const double4 p = rec[NR * it];
-            xi = p.x; yi = p.y; zi = p.z;
-            estr_rec_j<DYN>(rec + NR * it, Ji, DJi);
-        }
-        double e0 = 0, e1 = 0, e2 = 0, f0 = 0, f1 = 0, f2 = 0;
-        for (int64_t e = ch.e0; e < ch.e1; e++) {
-            const FmmCellDev B = cells[src[e]];
-            for (int sb = B.begin; sb < B.end; sb += P2P_BLOCK) {
+        const int nt = min(P2P_BLOCK, A.end - tb);
+        const int R = min(P2P_BLOCK / nt, DYN ? 2 : 16);
+        const int sl0 = lane / nt;
+        const int t = lane - sl0 * nt;             // target of this lane
+        const int sl = sl0 < R ? sl0 : 0;          // its slice (lanes past R nt repeat slice 0)
+        const double4 *ri = rec + NR * (tb + t);
+        const double xi = ri[0].x, yi = ri[0].y, zi = ri[0].z;
+        double Jr[9], DJr[9];
+        estr_rec_j<DYN>(rec + NR * tb, Jr, DJr);
+        EstrAcc acc;
+        for (int64_t eb = ch.e0; eb < ch.e1; eb += P2P_SLOTS) {
+            const int nl = (int)min<int64_t>(P2P_SLOTS, ch.e1 - eb);
+            __syncthreads();
+            const int total = stream_setup(cells, src, eb, nl, lane, lbeg, lpre);
+            // stream position of the lane's own particle, where the leaf itself is in the slot
+            int self = -1;
+            const unsigned long long own = __ballot(lane < nl && lbeg[lane] == A.begin);
+            if (own) self = lpre[__ffsll(own) - 1] + (tb - A.begin) + t;
+            for (int base = 0; base < total; base += P2P_BLOCK) {
                 __syncthreads();
-                const int js = sb + threadIdx.x;
-                if (js < B.end)
-                    for (int k = 0; k < NR; ++k) tile[NR * threadIdx.x + k] = rec[NR * js + k];
+                if (base + lane < total)
+                    estr_stage<KK, TRANSPOSED, DYN>(
+                        rec + NR * stream_particle(lbeg, lpre, nl, base + lane), Jr, DJr,
+                        tile + NL * lane);
                 __syncthreads();
-                const int cnt = min(P2P_BLOCK, B.end - sb);
-                for (int jj = 0; jj < cnt; ++jj) {
-                    const double4 a = tile[NR * jj], gm = tile[NR * jj + 1];
-                    double Jj[9], DJj[9];
-                    estr_rec_j<DYN>(tile + NR * jj, Jj, DJj);
-                    const double d1 = xi - a.x, d2 = yi - a.y, d3 = zi - a.z;
-                    const double r = sqrt(d1 * d1 + d2 * d2 + d3 * d3);
-                    const double is3 = a.w * a.w * a.w;
-                    double dJ[9], S0, S1, S2;
-                    for (int k = 0; k < 9; ++k) dJ[k] = Ji[k] - Jj[k];
-                    stretch_of<TRANSPOSED>(dJ, gm.x, gm.y, gm.z, S0, S1, S2);
-                    if constexpr (DYN) {
-                        double z, zD;
-                        zeta_zD_f64<KK>(r * a.w, z, zD);
-                        const double zs = z * is3, zDs = zD * is3;
-                        double T0, T1, T2;
-                        for (int k = 0; k < 9; ++k) dJ[k] = DJi[k] - DJj[k];
-                        stretch_of<TRANSPOSED>(dJ, gm.x, gm.y, gm.z, T0, T1, T2);
-                        e0 += zs * S0; e1 += zs * S1; e2 += zs * S2;
-                        f0 += zDs * S0 + zs * T0;
-                        f1 += zDs * S1 + zs * T1;
-                        f2 += zDs * S2 + zs * T2;
-                    } else {
-                        const double zs = zeta_f64<KK>(r * a.w) * is3;
-                        e0 += zs * S0; e1 += zs * S1; e2 += zs * S2;
-                    }
-                }
+                const int cnt = min(P2P_BLOCK, total - base);
+                for (int j = sl; j < cnt; j += R)
+                    estr_pair<KK, DYN>(tile + NL * j, xi, yi, zi, base + j == self, acc);
             }
         }
-        if (active) {
-            const double d[6] = {e0, e1, e2, f0, f1, f2};
+        double v[NV];
+        estr_values<TRANSPOSED, DYN>(acc, ri, Jr, DJr, v);
+        if (R > 1) {   // the slices of each target added in slice order
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                double w = v[k];
+                for (int s = 1; s < R; ++s) w += __shfl(v[k], t + s * nt);
+                v[k] = w;
+            }
+        }
+        if (lane < nt) {
             if (ch.part < 0)
-                estr_finish<NV>(d, perm[it], cap, E, DE);
+                estr_finish<NV>(v, perm[tb + lane], cap, E, DE);
             else
-                for (int k = 0; k < NV; ++k) part[k * pstride + ch.part + (it - A.begin)] = d[k];
+                for (int k = 0; k < NV; ++k)
+                    part[k * pstride + ch.part + (tb + lane - A.begin)] = v[k];
         }
     }
 }
@@ -2115,13 +2058,7 @@ hipError_t launch_fmm_estr(hipStream_t st, const FmmState &S, int kernel, int tr
 {
     if (f.np == 0) return hipSuccess;
     const bool dyn = DJ != nullptr;
-    if (dyn)
-        fmm_estr_gather_kernel<true><<<gridn(f.np, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            f.X, f.G, f.sigma, f.J, DJ, s.perm, f.np, f.cap, s.srcE);
-    else
-        fmm_estr_gather_kernel<false><<<gridn(f.np, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            f.X, f.G, f.sigma, f.J, DJ, s.perm, f.np, f.cap, s.srcE);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_pack_estr(st, f, DJ, s);
     if (e != hipSuccess) return e;
     const int64_t nleaf = (int64_t)S.plan.nleaves;
     if (nleaf == 0 || S.nchunk == 0) return hipSuccess;

@@ -180,6 +180,8 @@ hipError_t launch_uj_mixed_targets(hipStream_t st, int kernel, const DeviceField
                                    const int32_t *tperm, int64_t ldo, double *U, double *J,
                                    int reset);
 // Estr into f.E; with DJ (9 x cap) also its core-size derivative into DE.
+// Sorted FP64 Estr records of the field into s.srcE (DJ: with the core-size derivatives).
+hipError_t launch_pack_estr(hipStream_t st, const DeviceField &f, const double *DJ, Scratch &s);
 hipError_t launch_estr_f64(hipStream_t st, int kernel, int transposed, const DeviceField &f,
                            Scratch &s, const double *DJ = nullptr, double *DE = nullptr);
 // Core-size derivatives D[U] (3 x cap), D[J] (9 x cap) of every particle from

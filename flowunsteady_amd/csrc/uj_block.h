@@ -46,8 +46,8 @@ __device__ __forceinline__ void f64_pair_far(const double4 a, const double4 b, d
 // Any pair: the far form while every lane of the wave has rho^2 >= 90.25,
 // else the full evaluation; coincident pairs skipped
 // (src/FLOWUnsteady_processing_force.jl:895).  b.z holds pair_const_f64 here.
-// DS: the core-size derivatives D[U], D[J] in the same sums, which vanish
-// beyond rho^2 = 120 for the gaussian kernels.
+// DS: the core-size derivatives D[U], D[J] in the same sums, zero beyond
+// rho^2 = X_CORE for the gaussian kernels.
 template <int K, bool DS>
 __device__ __forceinline__ void f64_pair(const double4 a, const double4 b, double xi, double yi,
                                          double zi, double d[15])
