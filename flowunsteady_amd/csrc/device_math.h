@@ -94,27 +94,6 @@ __device__ __forceinline__ double eta_f64(double rho)
 // form A_D = h/r^3 = -4 pi zeta/sigma^3 and B_D = -4 pi zeta'/(rho sigma^5),
 // both finite at r = 0 and negligible beyond the core (no far field).
 
-// zeta(rho) and zD(rho) together (one exp).
-template <int K>
-__device__ __forceinline__ void zeta_zD_f64(double rho, double &z, double &zD)
-{
-    if constexpr (K == GAUSSIANERF) {
-        z = 0.06349363593424097 * exp(-0.5 * rho * rho);
-        zD = (rho * rho - 3.0) * z;
-    } else if constexpr (K == GAUSSIAN) {
-        const double r3 = rho * rho * rho;
-        z = 0.238732414637843 * exp(-r3);
-        zD = 3.0 * (r3 - 1.0) * z;
-    } else if constexpr (K == WINCKELMANS) {
-        const double q = rho * rho + 1.0;
-        z = 0.5968310365946075 / (q * q * q * sqrt(q));
-        zD = (4.0 - 7.0 / q) * z;
-    } else {
-        z = 0.0;
-        zD = 0.0;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // FP64 pair math of the all-pairs and near-field sums.
 //

@@ -55,7 +55,7 @@ __device__ __forceinline__ void stretch_of(const double J[9], const double g[3],
             S[k] = fma(J[k], g[0], fma(J[k + 3], g[1], J[k + 6] * g[2]));
 }
 
-// zeta and zD (zeta_zD_f64) over zeta's constant, at x = rho^2.
+// zeta and zD = -(3 zeta + rho zeta') over zeta's constant, at x = rho^2.
 template <int K>
 constexpr double ESTR_W = K == GAUSSIANERF ? 0.06349363593424097     // (2 pi)^-3/2
                           : K == GAUSSIAN  ? 0.238732414637843      // 3/(4 pi)

@@ -150,6 +150,22 @@ namespace vpmx {
 
 // Launchers (kernels.hip).  All enqueue on `st` and return hipSuccess or the
 // launch error.
+// Rows of the field and their places in the pinned staging (row k at h + k np).
+struct FieldRows {
+    int n = 0;
+    int row[25];
+    double *dev[25];
+    void add(int k, double *p)
+    {
+        row[n] = k;
+        dev[n++] = p;
+    }
+};
+// Staging to field, with the np flags at h + flags (doubles), and back.
+hipError_t launch_rows_in(hipStream_t st, const FieldRows &R, double *h, int64_t flags,
+                          uint8_t *flag, int64_t np);
+hipError_t launch_rows_out(hipStream_t st, const FieldRows &R, double *h, int64_t np);
+
 hipError_t launch_pack_f64(hipStream_t st, const DeviceField &f, Scratch &s);
 hipError_t launch_uj_f64(hipStream_t st, int kernel, const DeviceField &f, const Scratch &s,
                          int reset);

@@ -9,10 +9,12 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include <rocprofiler-sdk-roctx/roctx.h>
@@ -496,6 +498,41 @@ std::string where(int nf, int k, int64_t p)
     return s;
 }
 
+// fn(begin, end), which throws nothing, over [0, n): one host thread per HOST_GRAIN
+// particles, at most 16; what threads that could not be had would have taken
+// runs on the caller.  A particle is 344 bytes of the caller's matrix, 11 to 37 of
+// its 43 values touched: one thread moved 1,000,003 in about 15 ms each way (UJ
+// 76 -> 49 ms), 131,072 in 2 ms (4,099 probes 5.6 -> 2.7 ms).  Below HOST_GRAIN a
+// thread costs more to start (about 15 us) than its share saves.
+constexpr int64_t HOST_GRAIN = 16384;
+template <class F>
+void host_for(int64_t n, F fn)
+{
+    const int64_t nt = std::min<int64_t>({n / HOST_GRAIN, 16, (int64_t)std::thread::hardware_concurrency()});
+    if (nt <= 1) return fn((int64_t)0, n);
+    const int64_t chunk = (n + nt - 1) / nt;
+    std::vector<std::thread> th;
+    int64_t next = chunk;   // first particle no thread has taken; [0, chunk) is the caller's
+    try {
+        th.reserve(nt - 1);
+        for (; next < n; next += chunk) th.emplace_back(fn, next, std::min(n, next + chunk));
+    } catch (...) {
+    }
+    fn((int64_t)0, std::min(n, chunk));
+    if (next < n) fn(next, n);
+    for (auto &t : th) t.join();
+}
+
+// fn(column of the caller's matrix, slot) for the particles [q0, q1) of the fields.
+template <class T, class F>
+void each_particle(T *const *P, const std::vector<int64_t> &off, int64_t ld, int64_t q0, int64_t q1,
+                   F fn)
+{
+    size_t fk = std::upper_bound(off.begin(), off.end(), q0) - off.begin() - 1;
+    for (int64_t q = q0; q < q1; ++fk)
+        for (; q < std::min(off[fk + 1], q1); ++q) fn(P[fk] + (q - off[fk]) * ld, q);
+}
+
 int upload_fields(vpmx_ctx *c, int nf, const double *const *P, const int64_t *nps,
                   const vpmx_layout *L, bool with_uj)
 {
@@ -515,34 +552,50 @@ int upload_fields(vpmx_ctx *c, int nf, const double *const *P, const int64_t *np
     double *h = c->h_stage;
     uint8_t *hs = (uint8_t *)(h + nd);
     const int64_t ld = L->nrows;
-    bool any_static = false;
-    for (int fk = 0; fk < nf; ++fk) {
-        for (int64_t p = 0; p < nps[fk]; ++p) {
-            const double *col = P[fk] + p * ld;
-            const int64_t q = off[fk] + p;
+    std::atomic<bool> any_static{false};
+    std::atomic<int64_t> bad{np};   // first particle with values that are refused
+    host_for(np, [&](int64_t q0, int64_t q1) {
+        bool stat = false;
+        int64_t first = np;
+        each_particle(P, off, ld, q0, q1, [&](const double *col, int64_t q) {
+            bool ok = true;
             for (int k = 0; k < 3; ++k) {
                 const double x = col[L->X + k], g = col[L->Gamma + k];
-                if (!isfinite(x) || !isfinite(g))
-                    return fail(c, VPMX_EINVAL,
-                                where(nf, fk, p) + " has a non-finite position or circulation");
+                ok &= isfinite(x) && isfinite(g);
                 h[k * np + q] = x;
                 h[(3 + k) * np + q] = g;
             }
             const double sg = col[L->sigma];
-            if (!(sg > 0.0) || !isfinite(sg))
-                return fail(c, VPMX_EINVAL, where(nf, fk, p) + " has sigma = " + std::to_string(sg) +
-                                                " (must be positive and finite)");
+            ok &= sg > 0.0 && isfinite(sg);
+            if (!ok) first = std::min(first, q);
             h[6 * np + q] = sg;
             for (int k = 0; k < 3; ++k) h[(7 + k) * np + q] = L->C >= 0 ? col[L->C + k] : 0.0;
             h[10 * np + q] = L->vol >= 0 ? col[L->vol] : sg * sg * sg;
             const uint8_t st = (L->static_ >= 0 && col[L->static_] != 0.0) ? 1 : 0;
             hs[q] = st;
-            any_static |= st != 0;
+            stat |= st != 0;
             if (with_uj) {
                 for (int k = 0; k < 3; ++k) h[(11 + k) * np + q] = col[L->U + k];
                 for (int k = 0; k < 9; ++k) h[(14 + k) * np + q] = col[L->J + k];
             }
+        });
+        if (stat) any_static = true;
+        for (int64_t b = bad; first < b && !bad.compare_exchange_weak(b, first);) {
         }
+    });
+    if (bad < np) {
+        int rc = VPMX_OK;
+        each_particle(P, off, ld, bad, bad + 1, [&](const double *col, int64_t q) {
+            const int fk = (int)(std::upper_bound(off.begin(), off.end(), q) - off.begin()) - 1;
+            const std::string who = where(nf, fk, q - off[fk]);
+            const double sg = col[L->sigma];
+            bool xg = true;
+            for (int k = 0; k < 3; ++k) xg &= isfinite(col[L->X + k]) && isfinite(col[L->Gamma + k]);
+            rc = fail(c, VPMX_EINVAL,
+                      xg ? who + " has sigma = " + std::to_string(sg) + " (must be positive and finite)"
+                         : who + " has a non-finite position or circulation");
+        });
+        return rc;
     }
     f.np = np;
     f.any_static = any_static;
@@ -550,29 +603,24 @@ int upload_fields(vpmx_ctx *c, int nf, const double *const *P, const int64_t *np
     B.off = off;
     if (np == 0) return VPMX_OK;
     hipStream_t st = c->stream;
-    const size_t b = (size_t)np * sizeof(double);
-    for (int k = 0; k < 3; ++k) {
-        VPMX_HIP(c, hipMemcpyAsync(f.X + k * f.cap, h + k * np, b, hipMemcpyHostToDevice, st));
-        VPMX_HIP(c, hipMemcpyAsync(f.G + k * f.cap, h + (3 + k) * np, b, hipMemcpyHostToDevice, st));
-    }
-    VPMX_HIP(c, hipMemcpyAsync(f.sigma, h + 6 * np, b, hipMemcpyHostToDevice, st));
-    for (int k = 0; k < 3; ++k)
-        VPMX_HIP(c, hipMemcpyAsync(f.C + k * f.cap, h + (7 + k) * np, b, hipMemcpyHostToDevice, st));
-    VPMX_HIP(c, hipMemcpyAsync(f.vol, h + 10 * np, b, hipMemcpyHostToDevice, st));
-    VPMX_HIP(c, hipMemcpyAsync(f.is_static, hs, (size_t)np, hipMemcpyHostToDevice, st));
+    FieldRows R;
+    for (int k = 0; k < 3; ++k) R.add(k, f.X + k * f.cap);
+    for (int k = 0; k < 3; ++k) R.add(3 + k, f.G + k * f.cap);
+    R.add(6, f.sigma);
+    for (int k = 0; k < 3; ++k) R.add(7 + k, f.C + k * f.cap);
+    R.add(10, f.vol);
     if (with_uj) {
-        for (int k = 0; k < 3; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(f.U + k * f.cap, h + (11 + k) * np, b, hipMemcpyHostToDevice, st));
-        for (int k = 0; k < 9; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(f.J + k * f.cap, h + (14 + k) * np, b, hipMemcpyHostToDevice, st));
+        for (int k = 0; k < 3; ++k) R.add(11 + k, f.U + k * f.cap);
+        for (int k = 0; k < 9; ++k) R.add(14 + k, f.J + k * f.cap);
     }
+    VPMX_HIP(c, launch_rows_in(st, R, h, (int64_t)nd, f.is_static, np));
     if (B.nfields) {
         VPMX_TRY(ensure_batch(c, nf, np));
         VPMX_HIP(c, hipMemcpyAsync(B.doff, off.data(), off.size() * sizeof(int64_t),
                                    hipMemcpyHostToDevice, st));
         VPMX_HIP(c, launch_batch_fid(st, B, np));
     }
-    return sync(c);   // staging is reused: the copies must finish
+    return sync(c);   // staging is reused: it must have been read
 }
 
 int upload(vpmx_ctx *c, const double *P, int64_t np, const vpmx_layout *L, bool with_uj)
@@ -590,33 +638,25 @@ int download_fields(vpmx_ctx *c, int nf, double *const *P, const vpmx_layout *L,
     const std::vector<int64_t> &off = c->b.off;
     VPMX_TRY(ensure_stage(c, (size_t)25 * np * sizeof(double)));
     double *h = c->h_stage;
-    hipStream_t st = c->stream;
-    const size_t b = (size_t)np * sizeof(double);
+    FieldRows R;
     if (what & DL_STATE) {
-        for (int k = 0; k < 3; ++k) {
-            VPMX_HIP(c, hipMemcpyAsync(h + k * np, f.X + k * f.cap, b, hipMemcpyDeviceToHost, st));
-            VPMX_HIP(c, hipMemcpyAsync(h + (3 + k) * np, f.G + k * f.cap, b, hipMemcpyDeviceToHost, st));
-        }
-        VPMX_HIP(c, hipMemcpyAsync(h + 6 * np, f.sigma, b, hipMemcpyDeviceToHost, st));
+        for (int k = 0; k < 3; ++k) R.add(k, f.X + k * f.cap);
+        for (int k = 0; k < 3; ++k) R.add(3 + k, f.G + k * f.cap);
+        R.add(6, f.sigma);
     }
     if (what & DL_UJ) {
-        for (int k = 0; k < 3; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(h + (7 + k) * np, f.U + k * f.cap, b, hipMemcpyDeviceToHost, st));
-        for (int k = 0; k < 9; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(h + (10 + k) * np, f.J + k * f.cap, b, hipMemcpyDeviceToHost, st));
+        for (int k = 0; k < 3; ++k) R.add(7 + k, f.U + k * f.cap);
+        for (int k = 0; k < 9; ++k) R.add(10 + k, f.J + k * f.cap);
     }
     const bool sfs = (what & DL_SFS) != 0;
     if (sfs) {
-        for (int k = 0; k < 3; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(h + (19 + k) * np, f.E + k * f.cap, b, hipMemcpyDeviceToHost, st));
-        for (int k = 0; k < 3; ++k)
-            VPMX_HIP(c, hipMemcpyAsync(h + (22 + k) * np, f.C + k * f.cap, b, hipMemcpyDeviceToHost, st));
+        for (int k = 0; k < 3; ++k) R.add(19 + k, f.E + k * f.cap);
+        for (int k = 0; k < 3; ++k) R.add(22 + k, f.C + k * f.cap);
     }
+    VPMX_HIP(c, launch_rows_out(c->stream, R, h, np));
     VPMX_TRY(sync(c));
-    const int64_t ld = L->nrows;
-    for (int fk = 0; fk < nf; ++fk) {
-        for (int64_t q = off[fk]; q < off[fk + 1]; ++q) {
-            double *col = P[fk] + (q - off[fk]) * ld;
+    host_for(np, [&](int64_t q0, int64_t q1) {
+        each_particle(P, off, L->nrows, q0, q1, [&](double *col, int64_t q) {
             if (what & DL_STATE) {
                 for (int k = 0; k < 3; ++k) {
                     col[L->X + k] = h[k * np + q];
@@ -634,8 +674,8 @@ int download_fields(vpmx_ctx *c, int nf, double *const *P, const vpmx_layout *L,
                 if (L->C >= 0)
                     for (int k = 0; k < 3; ++k) col[L->C + k] = h[(22 + k) * np + q];
             }
-        }
-    }
+        });
+    });
     return VPMX_OK;
 }
 
