@@ -113,9 +113,11 @@ constexpr int P2P_CHUNK = 512;
 // Scratch of the device dual-tree traversal.
 struct DttBufs {
     int64_t cap_front = 0, cap_next = 0, cap_m2l = 0, cap_p2p = 0, cap_count = 0, cap_tmpk = 0;
+    int64_t cap_bsum = 0, cap_boff = 0;
     int2 *front = nullptr, *next = nullptr;
-    int *cnt_next = nullptr, *cnt_m2l = nullptr, *cnt_p2p = nullptr;
-    int64_t *off_next = nullptr, *off_m2l = nullptr, *off_p2p = nullptr;
+    uint16_t *act = nullptr;                 // per frontier pair: kind | children << 3
+    uint64_t *bsum = nullptr;                // per block of pairs: packed output counts
+    int64_t *boff = nullptr;                 // their exclusive sums, 3 per block
     uint64_t *m2l_keys = nullptr, *p2p_keys = nullptr, *keys_tmp = nullptr;
     int64_t *totals = nullptr;               // 3 counts + pair total
     int64_t *h_totals = nullptr;             // pinned

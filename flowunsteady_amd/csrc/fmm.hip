@@ -2293,8 +2293,11 @@ hipError_t launch_fmm_pse(hipStream_t st, const FmmState &S, int kernel, const D
 // ---------------------------------------------------------------------------
 // Level-synchronous: every frontier pair (target a, source b) is classified by
 // the same rules as fmm_traverse (M2L, P2P, or a split into child pairs);
-// exclusive scans of the per-pair output counts give each pair fixed output
-// slots, so the lists are deterministic without atomics.  The M2L and P2P
+// exclusive sums of the output counts in frontier order give each pair fixed
+// output slots, so the lists are deterministic without atomics.  A level is three
+// launches: pairs classified and counted per block, the blocks' counts summed up
+// by one workgroup (which leaves the level's totals in pinned host memory), and
+// the outputs written.  The M2L and P2P
 // lists are then radix-sorted (stable) on the target bits of their
 // (target, source) keys only: grouped by target for the CSR, each target's
 // sources in emission order (the host traversal orders them by source; the
@@ -2332,62 +2335,145 @@ __device__ __forceinline__ int dtt_action(const int2 pr, const FmmCellDev *__res
     return 4;
 }
 
+// Bound by launches and by the pairs' cells: with three device-wide scans per
+// level over per-pair counts and offsets (36 bytes per pair written and read back)
+// and the acceptance evaluated again to write, a level took 11 launches; rotor of
+// 200,003, 12 levels per UJ, step 50.6 -> 48.6 ms; blob of 786,433, 14 levels,
+// 372 -> 364 ms of device time per step.
+// A block's pairs: DTT_PER consecutive ones per thread.  The counts of a block
+// (children <= 64 each, M2L, P2P) travel packed, 21 bits each.
+constexpr int DTT_PER = 4, DTT_PAIRS = DTT_PER * FMM_BLOCK, DTT_BITS = 21;
+static_assert(64 * DTT_PAIRS < (1 << DTT_BITS), "a block's counts fit their fields");
+
+// kind | nsplit << 3 of a frontier pair, and its packed output counts.
+__device__ __forceinline__ uint64_t dtt_counts(unsigned act)
+{
+    const int kind = act & 7;
+    return (uint64_t)(act >> 3) | (uint64_t)(kind == 0) << DTT_BITS |
+           (uint64_t)(kind == 1) << (2 * DTT_BITS);
+}
+
+// Sum of v over the threads before this one; total over the block.
+__device__ __forceinline__ uint64_t dtt_block_scan(uint64_t v, uint64_t &total)
+{
+    __shared__ uint64_t wsum[FMM_BLOCK / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint64_t x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = __shfl_up((unsigned long long)x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    uint64_t before = 0;
+    total = 0;
+    for (int k = 0; k < FMM_BLOCK / 64; ++k) {
+        if (k < w) before += wsum[k];
+        total += wsum[k];
+    }
+    return before + x - v;
+}
+
 __global__ __launch_bounds__(FMM_BLOCK) void dtt_classify_kernel(const int2 *__restrict__ fr,
                                                                  int64_t nf,
                                                                  const FmmCellDev *__restrict__ cells,
                                                                  double theta, double sigcut,
-                                                                 int *__restrict__ cnext,
-                                                                 int *__restrict__ cm2l,
-                                                                 int *__restrict__ cp2p)
+                                                                 uint16_t *__restrict__ act,
+                                                                 uint64_t *__restrict__ bsum)
 {
-    const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (i >= nf) return;
-    int ns;
-    const int kind = dtt_action(fr[i], cells, theta, sigcut, ns);
-    cnext[i] = ns;
-    cm2l[i] = kind == 0;
-    cp2p[i] = kind == 1;
+    const int64_t i0 = (int64_t)blockIdx.x * DTT_PAIRS + threadIdx.x * DTT_PER;
+    uint64_t v = 0, total;
+    for (int k = 0; k < DTT_PER; ++k) {
+        if (i0 + k >= nf) break;
+        int ns;
+        const int kind = dtt_action(fr[i0 + k], cells, theta, sigcut, ns);
+        const unsigned a = (unsigned)kind | (unsigned)ns << 3;
+        act[i0 + k] = (uint16_t)a;
+        v += dtt_counts(a);
+    }
+    dtt_block_scan(v, total);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = total;
+}
+
+// Exclusive sums of the blocks' counts (boff[k nblk + b]) and the level's totals,
+// one workgroup: a run of consecutive blocks per thread, the threads' sums
+// scanned in LDS.
+constexpr int DTT_SCAN = 1024;
+__global__ __launch_bounds__(DTT_SCAN) void dtt_block_offsets_kernel(const uint64_t *__restrict__ bsum,
+                                                                     int64_t nblk,
+                                                                     int64_t *__restrict__ boff,
+                                                                     int64_t *__restrict__ totals)
+{
+    __shared__ int64_t wsum[3][DTT_SCAN / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int64_t run = (nblk + DTT_SCAN - 1) / DTT_SCAN;
+    const int64_t b0 = min(nblk, t * run), b1 = min(nblk, b0 + run);
+    constexpr uint64_t mask = ((uint64_t)1 << DTT_BITS) - 1;
+    int64_t v[3] = {0, 0, 0};
+    for (int64_t b = b0; b < b1; ++b)
+        for (int k = 0; k < 3; ++k) v[k] += (int64_t)((bsum[b] >> (k * DTT_BITS)) & mask);
+    int64_t x[3];
+    for (int k = 0; k < 3; ++k) {
+        x[k] = v[k];
+        for (int o = 1; o < 64; o <<= 1) {
+            const int64_t y = __shfl_up((long long)x[k], o);
+            if (lane >= o) x[k] += y;
+        }
+        if (lane == 63) wsum[k][w] = x[k];
+    }
+    __syncthreads();
+    for (int k = 0; k < 3; ++k) {
+        int64_t before = 0;
+        for (int q = 0; q < w; ++q) before += wsum[k][q];
+        if (t == DTT_SCAN - 1) totals[k] = before + x[k];
+        x[k] = before + x[k] - v[k];
+    }
+    for (int64_t b = b0; b < b1; ++b)
+        for (int k = 0; k < 3; ++k) {
+            boff[k * nblk + b] = x[k];
+            x[k] += (int64_t)((bsum[b] >> (k * DTT_BITS)) & mask);
+        }
 }
 
 __global__ __launch_bounds__(FMM_BLOCK) void dtt_emit_kernel(
-    const int2 *__restrict__ fr, int64_t nf, const FmmCellDev *__restrict__ cells, double theta,
-    double sigcut, const int64_t *__restrict__ onext, const int64_t *__restrict__ om2l,
-    const int64_t *__restrict__ op2p, int2 *__restrict__ next, uint64_t *__restrict__ m2l,
-    uint64_t *__restrict__ p2p, int64_t m2l_base, int64_t p2p_base, int nb)
+    const int2 *__restrict__ fr, int64_t nf, const FmmCellDev *__restrict__ cells,
+    const uint16_t *__restrict__ act, const int64_t *__restrict__ boff, int64_t nblk,
+    int2 *__restrict__ next, uint64_t *__restrict__ m2l, uint64_t *__restrict__ p2p,
+    int64_t m2l_base, int64_t p2p_base, int nb)
 {
-    const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (i >= nf) return;
-    const int2 pr = fr[i];
-    int ns;
-    const int kind = dtt_action(pr, cells, theta, sigcut, ns);
-    const uint64_t key = ((uint64_t)pr.x << nb) | (uint64_t)pr.y;
-    if (kind == 0) {
-        m2l[m2l_base + om2l[i]] = key;
-    } else if (kind == 1) {
-        p2p[p2p_base + op2p[i]] = key;
-    } else {
-        const FmmCellDev A = cells[pr.x], B = cells[pr.y];
-        int64_t o = onext[i];
-        if (kind == 2) {
-            for (int a = 0; a < A.nchild; a++)
-                for (int b = 0; b < A.nchild; b++) next[o++] = make_int2(A.child0 + a, A.child0 + b);
+    const int64_t i0 = (int64_t)blockIdx.x * DTT_PAIRS + threadIdx.x * DTT_PER;
+    unsigned a[DTT_PER];
+    uint64_t v = 0, total;
+    for (int k = 0; k < DTT_PER; ++k) {
+        a[k] = i0 + k < nf ? act[i0 + k] : 7u;   // 7: no outputs
+        v += dtt_counts(a[k]);
+    }
+    const uint64_t e = dtt_block_scan(v, total);
+    constexpr uint64_t mask = ((uint64_t)1 << DTT_BITS) - 1;
+    int64_t on = boff[blockIdx.x] + (int64_t)(e & mask);
+    int64_t om = m2l_base + boff[nblk + blockIdx.x] + (int64_t)((e >> DTT_BITS) & mask);
+    int64_t op = p2p_base + boff[2 * nblk + blockIdx.x] + (int64_t)(e >> (2 * DTT_BITS));
+    for (int k = 0; k < DTT_PER; ++k) {
+        const int kind = a[k] & 7;
+        if (kind > 4) break;
+        const int2 pr = fr[i0 + k];
+        const uint64_t key = ((uint64_t)pr.x << nb) | (uint64_t)pr.y;
+        if (kind == 0) {
+            m2l[om++] = key;
+        } else if (kind == 1) {
+            p2p[op++] = key;
+        } else if (kind == 2) {
+            const FmmCellDev A = cells[pr.x];
+            for (int x = 0; x < A.nchild; x++)
+                for (int y = 0; y < A.nchild; y++) next[on++] = make_int2(A.child0 + x, A.child0 + y);
         } else if (kind == 3) {
-            for (int a = 0; a < A.nchild; a++) next[o++] = make_int2(A.child0 + a, pr.y);
+            const FmmCellDev A = cells[pr.x];
+            for (int x = 0; x < A.nchild; x++) next[on++] = make_int2(A.child0 + x, pr.y);
         } else {
-            for (int b = 0; b < B.nchild; b++) next[o++] = make_int2(pr.x, B.child0 + b);
+            const FmmCellDev B = cells[pr.y];
+            for (int y = 0; y < B.nchild; y++) next[on++] = make_int2(pr.x, B.child0 + y);
         }
     }
-}
-
-// totals[k] = off_k[n-1] + cnt_k[n-1] for the three output kinds
-__global__ void dtt_totals_kernel(int64_t n, const int *cnext, const int *cm2l, const int *cp2p,
-                                  const int64_t *onext, const int64_t *om2l, const int64_t *op2p,
-                                  int64_t *totals)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    totals[0] = onext[n - 1] + cnext[n - 1];
-    totals[1] = om2l[n - 1] + cm2l[n - 1];
-    totals[2] = op2p[n - 1] + cp2p[n - 1];
 }
 
 // CSR offsets from keys sorted by target: off[c] = first key with target >= c.
@@ -2473,6 +2559,8 @@ hipError_t fmm_traverse_device(hipStream_t st, FmmState &S, int64_t ncell, doubl
         VPMX_CHK(hipMalloc((void **)&B.totals, 4 * sizeof(int64_t)));
         VPMX_CHK(hipHostMalloc((void **)&B.h_totals, 4 * sizeof(int64_t), hipHostMallocDefault));
     }
+    int64_t *h_totals_dev = nullptr;
+    VPMX_CHK(hipHostGetDevicePointer((void **)&h_totals_dev, B.h_totals, 0));
     VPMX_CHK(grow(&B.front, B.cap_front, 1, st));
     VPMX_CHK(grow(&B.next, B.cap_next, 1, st));
     const int2 root = make_int2(0, 0);
@@ -2480,50 +2568,23 @@ hipError_t fmm_traverse_device(hipStream_t st, FmmState &S, int64_t ncell, doubl
     int64_t nf = 1, nm2l = 0, np2p = 0;
     while (nf > 0) {
         res.steps++;
-        if (nf > B.cap_count) {
-            int64_t c1 = B.cap_count, c2 = B.cap_count, c3 = B.cap_count, c4 = B.cap_count,
-                    c5 = B.cap_count, c6 = B.cap_count;
-            VPMX_CHK(grow(&B.cnt_next, c1, nf, st));
-            VPMX_CHK(grow(&B.cnt_m2l, c2, nf, st));
-            VPMX_CHK(grow(&B.cnt_p2p, c3, nf, st));
-            VPMX_CHK(grow(&B.off_next, c4, nf, st));
-            VPMX_CHK(grow(&B.off_m2l, c5, nf, st));
-            VPMX_CHK(grow(&B.off_p2p, c6, nf, st));
-            B.cap_count = c1;
-            size_t need = 0;
-            VPMX_CHK(rocprim::exclusive_scan(nullptr, need, B.cnt_next, B.off_next, (int64_t)0,
-                                             (size_t)B.cap_count, rocprim::plus<int64_t>(), st));
-            if (need > B.tmp_bytes) {
-                if (B.tmp) (void)hipFree(B.tmp);
-                B.tmp = nullptr;
-                VPMX_CHK(hipMalloc((void **)&B.tmp, need));
-                B.tmp_bytes = need;
-            }
-        }
-        dtt_classify_kernel<<<gridn(nf, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            B.front, nf, S.cells, theta, sigcut, B.cnt_next, B.cnt_m2l, B.cnt_p2p);
+        const int64_t nblk = (nf + DTT_PAIRS - 1) / DTT_PAIRS;
+        VPMX_CHK(grow(&B.act, B.cap_count, nf, st));
+        VPMX_CHK(grow(&B.bsum, B.cap_bsum, nblk, st));
+        VPMX_CHK(grow(&B.boff, B.cap_boff, 3 * nblk, st));
+        dtt_classify_kernel<<<(unsigned)nblk, FMM_BLOCK, 0, st>>>(B.front, nf, S.cells, theta, sigcut,
+                                                                  B.act, B.bsum);
         VPMX_CHK(hipGetLastError());
-        size_t tb = B.tmp_bytes;
-        VPMX_CHK(rocprim::exclusive_scan(B.tmp, tb, B.cnt_next, B.off_next, (int64_t)0, (size_t)nf,
-                                         rocprim::plus<int64_t>(), st));
-        tb = B.tmp_bytes;
-        VPMX_CHK(rocprim::exclusive_scan(B.tmp, tb, B.cnt_m2l, B.off_m2l, (int64_t)0, (size_t)nf,
-                                         rocprim::plus<int64_t>(), st));
-        tb = B.tmp_bytes;
-        VPMX_CHK(rocprim::exclusive_scan(B.tmp, tb, B.cnt_p2p, B.off_p2p, (int64_t)0, (size_t)nf,
-                                         rocprim::plus<int64_t>(), st));
-        dtt_totals_kernel<<<1, 64, 0, st>>>(nf, B.cnt_next, B.cnt_m2l, B.cnt_p2p, B.off_next,
-                                            B.off_m2l, B.off_p2p, B.totals);
+        dtt_block_offsets_kernel<<<1, DTT_SCAN, 0, st>>>(B.bsum, nblk, B.boff, h_totals_dev);
         VPMX_CHK(hipGetLastError());
-        VPMX_CHK(hipMemcpyAsync(B.h_totals, B.totals, 3 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
         VPMX_CHK(hipStreamSynchronize(st));
         const int64_t nn = B.h_totals[0], am = B.h_totals[1], ap = B.h_totals[2];
         VPMX_CHK(grow(&B.next, B.cap_next, nn, st));
         VPMX_CHK(grow(&B.m2l_keys, B.cap_m2l, nm2l + am, st, nm2l));
         VPMX_CHK(grow(&B.p2p_keys, B.cap_p2p, np2p + ap, st, np2p));
-        dtt_emit_kernel<<<gridn(nf, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            B.front, nf, S.cells, theta, sigcut, B.off_next, B.off_m2l, B.off_p2p, B.next,
-            B.m2l_keys, B.p2p_keys, nm2l, np2p, nb);
+        dtt_emit_kernel<<<(unsigned)nblk, FMM_BLOCK, 0, st>>>(B.front, nf, S.cells, B.act, B.boff, nblk,
+                                                              B.next, B.m2l_keys, B.p2p_keys, nm2l,
+                                                              np2p, nb);
         VPMX_CHK(hipGetLastError());
         nm2l += am;
         np2p += ap;

@@ -766,8 +766,8 @@ void free_fmm(FmmState *S)
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     const DttBufs &B = S->dtt;
-    void *dptrs[] = {B.front, B.next, B.cnt_next, B.cnt_m2l, B.cnt_p2p, B.off_next, B.off_m2l,
-                     B.off_p2p, B.m2l_keys, B.p2p_keys, B.keys_tmp, B.totals, B.tmp};
+    void *dptrs[] = {B.front, B.next, B.act, B.bsum, B.boff, B.m2l_keys, B.p2p_keys, B.keys_tmp,
+                     B.totals, B.tmp};
     for (void *p : dptrs)
         if (p) (void)hipFree(p);
     if (B.h_totals) (void)hipHostFree(B.h_totals);
