@@ -2,7 +2,8 @@
 //
 //   uj_f64_kernel      all-pairs U and J in FP64, reference pair algebra
 //                      (src/FLOWUnsteady_processing_force.jl:888-905 extended to
-//                      J = grad U); LDS-tiled sources, one target per lane.
+//                      J = grad U); 64 targets per workgroup, whose waves share
+//                      the LDS tiles of sources.
 //   uj_mixed_kernel    all-pairs U and J with FP32 pair math on Morton-sorted
 //                      targets, coordinates relative to the block's first
 //                      target as FP32 (hi, lo) pairs (lo used within 7
