@@ -132,13 +132,15 @@ struct TreeBufs {
     int64_t cap_cell = 0, cap_lev = 0, cap_flags = 0;
     int32_t *tb = nullptr, *te = nullptr, *lev = nullptr, *child0 = nullptr, *nchild = nullptr;
     uint64_t *pre = nullptr;
-    int32_t *nk = nullptr, *flag = nullptr, *off = nullptr, *foff = nullptr;
+    int32_t *nk = nullptr;
+    uint64_t *bsum = nullptr;                // per block of a level's cells: packed counts
+    int64_t *boff = nullptr;                 // their exclusive sums, 3 per block
     int32_t *kb = nullptr, *ke = nullptr;
     int8_t *ko = nullptr;
     int32_t *lflag = nullptr, *pflag = nullptr, *lscan = nullptr, *pscan = nullptr;
     uint8_t *scan_tmp = nullptr;
     size_t scan_bytes = 0;
-    int32_t *h_tot = nullptr;
+    int64_t *h_tot = nullptr;
 };
 
 // Result sizes of a device traversal.

@@ -2708,60 +2708,66 @@ __global__ void tree_root_kernel(int32_t n, int32_t *tb, int32_t *te, int32_t *l
     parent[0] = -1;
 }
 
-// Level cells [lb, lb + m): child count nk[i], split flag, and the ranges and
-// octants of the non-empty children; entries nk[m] = flag[m] = 0 close the scans.
+// Level cells [lb, lb + m): child count nk[i], the ranges and octants of the
+// non-empty children (an octant ends where the next begins, so 7 searches of the
+// cell's key range), and per block the packed sums of children and split cells.
+// A level is three launches (16 searches and two device-wide scans with their
+// totals copied back one by one, 8 launches, before): UJ of 1,000,003 particles
+// 47.8 -> 46.3 ms, rotor step of 200,003 48.6 -> 47.5.
 __global__ __launch_bounds__(FMM_BLOCK) void tree_split_kernel(
     const uint64_t *__restrict__ key, const int32_t *__restrict__ tb,
     const int32_t *__restrict__ te, const uint64_t *__restrict__ pre,
     const int32_t *__restrict__ lev, int64_t lb, int64_t m, int ncrit, int32_t *__restrict__ nk,
-    int32_t *__restrict__ flag, int32_t *__restrict__ kb, int32_t *__restrict__ ke,
-    int8_t *__restrict__ ko)
+    int32_t *__restrict__ kb, int32_t *__restrict__ ke, int8_t *__restrict__ ko,
+    uint64_t *__restrict__ bsum)
 {
     const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (i > m) return;
-    if (i == m) {
-        nk[m] = 0;
-        flag[m] = 0;
-        return;
-    }
-    const int64_t c = lb + i;
-    const int32_t b = tb[c], e = te[c], l = lev[c];
     int cnt = 0;
-    if (e - b > ncrit && l < KEYBITS) {
-        const int shift = 3 * (KEYBITS - l - 1);
-        for (uint64_t o = 0; o < 8; o++) {
-            const uint64_t cp = (pre[c] << 3) | o;
-            const int32_t bb = key_lower_bound(key, b, e, cp << shift);
-            const int32_t ee = key_lower_bound(key, bb, e, (cp + 1) << shift);
-            if (ee == bb) continue;
-            kb[8 * i + cnt] = bb;
-            ke[8 * i + cnt] = ee;
-            ko[8 * i + cnt] = (int8_t)o;
-            cnt++;
+    if (i < m) {
+        const int64_t c = lb + i;
+        const int32_t b = tb[c], e = te[c], l = lev[c];
+        if (e - b > ncrit && l < KEYBITS) {
+            const int shift = 3 * (KEYBITS - l - 1);
+            int32_t bb = b;
+            for (uint64_t o = 0; o < 8; o++) {
+                const uint64_t cp = (pre[c] << 3) | o;
+                const int32_t ee = o == 7 ? e : key_lower_bound(key, bb, e, (cp + 1) << shift);
+                if (ee == bb) continue;
+                kb[8 * i + cnt] = bb;
+                ke[8 * i + cnt] = ee;
+                ko[8 * i + cnt] = (int8_t)o;
+                cnt++;
+                bb = ee;
+            }
         }
+        nk[i] = cnt;
     }
-    nk[i] = cnt;
-    flag[i] = cnt > 0;
+    uint64_t total;
+    dtt_block_scan((uint64_t)cnt | (uint64_t)(cnt > 0) << DTT_BITS, total);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-// Children of the level's cells from slot le + off[i]; parents' child links.
+// Children of the level's cells from slot le + (children of the cells before);
+// boff: the blocks' offsets (dtt_block_offsets_kernel); parents' child links.
 __global__ __launch_bounds__(FMM_BLOCK) void tree_emit_kernel(
     int64_t lb, int64_t m, int64_t le, const int32_t *__restrict__ nk,
-    const int32_t *__restrict__ off, const int32_t *__restrict__ kb,
+    const int64_t *__restrict__ boff, const int32_t *__restrict__ kb,
     const int32_t *__restrict__ ke, const int8_t *__restrict__ ko, int32_t *__restrict__ tb,
     int32_t *__restrict__ te, uint64_t *__restrict__ pre, int32_t *__restrict__ lev,
     int32_t *__restrict__ child0, int32_t *__restrict__ nchild, int32_t *__restrict__ parent)
 {
     const int64_t i = (int64_t)blockIdx.x * FMM_BLOCK + threadIdx.x;
-    if (i >= m) return;
     const int64_t c = lb + i;
-    const int cnt = nk[i];
+    const int cnt = i < m ? nk[i] : 0;
+    uint64_t total;
+    const uint64_t before = dtt_block_scan((uint64_t)cnt, total);
+    if (i >= m) return;
     if (cnt == 0) {
         child0[c] = -1;
         nchild[c] = 0;
         return;
     }
-    const int64_t first = le + off[i];
+    const int64_t first = le + boff[blockIdx.x] + (int64_t)before;
     child0[c] = (int32_t)first;
     nchild[c] = cnt;
     for (int r = 0; r < cnt; r++) {
@@ -2872,11 +2878,13 @@ static hipError_t grow_keep(T **p, int64_t need, int64_t keep, hipStream_t st)
 
 void free_tree_bufs(TreeBufs &B)
 {
-    for (int32_t **q : {&B.tb, &B.te, &B.lev, &B.child0, &B.nchild, &B.nk, &B.flag, &B.off,
-                        &B.foff, &B.kb, &B.ke, &B.lflag, &B.pflag, &B.lscan, &B.pscan})
+    for (int32_t **q : {&B.tb, &B.te, &B.lev, &B.child0, &B.nchild, &B.nk, &B.kb, &B.ke, &B.lflag,
+                        &B.pflag, &B.lscan, &B.pscan})
         if (*q) { (void)hipFree(*q); *q = nullptr; }
     if (B.pre) (void)hipFree(B.pre);
     if (B.ko) (void)hipFree(B.ko);
+    if (B.bsum) (void)hipFree(B.bsum);
+    if (B.boff) (void)hipFree(B.boff);
     if (B.scan_tmp) (void)hipFree(B.scan_tmp);
     if (B.h_tot) (void)hipHostFree(B.h_tot);
     B = TreeBufs{};
@@ -2917,7 +2925,9 @@ hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncr
                                  FmmPlan &pl, int64_t *nc_out)
 {
     TreeBufs &B = S.tree;
-    if (!B.h_tot) VPMX_CHK(hipHostMalloc((void **)&B.h_tot, 4 * sizeof(int32_t)));
+    if (!B.h_tot) VPMX_CHK(hipHostMalloc((void **)&B.h_tot, 3 * sizeof(int64_t)));
+    int64_t *h_tot_dev = nullptr;
+    VPMX_CHK(hipHostGetDevicePointer((void **)&h_tot_dev, B.h_tot, 0));
     // cell arrays: grown (keeping the built levels) as levels are added
     auto grow_cells = [&](int64_t need, int64_t keep) -> hipError_t {
         if (need <= B.cap_cell) return hipSuccess;
@@ -2936,9 +2946,8 @@ hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncr
         if (m + 1 <= B.cap_lev) return hipSuccess;
         const int64_t c = std::max<int64_t>({m + 1, B.cap_lev + B.cap_lev / 2, 4096});
         VPMX_CHK(grow_keep(&B.nk, c, 0, st));
-        VPMX_CHK(grow_keep(&B.flag, c, 0, st));
-        VPMX_CHK(grow_keep(&B.off, c, 0, st));
-        VPMX_CHK(grow_keep(&B.foff, c, 0, st));
+        VPMX_CHK(grow_keep(&B.bsum, (c + FMM_BLOCK - 1) / FMM_BLOCK, 0, st));
+        VPMX_CHK(grow_keep(&B.boff, 3 * ((c + FMM_BLOCK - 1) / FMM_BLOCK), 0, st));
         VPMX_CHK(grow_keep(&B.kb, 8 * c, 0, st));
         VPMX_CHK(grow_keep(&B.ke, 8 * c, 0, st));
         VPMX_CHK(grow_keep(&B.ko, 8 * c, 0, st));
@@ -2970,20 +2979,19 @@ hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncr
     for (;;) {
         const int64_t m = le - lb;
         VPMX_CHK(grow_level(m));
-        tree_split_kernel<<<gridn(m + 1, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            S.kout, B.tb, B.te, B.pre, B.lev, lb, m, ncrit, B.nk, B.flag, B.kb, B.ke, B.ko);
+        const int64_t nblk = (m + FMM_BLOCK - 1) / FMM_BLOCK;
+        tree_split_kernel<<<(unsigned)nblk, FMM_BLOCK, 0, st>>>(
+            S.kout, B.tb, B.te, B.pre, B.lev, lb, m, ncrit, B.nk, B.kb, B.ke, B.ko, B.bsum);
         VPMX_CHK(hipGetLastError());
-        VPMX_CHK(scan(B.nk, B.off, m + 1));
-        VPMX_CHK(scan(B.flag, B.foff, m + 1));
-        VPMX_CHK(hipMemcpyAsync(&B.h_tot[0], B.off + m, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-        VPMX_CHK(hipMemcpyAsync(&B.h_tot[1], B.foff + m, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        dtt_block_offsets_kernel<<<1, DTT_SCAN, 0, st>>>(B.bsum, nblk, B.boff, h_tot_dev);
+        VPMX_CHK(hipGetLastError());
         VPMX_CHK(hipStreamSynchronize(st));
         const int64_t total = B.h_tot[0];
         nsplit.push_back(B.h_tot[1]);
         levels.push_back({lb, le});
         VPMX_CHK(grow_cells(le + total, le));
         tree_emit_kernel<<<gridn(m, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            lb, m, le, B.nk, B.off, B.kb, B.ke, B.ko, B.tb, B.te, B.pre, B.lev, B.child0, B.nchild,
+            lb, m, le, B.nk, B.boff, B.kb, B.ke, B.ko, B.tb, B.te, B.pre, B.lev, B.child0, B.nchild,
             S.parent);
         VPMX_CHK(hipGetLastError());
         if (total == 0) break;
