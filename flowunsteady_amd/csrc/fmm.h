@@ -167,17 +167,28 @@ struct FmmTables {
     // of b; m2l_rounds = chunks per thread of a 256-thread block (1, 2, 4 or 8).
     std::vector<int> m2l_chunk, m2l_cfirst;
     int m2l_nchunk = 0, m2l_rounds = 1, m2l_chunk_len = 0;
-    // Matrix-core M2L (1 <= P <= M2L_MFMA_MAX_P) in the basis m2l_harm: for element
-    // (row, k) of tile t, at (row + 4 k) m2l_ntiles8 + t, the byte offset of a + b
-    // in E, or of the zero slot after it outside the region and in the padding.
+};
+
+// Tables of the matrix-core M2L (1 <= P <= M2L_MFMA_MAX_P) in one basis (host).
+struct M2LTables {
+    // For element (row, k) of tile t, at (row + 4 k) m2l_ntiles8 + t, the byte offset
+    // of a + b in E, or of the zero slot after it outside the region and in the padding.
+    std::vector<uint16_t> tile_idx;
     // Folding, CSR by basis index: multipole index a and coefficient (with
     // (-1)^|a| / a!); unfolding, CSR by full index b: basis index and
     // coefficient (with 1 / b!).
-    bool m2l_harm = true;
-    std::vector<uint16_t> m2l_tile_idx;
-    std::vector<int> m2l_fold_off, m2l_fold_idx, m2l_unf_off, m2l_unf_idx;
-    std::vector<double> m2l_fold_coef, m2l_unf_coef;
-    std::vector<int> m2l_erec;   // 4 per E entry, packed as m2l_mfma_kernel reads them
+    std::vector<int> fold_off, fold_idx, unf_off, unf_idx;
+    std::vector<double> fold_coef, unf_coef;
+    std::vector<int> erec;   // 4 per E entry, packed as m2l_mfma_kernel reads them
+};
+
+// The same on the device, with the operator rows (M2L_TAB_ROWS x m2l_trow).
+struct M2LBasis {
+    int p = -1;   // order they hold, -1: none
+    uint16_t *tile_idx = nullptr;
+    int *fold_off = nullptr, *fold_idx = nullptr, *unf_off = nullptr, *unf_idx = nullptr;
+    double *fold_coef = nullptr, *unf_coef = nullptr, *etab = nullptr;
+    int4 *erec = nullptr;
 };
 
 // Tree + lists of one evaluation (host).
@@ -211,14 +222,9 @@ struct FmmDev {
     const int4 *m2l_chunks = nullptr;
     const int *m2l_cfirst = nullptr;
     int m2l_nchunk = 0, m2l_rounds = 1;
-    const uint16_t *m2l_tile_idx = nullptr;
-    const int *m2l_fold_off = nullptr, *m2l_fold_idx = nullptr, *m2l_unf_off = nullptr,
-              *m2l_unf_idx = nullptr;
-    const double *m2l_fold_coef = nullptr, *m2l_unf_coef = nullptr;
-    const int4 *m2l_erec = nullptr;
-    const int4 *ijk = nullptr;        // per cell (ix, iy, iz, level)
-    const double *etab = nullptr;     // M2L_TAB_ROWS x m2l_trow operator rows
+    M2LBasis m2l;                     // of the basis m2l_harm
     bool m2l_harm = true;
+    const int4 *ijk = nullptr;        // per cell (ix, iy, iz, level)
     double ext = 1.0;                 // edge of the root cell
     // near-field work items (fmm_p2p_chunks)
     const P2PChunk *chunks = nullptr;
@@ -239,11 +245,9 @@ struct FmmState {
     double *m2m_coef = nullptr, *l2l_coef = nullptr, *m2l_tcoef = nullptr;
     int4 *m2l_chunks = nullptr;
     int *m2l_cfirst = nullptr;
-    uint16_t *m2l_tile_idx = nullptr;
-    int *m2l_fold_off = nullptr, *m2l_fold_idx = nullptr, *m2l_unf_off = nullptr,
-        *m2l_unf_idx = nullptr;
-    double *m2l_fold_coef = nullptr, *m2l_unf_coef = nullptr;
-    int4 *m2l_erec = nullptr;
+    // matrix-core M2L of order dev_tab_p: [0] FULL, [1] HARM, each built at its
+    // first use and kept (a field with an SFS model may use both in turn)
+    M2LBasis m2l[2];
     // near-field work items: per leaf chunk count / partial slots (scanned in
     // place into offsets, nleaf + 1 each), the items, the partial sums
     int64_t cap_leaf = 0, cap_chunk = 0, cap_part = 0, nchunk = 0, nslot = 0;
@@ -266,10 +270,6 @@ struct FmmState {
     double *ssig = nullptr;
     uint8_t *sort_tmp = nullptr;
     size_t sort_bytes = 0;
-    // matrix-core M2L operator rows of order etab_p, basis etab_harm
-    double *etab = nullptr;
-    int etab_p = -1;
-    bool etab_harm = true, dev_tab_harm = true;
     // statistics of the last evaluation
     double stats[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     DttBufs dtt;
@@ -315,13 +315,14 @@ hipError_t fmm_traverse_device(hipStream_t st, FmmState &S, int64_t ncell, doubl
 hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncrit, FmmPlan &pl,
                                  int64_t *nc_out);
 void free_tree_bufs(TreeBufs &B);
-// The operator table of the matrix-core M2L for order P (1..M2L_MFMA_MAX_P) and
-// basis, built once per order from the uploaded recurrence records S.m2l_erec.
-hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P, bool harm);
+// Operator rows B.etab of the matrix-core M2L for order P (1..M2L_MFMA_MAX_P) and
+// basis, from the uploaded recurrence records B.erec.
+hipError_t fmm_m2l_rows(hipStream_t st, M2LBasis &B, int P, bool harm);
 
 void fmm_build_tree(FmmPlan &pl, const uint64_t *key, const double *ssig, int64_t n, int ncrit);
 void fmm_traverse(FmmPlan &pl, double theta, double sigcut);
-void fmm_build_tables(FmmTables &T, int P, bool harm);
+void fmm_build_tables(FmmTables &T, int P);
+void fmm_build_m2l_tables(M2LTables &T, int P, bool harm);
 void fmm_plan_host(FmmPlan &pl, int64_t n, const double *X, const double *sig, int ncrit,
                    double theta, double sigcut);
 

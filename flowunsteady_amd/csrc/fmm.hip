@@ -1490,14 +1490,13 @@ void fmm_traverse(FmmPlan &pl, double theta, double sigcut)
 }
 
 // Operator tables for expansion order P (host build, uploaded once per P).
-void fmm_build_tables(FmmTables &T, int P, bool harm)
+void fmm_build_tables(FmmTables &T, int P)
 {
     MIndex M;
     M.build(P);
     const int K = M.K;
     T.P = P;
     T.K = K;
-    T.m2l_harm = harm;
     T.mi = M.mi;
     // derivative recurrence: idx(k - e_i), idx(k - 2 e_i)
     T.rec1.assign(4 * K, -1);
@@ -1593,93 +1592,6 @@ void fmm_build_tables(FmmTables &T, int P, bool harm)
         T.m2l_rounds = best_rounds;
         T.m2l_chunk_len = best_len;
     }
-    // matrix-core M2L: folding onto the harmonic basis, E records, and the E
-    // offset of every tile element
-    T.m2l_fold_off.clear(); T.m2l_fold_idx.clear(); T.m2l_fold_coef.clear();
-    T.m2l_unf_off.clear(); T.m2l_unf_idx.clear(); T.m2l_unf_coef.clear();
-    T.m2l_erec.clear();
-    T.m2l_tile_idx.clear();
-    if (P >= 1 && P <= M2L_MFMA_MAX_P) {
-        auto fact = [](int n) {
-            double f = 1.0;
-            for (int i = 2; i <= n; i++) f *= i;
-            return f;
-        };
-        const int H = m2l_dim(harm, P), NE = m2l_ne(harm, P), N8 = m2l_ntiles8(harm, P);
-        // basis index of (i, j, r), and E entry of (i, j, k) (-1 where an
-        // exponent is negative)
-        auto hidx = [&](int i, int j, int r) {
-            const int n = i + j + r;
-            return harm ? n * n + (r ? n + 1 : 0) + j : M.idx(i, j, r);
-        };
-        auto eidx = [&](int i, int j, int k) {
-            if (i < 0 || j < 0 || k < 0) return -1;
-            const int n = i + j + k;
-            return harm ? m2l_ebase(true, n) + (k == 0 ? 0 : k == 1 ? n + 1 : 2 * n + 1) + j
-                        : M.idx(i, j, k);
-        };
-        std::vector<int> hm(3 * H);   // exponents of each basis index
-        for (int k = 0; k < K; k++) {
-            const int *m = &M.mi[3 * k];
-            if (harm && m[2] > 1) continue;
-            const int h = hidx(m[0], m[1], m[2]);
-            for (int q = 0; q < 3; q++) hm[3 * h + q] = m[q];
-        }
-        // (I, J, r) collects a = (I - 2t, J - 2u, r + 2(t + u)) with (-1)^q C(q, t), q = t + u
-        T.m2l_fold_off.push_back(0);
-        for (int h = 0; h < H; h++) {
-            const int I = hm[3 * h], J = hm[3 * h + 1], r = hm[3 * h + 2];
-            for (int t = 0; 2 * t <= (harm ? I : 0); t++)
-                for (int u = 0; 2 * u <= (harm ? J : 0); u++) {
-                    const int a[3] = {I - 2 * t, J - 2 * u, r + 2 * (t + u)}, q = t + u;
-                    T.m2l_fold_idx.push_back(M.idx(a[0], a[1], a[2]));
-                    T.m2l_fold_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) *
-                                              ((I + J + r) % 2 ? -1.0 : 1.0) /
-                                              (fact(a[0]) * fact(a[1]) * fact(a[2])));
-                }
-            T.m2l_fold_off.push_back((int)T.m2l_fold_idx.size());
-        }
-        // l'_(i, j, r + 2q) = (-1)^q sum_t C(q, t) l'_(i + 2t, j + 2(q - t), r)
-        T.m2l_unf_off.push_back(0);
-        for (int k = 0; k < K; k++) {
-            const int *m = &M.mi[3 * k];
-            const int q = harm ? m[2] / 2 : 0, r = m[2] - 2 * q;
-            for (int t = 0; t <= q; t++) {
-                T.m2l_unf_idx.push_back(hidx(m[0] + 2 * t, m[1] + 2 * (q - t), r));
-                T.m2l_unf_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) /
-                                         (fact(m[0]) * fact(m[1]) * fact(m[2])));
-            }
-            T.m2l_unf_off.push_back((int)T.m2l_unf_idx.size());
-        }
-        T.m2l_erec.assign(4 * NE, 0);
-        for (int n = 0; n <= P; n++)
-            for (int z = 0; z <= (harm ? std::min(n, 2) : n); z++)
-                for (int y = 0; y <= n - z; y++) {
-                    const int x = n - z - y, k = eidx(x, y, z);
-                    int j[6] = {eidx(x - 1, y, z), eidx(x, y - 1, z), eidx(x, y, z - 1),
-                                eidx(x - 2, y, z), eidx(x, y - 2, z), eidx(x, y, z - 2)};
-                    for (int &v : j)
-                        if (v < 0) v = NE;
-                    // byte offsets of the entries the recurrence reads, and
-                    // k! | |k| << 24 (k! <= 10! < 2^22)
-                    T.m2l_erec[4 * k] = 8 * j[0] | (8 * j[1] << 16);
-                    T.m2l_erec[4 * k + 1] = 8 * j[2] | (8 * j[3] << 16);
-                    T.m2l_erec[4 * k + 2] = 8 * j[4] | (8 * j[5] << 16);
-                    T.m2l_erec[4 * k + 3] = (int)(fact(x) * fact(y) * fact(z)) | (n << 24);
-                }
-        T.m2l_tile_idx.assign((size_t)16 * N8, (uint16_t)(8 * NE));
-        int t = 0;
-        for (int ta = 0; ta < m2l_ntile1(harm, P); ta++)
-            for (int tb = 0; tb < m2l_nrows(harm, P, ta); tb++, t++)
-                for (int e = 0; e < 16; e++) {
-                    const int row = e & 3, kk = e >> 2, a = 4 * ta + kk, b = 4 * tb + row;
-                    if (a >= H || b >= H) continue;
-                    const int *ma = &hm[3 * a], *mb = &hm[3 * b];
-                    const int sx = ma[0] + mb[0], sy = ma[1] + mb[1], sz = ma[2] + mb[2];
-                    if (sx + sy + sz > P) continue;
-                    T.m2l_tile_idx[(size_t)e * N8 + t] = (uint16_t)(8 * eidx(sx, sy, sz));
-                }
-    }
     // L2P: idx(b + e_j) and idx(b + e_j + e_l)
     T.d1.assign(4 * K, -1);
     T.d2a.assign(4 * K, -1);
@@ -1700,6 +1612,95 @@ void fmm_build_tables(FmmTables &T, int P, bool harm)
             if (m < 3) T.d2a[4 * k + m] = v; else T.d2b[4 * k + m - 3] = v;
         }
     }
+}
+
+// Matrix-core M2L of order P (1..M2L_MFMA_MAX_P) and basis: folding onto the
+// basis, E records, and the E offset of every tile element.
+void fmm_build_m2l_tables(M2LTables &T, int P, bool harm)
+{
+    MIndex M;
+    M.build(P);
+    const int K = M.K;
+    T = M2LTables{};
+    auto fact = [](int n) {
+        double f = 1.0;
+        for (int i = 2; i <= n; i++) f *= i;
+        return f;
+    };
+    const int H = m2l_dim(harm, P), NE = m2l_ne(harm, P), N8 = m2l_ntiles8(harm, P);
+    // basis index of (i, j, r), and E entry of (i, j, k) (-1 where an
+    // exponent is negative)
+    auto hidx = [&](int i, int j, int r) {
+        const int n = i + j + r;
+        return harm ? n * n + (r ? n + 1 : 0) + j : M.idx(i, j, r);
+    };
+    auto eidx = [&](int i, int j, int k) {
+        if (i < 0 || j < 0 || k < 0) return -1;
+        const int n = i + j + k;
+        return harm ? m2l_ebase(true, n) + (k == 0 ? 0 : k == 1 ? n + 1 : 2 * n + 1) + j
+                    : M.idx(i, j, k);
+    };
+    std::vector<int> hm(3 * H);   // exponents of each basis index
+    for (int k = 0; k < K; k++) {
+        const int *m = &M.mi[3 * k];
+        if (harm && m[2] > 1) continue;
+        const int h = hidx(m[0], m[1], m[2]);
+        for (int q = 0; q < 3; q++) hm[3 * h + q] = m[q];
+    }
+    // (I, J, r) collects a = (I - 2t, J - 2u, r + 2(t + u)) with (-1)^q C(q, t), q = t + u
+    T.fold_off.push_back(0);
+    for (int h = 0; h < H; h++) {
+        const int I = hm[3 * h], J = hm[3 * h + 1], r = hm[3 * h + 2];
+        for (int t = 0; 2 * t <= (harm ? I : 0); t++)
+            for (int u = 0; 2 * u <= (harm ? J : 0); u++) {
+                const int a[3] = {I - 2 * t, J - 2 * u, r + 2 * (t + u)}, q = t + u;
+                T.fold_idx.push_back(M.idx(a[0], a[1], a[2]));
+                T.fold_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) *
+                                      ((I + J + r) % 2 ? -1.0 : 1.0) /
+                                      (fact(a[0]) * fact(a[1]) * fact(a[2])));
+            }
+        T.fold_off.push_back((int)T.fold_idx.size());
+    }
+    // l'_(i, j, r + 2q) = (-1)^q sum_t C(q, t) l'_(i + 2t, j + 2(q - t), r)
+    T.unf_off.push_back(0);
+    for (int k = 0; k < K; k++) {
+        const int *m = &M.mi[3 * k];
+        const int q = harm ? m[2] / 2 : 0, r = m[2] - 2 * q;
+        for (int t = 0; t <= q; t++) {
+            T.unf_idx.push_back(hidx(m[0] + 2 * t, m[1] + 2 * (q - t), r));
+            T.unf_coef.push_back((q % 2 ? -1.0 : 1.0) * binom(q, t) /
+                                 (fact(m[0]) * fact(m[1]) * fact(m[2])));
+        }
+        T.unf_off.push_back((int)T.unf_idx.size());
+    }
+    T.erec.assign(4 * NE, 0);
+    for (int n = 0; n <= P; n++)
+        for (int z = 0; z <= (harm ? std::min(n, 2) : n); z++)
+            for (int y = 0; y <= n - z; y++) {
+                const int x = n - z - y, k = eidx(x, y, z);
+                int j[6] = {eidx(x - 1, y, z), eidx(x, y - 1, z), eidx(x, y, z - 1),
+                            eidx(x - 2, y, z), eidx(x, y - 2, z), eidx(x, y, z - 2)};
+                for (int &v : j)
+                    if (v < 0) v = NE;
+                // byte offsets of the entries the recurrence reads, and
+                // k! | |k| << 24 (k! <= 10! < 2^22)
+                T.erec[4 * k] = 8 * j[0] | (8 * j[1] << 16);
+                T.erec[4 * k + 1] = 8 * j[2] | (8 * j[3] << 16);
+                T.erec[4 * k + 2] = 8 * j[4] | (8 * j[5] << 16);
+                T.erec[4 * k + 3] = (int)(fact(x) * fact(y) * fact(z)) | (n << 24);
+            }
+    T.tile_idx.assign((size_t)16 * N8, (uint16_t)(8 * NE));
+    int t = 0;
+    for (int ta = 0; ta < m2l_ntile1(harm, P); ta++)
+        for (int tb = 0; tb < m2l_nrows(harm, P, ta); tb++, t++)
+            for (int e = 0; e < 16; e++) {
+                const int row = e & 3, kk = e >> 2, a = 4 * ta + kk, b = 4 * tb + row;
+                if (a >= H || b >= H) continue;
+                const int *ma = &hm[3 * a], *mb = &hm[3 * b];
+                const int sx = ma[0] + mb[0], sy = ma[1] + mb[1], sz = ma[2] + mb[2];
+                if (sx + sy + sz > P) continue;
+                T.tile_idx[(size_t)e * N8 + t] = (uint16_t)(8 * eidx(sx, sy, sz));
+            }
 }
 
 // ---------------------------------------------------------------------------
@@ -2890,24 +2891,17 @@ void free_tree_bufs(TreeBufs &B)
     B = TreeBufs{};
 }
 
-hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P, bool harm)
+hipError_t fmm_m2l_rows(hipStream_t st, M2LBasis &B, int P, bool harm)
 {
-    if (P < 1 || P > M2L_MFMA_MAX_P || (S.etab_p == P && S.etab_harm == harm)) return hipSuccess;
-    if (!S.m2l_erec) return hipErrorInvalidValue;
-    if (S.etab) {
-        VPMX_CHK(hipStreamSynchronize(st));
-        VPMX_CHK(hipFree(S.etab));
-        S.etab = nullptr;
-        S.etab_p = -1;
-    }
-    VPMX_CHK(hipMalloc((void **)&S.etab, (size_t)M2L_TAB_ROWS * m2l_trow(harm, P) * sizeof(double)));
+    if (P < 1 || P > M2L_MFMA_MAX_P || !B.erec || B.etab) return hipErrorInvalidValue;
+    VPMX_CHK(hipMalloc((void **)&B.etab, (size_t)M2L_TAB_ROWS * m2l_trow(harm, P) * sizeof(double)));
     const unsigned g = gridn(M2L_TAB_ROWS, FMM_BLOCK);
 #define VPMX_ETAB(PP)                                                                       \
     case PP:                                                                                \
         if (harm)                                                                           \
-            m2l_etab_kernel<PP, true><<<g, FMM_BLOCK, 0, st>>>(S.m2l_erec, S.etab);         \
+            m2l_etab_kernel<PP, true><<<g, FMM_BLOCK, 0, st>>>(B.erec, B.etab);             \
         else                                                                                \
-            m2l_etab_kernel<PP, false><<<g, FMM_BLOCK, 0, st>>>(S.m2l_erec, S.etab);        \
+            m2l_etab_kernel<PP, false><<<g, FMM_BLOCK, 0, st>>>(B.erec, B.etab);            \
         break;
     switch (P) {
         VPMX_ETAB(1) VPMX_ETAB(2) VPMX_ETAB(3) VPMX_ETAB(4) VPMX_ETAB(5)
@@ -2915,10 +2909,7 @@ hipError_t fmm_m2l_table(hipStream_t st, FmmState &S, int P, bool harm)
     default: return hipErrorInvalidValue;
     }
 #undef VPMX_ETAB
-    VPMX_CHK(hipGetLastError());
-    S.etab_p = P;
-    S.etab_harm = harm;
-    return hipSuccess;
+    return hipGetLastError();
 }
 
 hipError_t fmm_build_tree_device(hipStream_t st, FmmState &S, int64_t n, int ncrit,
@@ -3229,18 +3220,18 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
         if (e != hipSuccess) return e;
     }
     if (d.ncell > 0 && P >= 1 && P <= M2L_MFMA_MAX_P) {
-        if (!d.ijk || !d.etab) return hipErrorInvalidValue;
+        if (!d.ijk || d.m2l.p != P) return hipErrorInvalidValue;
         // the kernel's multipoles lie in L (written only by the unfolding) and its
         // result in M (whose multipoles have no reader after the fold)
         const bool harm = d.m2l_harm;
         const int H = m2l_dim(harm, P), HS = m2l_hrow(harm, P);
         const int64_t nf = ((int64_t)d.ncell + 1) * 3 * HS, nl = (int64_t)d.ncell * 3 * K;
         (harm ? m2l_fold_kernel<true> : m2l_fold_kernel<false>)<<<gridn(nf, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            d.M, d.ncell, K, H, HS, d.m2l_fold_off, d.m2l_fold_idx, d.m2l_fold_coef, d.ijk, d.ext,
+            d.M, d.ncell, K, H, HS, d.m2l.fold_off, d.m2l.fold_idx, d.m2l.fold_coef, d.ijk, d.ext,
             d.L);
         const auto go = [&](auto fn) {
             fn<<<m2l_mfma_grid((const void *)fn, P, harm, d.ncell), 64, 0, st>>>(
-                d.ijk, d.ncell, d.m2l_off, d.m2l_src, d.m2l_erec, d.m2l_tile_idx, d.etab, d.L,
+                d.ijk, d.ncell, d.m2l_off, d.m2l_src, d.m2l.erec, d.m2l.tile_idx, d.m2l.etab, d.L,
                 (int64_t)d.ncell, d.M);
         };
 #define VPMX_M2LM(PP)                                                                           \
@@ -3259,7 +3250,7 @@ hipError_t launch_fmm_eval(hipStream_t st, const FmmDev &d, const FmmPlan &pl, i
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         (harm ? m2l_unfold_kernel<true> : m2l_unfold_kernel<false>)<<<gridn(nl, FMM_BLOCK), FMM_BLOCK, 0, st>>>(
-            d.M, (int64_t)d.ncell * 3, K, H, d.m2l_unf_off, d.m2l_unf_idx, d.m2l_unf_coef, d.ijk,
+            d.M, (int64_t)d.ncell * 3, K, H, d.m2l.unf_off, d.m2l.unf_idx, d.m2l.unf_coef, d.ijk,
             d.ext, d.L);
         e = hipGetLastError();
         if (e != hipSuccess) return e;

@@ -739,16 +739,53 @@ int fmm_tables_to_device(vpmx_ctx *c, FmmState &S)
     VPMX_TRY(upload_as(c, &S.m2l_tcoef, T.m2l_coef));
     VPMX_TRY(upload_as(c, &S.m2l_chunks, T.m2l_chunk));
     VPMX_TRY(upload_as(c, &S.m2l_cfirst, T.m2l_cfirst));
-    VPMX_TRY(upload_as(c, &S.m2l_tile_idx, T.m2l_tile_idx));
-    VPMX_TRY(upload_as(c, &S.m2l_fold_off, T.m2l_fold_off));
-    VPMX_TRY(upload_as(c, &S.m2l_fold_idx, T.m2l_fold_idx));
-    VPMX_TRY(upload_as(c, &S.m2l_fold_coef, T.m2l_fold_coef));
-    VPMX_TRY(upload_as(c, &S.m2l_unf_off, T.m2l_unf_off));
-    VPMX_TRY(upload_as(c, &S.m2l_unf_idx, T.m2l_unf_idx));
-    VPMX_TRY(upload_as(c, &S.m2l_unf_coef, T.m2l_unf_coef));
-    VPMX_TRY(upload_as(c, &S.m2l_erec, T.m2l_erec));
     S.dev_tab_p = T.P;
-    S.dev_tab_harm = T.m2l_harm;
+    return VPMX_OK;
+}
+
+void free_m2l_basis(M2LBasis &B)
+{
+    void *ptrs[] = {B.tile_idx, B.fold_off, B.fold_idx, B.unf_off, B.unf_idx, B.fold_coef,
+                    B.unf_coef, B.etab, B.erec};
+    for (void *p : ptrs)
+        if (p) (void)hipFree(p);
+    B = M2LBasis{};
+}
+
+int m2l_basis_to_device(vpmx_ctx *c, M2LBasis &B, int P, bool harm)
+{
+    M2LTables T;
+    fmm_build_m2l_tables(T, P, harm);
+    free_m2l_basis(B);   // what a call that failed may have left
+    VPMX_TRY(upload_as(c, &B.tile_idx, T.tile_idx));
+    VPMX_TRY(upload_as(c, &B.fold_off, T.fold_off));
+    VPMX_TRY(upload_as(c, &B.fold_idx, T.fold_idx));
+    VPMX_TRY(upload_as(c, &B.fold_coef, T.fold_coef));
+    VPMX_TRY(upload_as(c, &B.unf_off, T.unf_off));
+    VPMX_TRY(upload_as(c, &B.unf_idx, T.unf_idx));
+    VPMX_TRY(upload_as(c, &B.unf_coef, T.unf_coef));
+    VPMX_TRY(upload_as(c, &B.erec, T.erec));
+    VPMX_HIP(c, fmm_m2l_rows(c->stream, B, P, harm));
+    B.p = P;
+    return VPMX_OK;
+}
+
+// Operator tables of an evaluation of order P with the M2L's basis harm.  Those
+// of one order are held at a time, in both bases once both were used: keyed on
+// the basis as well, the tables were rebuilt (a host build, two dozen uploads,
+// hundreds of MB freed and allocated) whenever a UJ without the stretching pass came
+// between mixed steps with an SFS model: 20,000 particles, p = 8, a dynamic step and
+// a UJ 39.4 ms so, 31.4 ms with both kept.
+int fmm_ensure_tables(vpmx_ctx *c, FmmState &S, int P, bool harm)
+{
+    if (S.dev_tab_p != P) {
+        S.dev_tab_p = -1;
+        for (M2LBasis &B : S.m2l) free_m2l_basis(B);
+        fmm_build_tables(S.tab, P);
+        VPMX_TRY(fmm_tables_to_device(c, S));
+    }
+    M2LBasis &B = S.m2l[harm];
+    if (P >= 1 && P <= M2L_MFMA_MAX_P && B.p != P) VPMX_TRY(m2l_basis_to_device(c, B, P, harm));
     return VPMX_OK;
 }
 
@@ -757,14 +794,13 @@ void free_fmm(FmmState *S)
     if (!S) return;
     void *ptrs[] = {S->mi, S->m2m_off, S->l2l_off, S->m2l_toff, S->rec1, S->rec2, S->d1, S->d2a,
                     S->d2b, S->m2m_idx, S->l2l_idx, S->m2l_tidx, S->m2m_coef, S->l2l_coef,
-                    S->m2l_tcoef, S->m2l_chunks, S->m2l_cfirst, S->m2l_tile_idx, S->m2l_fold_off,
-                    S->m2l_fold_idx, S->m2l_fold_coef, S->m2l_unf_off, S->m2l_unf_idx,
-                    S->m2l_unf_coef, S->m2l_erec, S->chunk_buf, S->chunks, S->part, S->chunk_tmp,
-                    S->cells, S->ijk, S->etab, S->leaves, S->parents, S->kids, S->parent,
+                    S->m2l_tcoef, S->m2l_chunks, S->m2l_cfirst, S->chunk_buf, S->chunks, S->part,
+                    S->chunk_tmp, S->cells, S->ijk, S->leaves, S->parents, S->kids, S->parent,
                     S->m2l_off, S->p2p_off, S->m2l_src, S->p2p_src, S->M, S->L, S->kin, S->kout,
                     S->ssig, S->sort_tmp};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    for (M2LBasis &B : S->m2l) free_m2l_basis(B);
     const DttBufs &B = S->dtt;
     void *dptrs[] = {B.front, B.next, B.act, B.bsum, B.boff, B.m2l_keys, B.p2p_keys, B.keys_tmp,
                      B.totals, B.tmp};
@@ -843,20 +879,17 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool harm, bool lis
         MarkScope ms(c, "vpmx fmm tree");
         VPMX_HIP(c, fmm_build_tree_device(st, S, n, P->ncrit, pl, &nc));
     }
-    // device: tables (once per p), expansions
-    if (S.dev_tab_p != P->p || S.dev_tab_harm != harm) {
-        fmm_build_tables(S.tab, P->p, harm);
-        VPMX_TRY(fmm_tables_to_device(c, S));
-    }
-    VPMX_HIP(c, fmm_m2l_table(st, S, P->p, harm));
-    const int K = S.tab.K;
-    // L also holds the multipoles the matrix-core M2L reads (and a zero row)
-    const int64_t ncoef = (nc + 1) * 3 * std::max(K, m2l_hrow(harm, P->p));
-    if (ncoef > S.cap_coef) {
-        const int64_t cap = std::max<int64_t>(ncoef, S.cap_coef + S.cap_coef / 2);
-        VPMX_TRY(dalloc(c, &S.M, cap));
-        VPMX_TRY(dalloc(c, &S.L, cap));
-        S.cap_coef = cap;
+    // device: tables (once per p and basis), expansions
+    if (!lists_only) {
+        VPMX_TRY(fmm_ensure_tables(c, S, P->p, harm));
+        // L also holds the multipoles the matrix-core M2L reads (and a zero row)
+        const int64_t ncoef = (nc + 1) * 3 * std::max(S.tab.K, m2l_hrow(harm, P->p));
+        if (ncoef > S.cap_coef) {
+            const int64_t cap = std::max<int64_t>(ncoef, S.cap_coef + S.cap_coef / 2);
+            VPMX_TRY(dalloc(c, &S.M, cap));
+            VPMX_TRY(dalloc(c, &S.L, cap));
+            S.cap_coef = cap;
+        }
     }
     VPMX_TRY(sync(c));
     const double t1 = now_ms();
@@ -884,7 +917,7 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool harm, bool lis
 
     FmmDev d;
     d.P = P->p;
-    d.K = K;
+    d.K = S.tab.K;
     d.ncell = (int)nc;
     d.nleaf = (int)pl.nleaves;
     d.cells = S.cells;
@@ -919,18 +952,10 @@ int run_fmm(vpmx_ctx *c, const vpmx_uj_params *P, int reset, bool harm, bool lis
     d.m2l_cfirst = S.m2l_cfirst;
     d.m2l_nchunk = S.tab.m2l_nchunk;
     d.m2l_rounds = S.tab.m2l_rounds;
-    d.m2l_tile_idx = S.m2l_tile_idx;
-    d.m2l_fold_off = S.m2l_fold_off;
-    d.m2l_fold_idx = S.m2l_fold_idx;
-    d.m2l_fold_coef = S.m2l_fold_coef;
-    d.m2l_unf_off = S.m2l_unf_off;
-    d.m2l_unf_idx = S.m2l_unf_idx;
-    d.m2l_unf_coef = S.m2l_unf_coef;
-    d.m2l_erec = S.m2l_erec;
-    d.ijk = S.ijk;
-    d.etab = S.etab;
-    d.ext = pl.ext;
+    d.m2l = S.m2l[harm];
     d.m2l_harm = harm;
+    d.ijk = S.ijk;
+    d.ext = pl.ext;
     d.chunks = S.chunks;
     d.chunk_off = S.chunk_off;
     d.part_base = S.part_base;
