@@ -498,18 +498,21 @@ std::string where(int nf, int k, int64_t p)
     return s;
 }
 
-// fn(begin, end), which throws nothing, over [0, n): one host thread per HOST_GRAIN
-// particles, at most 16; what threads that could not be had would have taken
-// runs on the caller.  A particle is 344 bytes of the caller's matrix, 11 to 37 of
-// its 43 values touched: one thread moved 1,000,003 in about 15 ms each way (UJ
-// 76 -> 49 ms), 131,072 in 2 ms (4,099 probes 5.6 -> 2.7 ms).  Below HOST_GRAIN a
-// thread costs more to start (about 15 us) than its share saves.
-constexpr int64_t HOST_GRAIN = 16384;
+// fn(begin, end), which throws nothing, over [0, n): the caller alone below HOST_MIN
+// particles, from there one host thread per HOST_GRAIN, at most 16; what threads
+// that could not be had would have taken runs on the caller.  A particle is 344
+// bytes of the caller's matrix, 11 to 37 of its 43 values touched: one thread moved
+// 1,000,003 in about 15 ms each way (UJ 76 -> 49 ms), 131,072 in 2 ms.  Starting
+// threads and waiting for them costs up to 0.4 ms a call, so with few the shares
+// save less: field up and state down on one thread / on n / HOST_GRAIN, medians,
+// 35,500 particles 0.67 / 1.10 ms, 50,000 0.94 / 1.14, 70,000 1.4 / 1.3, 100,000
+// 2.6 / 1.6.
+constexpr int64_t HOST_GRAIN = 16384, HOST_MIN = 65536;
 template <class F>
 void host_for(int64_t n, F fn)
 {
     const int64_t nt = std::min<int64_t>({n / HOST_GRAIN, 16, (int64_t)std::thread::hardware_concurrency()});
-    if (nt <= 1) return fn((int64_t)0, n);
+    if (n < HOST_MIN || nt <= 1) return fn((int64_t)0, n);
     const int64_t chunk = (n + nt - 1) / nt;
     std::vector<std::thread> th;
     int64_t next = chunk;   // first particle no thread has taken; [0, chunk) is the caller's
