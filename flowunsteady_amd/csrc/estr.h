@@ -5,12 +5,15 @@
 // as the direct and the near-field kernels share it.
 //
 // S is linear in both arguments, so with J, DJ taken relative to a reference
-// (the first target of the workgroup)
 //   E_i = S(J_i, sum_j zeta_j Gamma_j) - sum_j zeta_j S(J_j, Gamma_j):
 // the stretching of a source is formed once when its record enters LDS, and a
-// pair adds 6 products (15 with D[E]) in place of 21 (45).  The reference keeps
-// the two parts near the size of J's variation over the neighbours that zeta
-// reaches.  A particle's own term, zero, is left out by index, so that an
+// pair adds 6 products (15 with D[E]) in place of 21 (45).  The reference is the
+// J (and the DJ) of least norm among the workgroup's targets (estr_least): then
+// |J_i - J_ref| <= 2 |J_i|, so that the two parts round no coarser than the J_i and
+// J_j they are made of, also where the workgroup holds a far stronger vortex, and
+// near the size of J's variation where J is smooth.  (With the first target as the
+// reference a weak cluster in a strong vortex's workgroup lost the digits of their
+// ratio.)  A particle's own term, zero, is left out by index, so that an
 // isolated particle gets E = 0 and no rounding of its own stretching.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -41,6 +44,36 @@ __device__ __forceinline__ void estr_rec_j(const double4 *r, double *Jv, double 
         DJv[0] = q4.y; DJv[1] = q4.z; DJv[2] = q4.w;
         DJv[3] = q5.x; DJv[4] = q5.y; DJv[5] = q5.z; DJv[6] = q5.w;
         DJv[7] = q6.x; DJv[8] = q6.y;
+    }
+}
+
+// The index, over the wave's lanes, whose J has the least norm (to 20 bits; NaN
+// last, ties to the lowest index): the same in every lane.
+__device__ __forceinline__ int estr_least(const double J[9], int index)
+{
+    double q = 0.0;
+    for (int k = 0; k < 9; ++k) q += fabs(J[k]);
+    uint64_t key = (uint64_t)(uint32_t)__double2hiint(q) << 32 | (uint32_t)index;
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint64_t other = __shfl_xor((unsigned long long)key, o);
+        key = other < key ? other : key;
+    }
+    return __builtin_amdgcn_readfirstlane((int)(uint32_t)key);
+}
+
+// J and DJ of the references among the records rec[NR index], index = the lane's own.
+template <bool DYN>
+__device__ __forceinline__ void estr_reference(const double4 *rec, int index, double Jr[9],
+                                               double DJr[9])
+{
+    constexpr int NR = ESTR_NR<DYN>;
+    double J[9], DJ[9], other[9];
+    estr_rec_j<DYN>(rec + NR * index, J, DJ);
+    const int ij = estr_least(J, index);
+    estr_rec_j<DYN>(rec + NR * ij, Jr, other);
+    if constexpr (DYN) {
+        const int id = estr_least(DJ, index);
+        estr_rec_j<DYN>(rec + NR * id, other, DJr);
     }
 }
 

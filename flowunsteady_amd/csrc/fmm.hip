@@ -1759,7 +1759,7 @@ __global__ __launch_bounds__(P2P_BLOCK) void fmm_estr_kernel(const P2PChunk *__r
         const double4 *ri = rec + NR * (tb + t);
         const double xi = ri[0].x, yi = ri[0].y, zi = ri[0].z;
         double Jr[9], DJr[9];
-        estr_rec_j<DYN>(rec + NR * tb, Jr, DJr);
+        estr_reference<DYN>(rec + NR * tb, t, Jr, DJr);
         EstrAcc acc;
         for (int64_t eb = ch.e0; eb < ch.e1; eb += P2P_SLOTS) {
             const int nl = (int)min<int64_t>(P2P_SLOTS, ch.e1 - eb);

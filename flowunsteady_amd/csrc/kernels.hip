@@ -936,7 +936,7 @@ __global__ __launch_bounds__(UJ_BLOCK) void estr_f64_kernel(const double4 *__res
     const double4 *ri = src + NR * it;
     const double xi = ri[0].x, yi = ri[0].y, zi = ri[0].z;
     double Jr[9], DJr[9];
-    estr_rec_j<DYN>(src + NR * t0, Jr, DJr);
+    estr_reference<DYN>(src + NR * t0, (int)(it - t0), Jr, DJr);
     EstrAcc e;
     for (int64_t base = s0; base < s1; base += UJ_BLOCK) {
         __syncthreads();
