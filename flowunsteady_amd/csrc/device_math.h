@@ -115,11 +115,16 @@ __device__ __forceinline__ double eta_f64(double rho)
 //                loses the digits of g ~ rho^3 as rho -> 0, so on x < 2.25
 //                g/(sqrt(2/pi) rho^3) is a degree-12 polynomial in x (relative
 //                error 2e-18); it runs only when some lane of the wave needs it.
+//   gaussian     with y = rho^3, g = 1 - e^{-y}, which loses the digits of y in
+//                the same way: on y < 0.729 (1 - e^{-y})/(3 y) is a polynomial
+//                of degree 11 in y through its Chebyshev points (relative error
+//                4e-19), again only when some lane of the wave needs it.
 //   B            from A and E: g' = sqrt(2/pi) rho^2 E gives
-//                  B = (sqrt(2/pi) E / sigma^3 - 3 A) / r^2.
-// Largest relative errors, all in units of 1e-16 against 50 digits (the
-// closed forms through libm in brackets): A 2 (6.8e4 at rho = 0.1, 50 at 0.5,
-// 3 beyond 1.5), B r^2 / A 13 (2e5, 140, 13).
+//                  B = (sqrt(2/pi) E / sigma^3 - 3 A) / r^2,
+//                and g' = 3 rho^2 E the same with 3 E (gaussian).
+// Largest relative errors of the gaussian-erf pair, in units of 1e-16 against 50
+// digits (the closed forms through libm in brackets): A 2 (6.8e4 at rho = 0.1, 50
+// at 0.5, 3 beyond 1.5), B r^2 / A 13 (2e5, 140, 13).
 constexpr double EXP_HALF[12] = {
     1.0, -0.5, 0.12500000000000044, -0.02083333333333271, 0.002604166666655789,
     -0.0002604166666737258, 2.1701388986348433e-05, -1.5500991744385246e-06,
@@ -130,6 +135,10 @@ constexpr double GERF_SMALL[13] = {
     0.00023674242414118443, -2.0032050981917798e-05, 1.4467586856913403e-06,
     -9.118156851100948e-08, 5.098357695475492e-09, -2.5590008622494337e-10,
     1.1533875250279058e-11, -4.43463176124452e-13, 1.1180962860624989e-14};
+constexpr double GAUSS_SMALL[12] = {
+    0.3333333333333333, -0.16666666666666663, 0.055555555555552825, -0.013888888888818948,
+    0.0027777777768501506, -0.00046296295569622385, 6.613752999693705e-05, -8.267077184672925e-06,
+    9.18316839368122e-07, -9.147752444530947e-08, 7.994446675776673e-09, -4.983267225562206e-10};
 constexpr double ERFCX_T[12] = {
     3.672063975485439e-05, 0.19869558511481117, 0.20696658778029875, 0.14321399007711033,
     0.3340213070606755, -0.34968381664740894, 1.0381635337255333, -1.3184589318799849,
@@ -138,6 +147,7 @@ constexpr double TWO_LN2_HI = 1.386294361119326, TWO_LN2_LO = 5.647058112606315e
 constexpr double NEG_HALF_LOG2E = -0.7213475204444817;   // -log2(e)/2
 constexpr double ROUND_MAGIC = 6755399441055744.0;       // 1.5 * 2^52
 constexpr double X_SMALL = 2.25;                         // rho^2 below which the series runs
+constexpr double Y_SMALL = 0.729;                        // rho^3 of the gaussian kernel's
 constexpr double X_FAR = 90.25;    // rho = 9.5: 1 - g < 3e-19 and rho g' < 2e-17, the pair is singular
 constexpr double RHO_FAR = 9.5;
 constexpr double X_CORE = 1500.0;  // e^{-x/2} is zero: so are zeta and the core-size derivatives
@@ -227,9 +237,13 @@ __device__ __forceinline__ void radial_f64(double r2, double x, double rinv, dou
             *BD = e * (is * is);
         }
     } else if constexpr (K == GAUSSIAN) {
-        const double rho = r2 * rinv * is;
-        const double E = exp_mhalf(2.0 * rho * rho * rho), e = E * kz;
+        const double rho = r2 * rinv * is, y = rho * rho * rho;
+        const double E = exp_mhalf(2.0 * y), e = E * kz;
         A = (1.0 - E) * (ri2 * rinv);
+        if (__any(y < Y_SMALL)) {
+            const double p = horner_f64(GAUSS_SMALL, y) * kz;
+            A = y < Y_SMALL ? p : A;
+        }
         B = fma(-3.0, A, e) * ri2;
         if constexpr (DYN) {
             *AD = -e;
