@@ -202,12 +202,13 @@ __device__ __forceinline__ double exp_mhalf(double x)
 
 // Constant of a source that its pairs need besides 1/sigma: gaussian-erf
 // sqrt(2/pi)/sigma^3, gaussian 3/sigma^3, Winckelmans sigma^2 (finite also
-// for cores so small that 1/sigma^3 overflows).
+// for cores so small that 1/sigma^3 overflows; NaN for a NaN core).
 template <int K>
 __device__ __forceinline__ double pair_const_f64(double sigma, double is)
 {
-    if constexpr (K == GAUSSIANERF) return fmin(SQRT2_PI * is * is * is, 1e300);
-    else if constexpr (K == GAUSSIAN) return fmin(3.0 * is * is * is, 1e300);
+    const double is3 = is * is * is;
+    if constexpr (K == GAUSSIANERF) return is3 > 1e300 ? 1e300 : SQRT2_PI * is3;
+    else if constexpr (K == GAUSSIAN) return is3 > 1e300 ? 1e300 : 3.0 * is3;
     else if constexpr (K == WINCKELMANS) return sigma * sigma;
     else return 0.0;
 }
@@ -240,9 +241,9 @@ __device__ __forceinline__ void radial_f64(double r2, double x, double rinv, dou
         const double rho = r2 * rinv * is, y = rho * rho * rho;
         const double E = exp_mhalf(2.0 * y), e = E * kz;
         A = (1.0 - E) * (ri2 * rinv);
-        if (__any(y < Y_SMALL)) {
+        if (!__all(y >= Y_SMALL)) {   // with a NaN: exp_mhalf drops it
             const double p = horner_f64(GAUSS_SMALL, y) * kz;
-            A = y < Y_SMALL ? p : A;
+            A = y >= Y_SMALL ? A : p;
         }
         B = fma(-3.0, A, e) * ri2;
         if constexpr (DYN) {
