@@ -198,10 +198,12 @@ __global__ __launch_bounds__(EW_BLOCK) void uj_f64_split_reduce_kernel(const dou
     *o = reset ? v : *o + v;
 }
 
-// Split of an FP64 launch over nt targets and n sources: about 4096 workgroups
-// of 64 targets, so that the few that find near pairs everywhere even out
-// over the 256 CUs, in segments of at least 64 sources.  nseg nt stays below
-// 262,144 + 64 nseg, so the partials fit kpart.
+// Split of an FP64 launch over nt targets and n sources: floor(4096 / nb)
+// segments of at least 64 sources, so more than 2730 and at most 4096
+// workgroups of 64 targets, so that the few that find near pairs everywhere even
+// out over the 256 CUs.  The last size that is split is 131,072 targets (2048
+// blocks, two segments).  nseg nt stays below 262,144 + 64 nseg, so the partials
+// fit kpart.
 struct Split {
     int nseg;
     int64_t seglen;
@@ -220,13 +222,13 @@ static Split split_f64_for(int64_t nt, int64_t n)
 }
 
 // Split of a mixed launch over nb target blocks of 256 and n sources: the
-// source range is cut into segments (whole tiles of 256) so that about 2048
-// workgroups run, twice what the chip holds at a time, the second half evening
-// out near and far blocks.  With 1024 workgroups, and no split from 512 target
-// blocks on, the Winckelmans cube of 131,071 ran as 512 workgroups, two waves
-// per SIMD: 22.7 -> 18.0 ms per UJ.  From 2048 blocks on (n = 524,288) the
-// segments' sums (nseg nt <= 2048 256 slots of 14 doubles, written and read
-// again) would buy nothing.  Partial sums go through `part`.
+// source range is cut into floor(2048 / nb) segments (whole tiles of 256), so that
+// more than 1365 and at most 2048 workgroups run, up to twice what the chip
+// holds at a time, the second half evening out near and far blocks.  With 1024
+// workgroups, and no split from 512 target blocks on, the Winckelmans cube of
+// 131,071 ran as 512 workgroups, two waves per SIMD: 22.7 -> 18.0 ms per UJ.  The
+// last size that is split is n = 262,144 (1024 blocks, two segments); the partial
+// sums, in `part`, fill at most 2048 x 256 slots of 14 doubles.
 static Split split_for(int64_t nb, int64_t n)
 {
     const int64_t nseg = std::min<int64_t>(2048 / std::max<int64_t>(nb, 1), (n + UJ_BLOCK - 1) / UJ_BLOCK);
