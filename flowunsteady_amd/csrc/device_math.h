@@ -206,11 +206,14 @@ __device__ __forceinline__ double exp_mhalf(double x)
 template <int K>
 __device__ __forceinline__ double pair_const_f64(double sigma, double is)
 {
-    const double is3 = is * is * is;
-    if constexpr (K == GAUSSIANERF) return is3 > 1e300 ? 1e300 : SQRT2_PI * is3;
-    else if constexpr (K == GAUSSIAN) return is3 > 1e300 ? 1e300 : 3.0 * is3;
-    else if constexpr (K == WINCKELMANS) return sigma * sigma;
-    else return 0.0;
+    if constexpr (K == GAUSSIANERF || K == GAUSSIAN) {
+        const double k = (K == GAUSSIANERF ? SQRT2_PI : 3.0) * is * is * is;
+        return k > 1e300 ? 1e300 : k;
+    } else if constexpr (K == WINCKELMANS) {
+        return sigma * sigma;
+    } else {
+        return 0.0;
+    }
 }
 
 // A and B of a pair with r2 > 0, x = r2/sigma^2, rinv = 1/r, ri2 = rinv^2;
