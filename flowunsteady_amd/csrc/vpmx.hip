@@ -502,12 +502,13 @@ std::string where(int nf, int k, int64_t p)
 // particles, from there one host thread per HOST_GRAIN, at most 16; what threads
 // that could not be had would have taken runs on the caller.  A particle is 344
 // bytes of the caller's matrix, 11 to 37 of its 43 values touched: one thread moved
-// 1,000,003 in about 15 ms each way (UJ 76 -> 49 ms), 131,072 in 2 ms.  Starting
-// threads and waiting for them costs up to 0.4 ms a call, so with few the shares
-// save less: field up and state down on one thread / on n / HOST_GRAIN, medians,
-// 35,500 particles 0.67 / 1.10 ms, 50,000 0.94 / 1.14, 70,000 1.4 / 1.3, 100,000
-// 2.6 / 1.6.
-constexpr int64_t HOST_GRAIN = 16384, HOST_MIN = 65536;
+// 1,000,003 in about 15 ms each way (UJ 76 -> 49 ms), 131,072 in 2 ms.  Threads cost
+// their start, and take the matrix's lines from the caller's cache where it holds
+// them.  Mixed FMM UJ (p = 2), medians in ms, on the caller alone / on n /
+// HOST_GRAIN threads, one matrix called again and again, and matrices out of cache:
+//   33,000   3.09 / 3.37, 3.38 / 3.48        50,000   3.01 / 3.24, 3.57 / 3.35
+//   40,000   2.73 / 2.94, 3.13 / 3.19        70,000   3.76 / 3.71, 4.48 / 3.86
+constexpr int64_t HOST_GRAIN = 16384, HOST_MIN = 3 * HOST_GRAIN;
 template <class F>
 void host_for(int64_t n, F fn)
 {

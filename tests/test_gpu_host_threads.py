@@ -1,4 +1,4 @@
-"""When host threads gather and scatter the caller's matrix: none below 65,536
+"""When host threads gather and scatter the caller's matrix: none below 49,152
 particles, where starting them costs more than they save, some from there on.
 Thread ids are handed out in sequence, so the ids of two threads started right
 before and after a call tell how many it started; another process can only add
@@ -23,8 +23,8 @@ def thread_id():
     return t.native_id
 
 
-@pytest.mark.parametrize("n,threaded", [(1000, False), (33000, False), (50000, False),
-                                        (65535, False), (65536, True), (200003, True)])
+@pytest.mark.parametrize("n,threaded", [(1000, False), (33000, False), (49151, False),
+                                        (49152, True), (65536, True), (200003, True)])
 def test_threads_of_a_call(n, threaded):
     rng = np.random.default_rng(n)
     pf = make_field(rng.uniform(-1, 1, (n, 3)), rng.normal(0, 1, (n, 3)), np.full(n, 0.1))
