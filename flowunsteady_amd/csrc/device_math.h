@@ -102,7 +102,7 @@ __device__ __forceinline__ double eta_f64(double rho)
 // their error at a few 1e-16, written from the mathematics below instead of
 // through libm's exp, erf, sqrt and division (169 FP64 instructions per near
 // pair with those, 88 so and 16 more where the series runs; one UJ_gpu call on
-// a rotor wake of 70,001: 24.9 -> 14.8 ms, the kernel at the full issue rate):
+// a rotor wake of 70,001: 24.9 -> 14.8 ms, 81 % of the issue cycles in use):
 //
 //   1/r          v_rsq_f64 and one third-order Newton step
 //   e^{-x/2}     2^k P(x + 2 k ln 2), P the degree-11 minimax of e^{-t/2} on
@@ -475,7 +475,7 @@ VPMX_HD void radial_near_f32(float r2, float rinv, float p0, float p1,
 }
 
 // Radial coefficients (A_D, B_D) of the core-size derivative of one pair in
-// FP32 (see h_dh_f64); p0, p1 as for radial_near_f32.
+// FP32 (in FP64: radial_dsig_f64); p0, p1 as for radial_near_f32.
 //   gaussianerf  A_D = -sqrt(2/pi) e^{-rho^2/2} / sigma^3,  B_D = sqrt(2/pi) e^{-rho^2/2} / sigma^5
 //   gaussian     A_D = -3 e^{-rho^3} / sigma^3,             B_D = 9 rho e^{-rho^3} / sigma^5
 //   winckelmans  A_D = -15/2 sigma^4 s^-7,                 B_D = 105/2 sigma^4 s^-9,  s^2 = r^2 + sigma^2

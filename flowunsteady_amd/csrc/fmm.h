@@ -22,11 +22,13 @@ constexpr int FMM_MAX_P = 12;   // K = 455 <= 2 coefficients per thread of 256
 // which gives the same truncated sum.  At P = 8 the operator's region
 // |a| + |b| <= P then holds 1,365 instead of 3,003 entries, a column 81 instead
 // of 165, and E (whose indices a + b have z exponent <= 2) 109 instead of 165.
-// FULL: every coefficient.  Half the speed; kept for the mixed-precision steps
-// with an SFS model, whose stretching pass rounds differences of J to FP32: the
-// other basis' J differs by 1e-15, which flips a few of those roundings, and a
-// particle's Estr or C then moves by an FP32 ulp (up to 1e-7 of the largest of
-// 786,433) from one version of this library to the next.
+// FULL: every coefficient, half the speed and no more accurate.  The mixed
+// evaluations that a stretching pass follows take it: that pass rounds differences
+// of J to FP32, J of the other basis differs by 1e-15, which flips a few of those
+// roundings, and a particle's Estr or C then moves by an FP32 ulp (up to 1.6e-7 of
+// the largest of 786,433).  FULL keeps those outputs where they were, at 49
+// instead of 27 ms per UJ of that field.  (So U and J of a mixed UJ with sfs = 1
+// differ from those with sfs = 0 by that 1e-15.)
 //
 // Coefficient order: graded; FULL as the Cartesian index (x, then y
 // descending); HARM degree n = indices n^2 .. n^2 + 2n: (n-j, j, 0), then

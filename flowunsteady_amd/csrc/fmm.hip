@@ -19,9 +19,8 @@
 // (target A, source B) goes to M2L when (R_A + R_B) < theta |c_A - c_B| and the
 // gap |c_A - c_B| - R_A - R_B >= sigcut * max sigma in B (so the singular far
 // field matches the regularised kernel to its tail), else the larger cell is
-// split; leaf-leaf pairs go to P2P.  The tree build and traversal run on the
-// host from the GPU-sorted keys; every expansion and pair kernel runs on the
-// GPU.
+// split; leaf-leaf pairs go to P2P.  Tree, traversal, expansions and pair kernels
+// all run on the GPU (the host build and traversal here serve the plan counts).
 #include <math.h>
 #include <string.h>
 
@@ -390,8 +389,11 @@ __global__ __launch_bounds__(FMM_BLOCK) void m2l_kernel(const FmmCellDev *__rest
 // every source of the block, one 4 x 4 tile per b-tile, in registers.  At the
 // end the four blocks are added (fixed order).
 //
-// Bound by the LDS gathers (105 ds_read_b64 per group of four sources at P = 8,
-// about 6 cycles each) ahead of the MFMAs (105, 16 cycles on each of 4 SIMDs).
+// At P = 8 bound by the LDS gathers (105 ds_read_b64 per group of four sources,
+// about 6 cycles each) ahead of the MFMAs (105, 16 cycles on each of 4 SIMDs),
+// which are 37 % busy.  At P = 4 on the 15,000 cells of a rotor wake of 200,003
+// (545 sources each) the grid is what binds: one block per 8 cells is 1.2 waves
+// per SIMD, the MFMAs 12 % busy.
 // In the full Cartesian basis (215 tiles; C and B 84 registers each, two waves
 // per SIMD) the kernel was latency-bound at twice the work: blob of 786,433,
 // P = 8, 61.2 -> 27.6 ms per UJ; rotor wake of 1,000,003, core-aware, 28.4 ->
@@ -1032,9 +1034,10 @@ __device__ __forceinline__ int stream_particle(const int32_t *lbeg, const int32_
 
 // P2P near field, FP64: one wave per work item (a target leaf and a run of its
 // list), the source leaves streamed through LDS and the targets of small
-// leaves replicated as in p2p_mixed_kernel: a leaf holds ncrit / 2 particles on
-// average, so with one target per lane half of them idled.  R = 64 / nt slices
-// (at most 16); their values are added in slice order by lane reads.  Adds to
+// leaves replicated as in p2p_mixed_kernel: a leaf of ncrit = 50 holds 14 to 16
+// particles on average on a rotor wake, so with one target per lane most of them
+// idled.  R = 64 / nt slices (at most 16); their values are added in slice order
+// by lane reads.  Adds to
 // U, J (or writes partial sums).  DYN: the core-size derivative D[J] of the
 // dynamic SFS model in the same pass, which shares the separation, the
 // exponential and the cross product; a pass of its own cost 0.69 of this one.
@@ -1043,10 +1046,13 @@ __device__ __forceinline__ int stream_particle(const int32_t *lbeg, const int32_
 // blob the CPU FMM (one sum per target, list order) is 1.3e-12 of max |Gamma|
 // off its own terms added in long double, this kernel 8e-13 (R <= 16: 7e-13,
 // one lane per target: 1.9e-12), and R <= 2 keeps the two within 1e-12 of each
-// other; leaves of ncrit = 50 mostly take R = 2 in any case.
-// Bound by FP64 issue (91 instructions per pair, 112 with D[J]).  Rotor wakes,
-// p = 4, per UJ: 200,003 particles 21.0 -> 7.5 ms; 100,003 with D[J]
-// 13.1 + 9.0 -> 6.6 ms.
+// other.  It leaves lanes repeating slice 0 in every leaf of 21 or fewer targets,
+// which hold more than half of the particles: 0.45 of the lanes are in use.
+// 91 instructions per pair, 112 with D[J].  Rotor wakes, p = 4, per UJ: 200,003
+// particles 21.0 -> 7.3 ms; 100,003 with D[J] 13.1 + 9.0 -> 6.5 ms.  The vector
+// units are 49 % busy (58 with D[J]) and hold 1.8 of the 4 waves that fit a
+// SIMD on average: the items, runs of at most 512 list entries, differ much in
+// length, and the end of the launch runs on the longest few.
 //
 // J is summed with its Kronecker part A eps_klm G_m pair by pair: the two parts
 // of near pairs largely cancel, and summed apart (as the direct kernels do, 3
@@ -1730,7 +1736,8 @@ __device__ __forceinline__ void estr_finish(const double *d, int64_t i, int64_t 
 // Estr over the near-field lists, FP64; DYN adds D[E] (the pair sums of
 // estr.h).  One wave per work item, the source leaves streamed through LDS and
 // the targets of small leaves replicated as in p2p_f64_kernel (with D[E] at most
-// twice, as there).  Bound by FP64 issue, 31 instructions per pair, 42 with D[E].
+// twice, as there).  31 instructions per pair, 42 with D[E]; the vector units are
+// 56 % busy, with the items' lengths and lane use of that kernel.
 // 100,003 particles with D[E], ncrit = 50: 8.6 -> 3.2 ms (one lane per target,
 // leaf by leaf, before).
 template <int KK, bool TRANSPOSED, bool DYN>

@@ -198,10 +198,11 @@ __device__ __forceinline__ void uj_f64_store(const double v[12], int64_t i, int6
 // first target in FP64 and rounded to FP32; FP32 partials are folded into
 // FP64 every MIXED_FOLD pairs (once per tile for far tiles).  d = (U0..2, W0..2, J0..7) before the -1/(4 pi) factor.
 //
-// Bound by FP32 issue: a far pair is 34 instructions, about 74 cycles of its SIMD
-// at the rate of two per four cycles, and takes 105 with four waves per SIMD
-// (cube of 1,048,576: 749 ms per UJ).  Two targets per thread halve the LDS reads
-// but leave two or three waves: 925-1036 ms; five waves spill: 843 ms.  The
+// A far pair is 34 instructions, about 74 cycles of its SIMD at the rate of two per
+// four cycles, and takes 105: the vector units are 71 % busy, and the four waves
+// per SIMD that 112 registers allow do not cover the rest (cube of 1,048,576:
+// 749-765 ms per UJ).  Two targets per thread halve the LDS reads but leave two
+// or three waves: 925-1036 ms; five waves spill: 843 ms.  The
 // unroll counts keep the near loop at 112 VGPRs, four waves (4 and 4 in place of
 // 8 and 2: 753 ms; a batch of 24 fields 45.0 against 43.5).
 //
