@@ -498,32 +498,41 @@ std::string where(int nf, int k, int64_t p)
     return s;
 }
 
-// fn(begin, end), which throws nothing, over [0, n): the caller alone below HOST_MIN
-// particles, from there one host thread per HOST_GRAIN, at most 16; what threads
-// that could not be had would have taken runs on the caller.  A particle is 344
-// bytes of the caller's matrix, 11 to 37 of its 43 values touched: one thread moved
-// 1,000,003 in about 15 ms each way (UJ 76 -> 49 ms), 131,072 in 2 ms.  Threads cost
-// their start, and take the matrix's lines from the caller's cache where it holds
-// them.  Mixed FMM UJ (p = 2), medians in ms, on the caller alone / on n /
-// HOST_GRAIN threads, one matrix called again and again, and matrices out of cache:
-//   33,000   3.09 / 3.37, 3.38 / 3.48        50,000   3.01 / 3.24, 3.57 / 3.35
-//   40,000   2.73 / 2.94, 3.13 / 3.19        70,000   3.76 / 3.71, 4.48 / 3.86
-constexpr int64_t HOST_GRAIN = 16384, HOST_MIN = 3 * HOST_GRAIN;
+// fn(begin, end), which throws nothing, over [0, n) in blocks: the caller and, per
+// HOST_GRAIN particles, one host thread, at most 16 together; without threads
+// that could not be had the others take their blocks.  A particle is 344 bytes of
+// the caller's matrix, 11 to 37 of its 43 values touched: one thread moved
+// 1,000,003 in about 15 ms each way (UJ 76 -> 49 ms), 131,072 in 2 ms.
+// The caller takes its blocks from the front and the threads theirs from the back:
+// a thread starts late, and writes lines that the caller's cache holds from the
+// last call at a fraction of the caller's own speed, so equal shares waited for
+// it, and shares that move would have the caller fetch its lines back.  Mixed FMM UJ
+// (p = 2), medians in ms, alone / equal shares / this, one matrix called again and
+// again, and many that no cache holds:
+//   33,500   3.2 / 3.6 / 3.2,   3.8 / 3.8 / 3.6     100,000   5.7 / 4.8 / 4.7,   6.1 / 4.9 / 4.8
+//   48,500   3.0 / 3.5 / 3.0,   4.1 / 3.7 / 3.6   1,000,000   43.9 / 29.7 / 29.0,   44.2 / 27.9 / 27.2
+// Below 32,768 a thread's start (about 15 us) costs more than it saves.
+constexpr int64_t HOST_GRAIN = 16384, HOST_BLOCK = 2048;
 template <class F>
 void host_for(int64_t n, F fn)
 {
     const int64_t nt = std::min<int64_t>({n / HOST_GRAIN, 16, (int64_t)std::thread::hardware_concurrency()});
-    if (n < HOST_MIN || nt <= 1) return fn((int64_t)0, n);
-    const int64_t chunk = (n + nt - 1) / nt;
+    if (nt <= 1) return fn((int64_t)0, n);
+    const int64_t nb = (n + HOST_BLOCK - 1) / HOST_BLOCK;
+    std::atomic<int64_t> claimed{0}, back{0};
+    const auto work = [&](bool caller) {
+        for (int64_t front = 0; claimed.fetch_add(1, std::memory_order_relaxed) < nb;) {
+            const int64_t b = caller ? front++ : nb - 1 - back.fetch_add(1, std::memory_order_relaxed);
+            fn(b * HOST_BLOCK, std::min(n, (b + 1) * HOST_BLOCK));
+        }
+    };
     std::vector<std::thread> th;
-    int64_t next = chunk;   // first particle no thread has taken; [0, chunk) is the caller's
     try {
         th.reserve(nt - 1);
-        for (; next < n; next += chunk) th.emplace_back(fn, next, std::min(n, next + chunk));
-    } catch (...) {
+        for (int64_t t = 1; t < nt; ++t) th.emplace_back(work, false);
+    } catch (...) {   // fewer threads: the others take their blocks
     }
-    fn((int64_t)0, std::min(n, chunk));
-    if (next < n) fn(next, n);
+    work(true);
     for (auto &t : th) t.join();
 }
 

@@ -1,10 +1,12 @@
-"""When host threads gather and scatter the caller's matrix: none below 49,152
-particles, where starting them costs more than they save, some from there on.
-Thread ids are handed out in sequence, so the ids of two threads started right
-before and after a call tell how many it started; another process can only add
-to that, hence the least of several tries."""
+"""Host threads may not make a call slower: the matrix goes up and the state comes
+back, again and again, right above the size from which threads help (35,500) and
+right below it (32,000).  Per particle the former may not cost more (15 % allowed;
+0.8 is usual).  Equal shares for two threads, of which the late one writes lines
+that the caller's cache holds, cost up to 1.8 times as much, now and then: nine of
+twelve medians have to pass.  And every particle is moved exactly once, whatever
+the share of each thread."""
 import ctypes
-import threading
+import time
 
 import numpy as np
 import pytest
@@ -16,34 +18,42 @@ from helpers import make_field
 pytestmark = pytest.mark.gpu
 
 
-def thread_id():
-    t = threading.Thread(target=lambda: None)
-    t.start()
-    t.join()
-    return t.native_id
-
-
-@pytest.mark.parametrize("n,threaded", [(1000, False), (33000, False), (49151, False),
-                                        (49152, True), (65536, True), (200003, True)])
-def test_threads_of_a_call(n, threaded):
+def field(n):
     rng = np.random.default_rng(n)
-    pf = make_field(rng.uniform(-1, 1, (n, 3)), rng.normal(0, 1, (n, 3)), np.full(n, 0.1))
+    return make_field(rng.uniform(-1, 1, (n, 3)), rng.normal(0, 1, (n, 3)),
+                      rng.uniform(0.1, 0.2, n))
+
+
+def there_and_back(pf):
     ctx, L = vpm._context(0), N.lib()
+    ctx.check(L.vpmx_upload(ctx.ptr, pf._ptr(), pf.np, ctypes.byref(pf.layout)))
+    ctx.check(L.vpmx_download(ctx.ptr, pf._ptr(), pf.np, ctypes.byref(pf.layout)))
+
+
+def per_particle(pf):
+    t = []
+    for _ in range(30):
+        a = time.perf_counter()
+        there_and_back(pf)
+        t.append(time.perf_counter() - a)
+    return np.median(t) / pf.np
+
+
+def test_threads_do_not_cost_more_than_they_save():
+    below, above = field(32000), field(35500)
+    ratios = sorted(per_particle(above) / per_particle(below) for _ in range(12))
+    print(np.round(ratios, 2))
+    assert ratios[8] < 1.15, ratios
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 34816, 34817, 49151, 65536, 99999, 300001])
+def test_every_particle_is_moved(n):
+    pf = field(n)
     before = pf.particles.copy()
-
-    def there_and_back():
-        ctx.check(L.vpmx_upload(ctx.ptr, pf._ptr(), n, ctypes.byref(pf.layout)))
-        ctx.check(L.vpmx_download(ctx.ptr, pf._ptr(), n, ctypes.byref(pf.layout)))
-
-    there_and_back()
-    started = []
-    for _ in range(8):
-        a = thread_id()
-        there_and_back()
-        started.append(thread_id() - a - 1)
     state = np.r_[vpm.X_INDEX, vpm.GAMMA_INDEX, vpm.SIGMA_INDEX]
-    assert np.array_equal(pf.particles[state], before[state])
-    if threaded:
-        assert max(started) > 0, started
-    else:
-        assert min(started) <= 0, started
+    ctx, L = vpm._context(0), N.lib()
+    for _ in range(4):
+        ctx.check(L.vpmx_upload(ctx.ptr, pf._ptr(), n, ctypes.byref(pf.layout)))
+        pf.particles[state] = np.nan
+        ctx.check(L.vpmx_download(ctx.ptr, pf._ptr(), n, ctypes.byref(pf.layout)))
+        assert np.array_equal(pf.particles[state], before[state])
